@@ -187,18 +187,6 @@ __device__ __forceinline__ uint32_t quant_tab(uint32_t val, uint32_t mask_byte, 
   return kQuant[(uint32_t)__builtin_popcount(mask_byte) * 768u + (uint32_t)(pbit + 1) * 256u + val];
 }
 
-// to_pixel_int through kQuant: a load per channel in place of the
-// comparisons and shifts (the annealing step quantises both endpoints of
-// every subset).
-__device__ __forceinline__ uint32_t to_pixel_tab(uint32_t p, uint32_t mask, int pbit) {
-  // the colour channels share one precision (qmask_of), alpha has its own
-  const uint32_t pb = (uint32_t)(pbit + 1) * 256u;
-  const uint32_t cb = (uint32_t)__builtin_popcount(mask & 0xFFu) * 768u + pb;
-  const uint32_t ab = (uint32_t)__builtin_popcount(mask >> 24) * 768u + pb;
-  return (uint32_t)kQuant[cb + chan(p, 0)] | ((uint32_t)kQuant[cb + chan(p, 1)] << 8) |
-         ((uint32_t)kQuant[cb + chan(p, 2)] << 16) | ((uint32_t)kQuant[ab + chan(p, 3)] << 24);
-}
-
 // ToPixel on integer-valued endpoints (uint32(c + 0.5) is then c).
 __device__ __forceinline__ uint32_t to_pixel_int(uint32_t p, uint32_t mask, int pbit) {
   uint32_t r = 0;
@@ -466,6 +454,16 @@ __device__ __forceinline__ uint32_t qmask_of(int color_prec, int alpha_prec) {
   return m;
 }
 
+// to_pixel_int for the fit's mask: a load per channel from kQuant in place
+// of the comparisons and shifts (the annealing step quantises both endpoints
+// of every subset).  The mask's bits per channel are the fit's precisions.
+__device__ __forceinline__ uint32_t to_pixel_tab(uint32_t p, const Fit &f, int pbit) {
+  const uint32_t pb = (uint32_t)(pbit + 1) * 256u;
+  const uint32_t cb = (uint32_t)f.color_prec * 768u + pb, ab = (uint32_t)f.alpha_prec * 768u + pb;
+  return (uint32_t)kQuant[cb + chan(p, 0)] | ((uint32_t)kQuant[cb + chan(p, 1)] << 8) |
+         ((uint32_t)kQuant[cb + chan(p, 2)] << 16) | ((uint32_t)kQuant[ab + chan(p, 3)] << 24);
+}
+
 // CompressSingleColor (Compressor.cpp:252-353) through the precomputed
 // per-value endpoint table.  Returns the per-pixel error; under the
 // nonuniform metric (NU) its float bit pattern, weighted by the unrotated
@@ -659,9 +657,15 @@ __device__ __forceinline__ uint32_t fit_key(uint64_t seed, uint64_t block_id, ui
   return mix32(k ^ tag);
 }
 
+// x: key + (draws made) * 0x9E3779B9, kept as a running sum.
 struct Rng {
-  uint32_t key, ctr;
-  __device__ __forceinline__ uint32_t next16() { return mix32(key + (ctr++) * 0x9E3779B9u) >> 16; }
+  uint32_t x;
+  __device__ __forceinline__ uint32_t next() {
+    const uint32_t h = mix32(x);
+    x += 0x9E3779B9u;
+    return h;
+  }
+  __device__ __forceinline__ uint32_t next16() { return next() >> 16; }
   // frand (Compressor.cpp:506-519)
   __device__ __forceinline__ float frand() {
     const uint32_t r = next16();
@@ -669,46 +673,56 @@ struct Rng {
   }
 };
 
-__device__ __forceinline__ uint32_t step_channel(uint32_t v, int s, bool minus) {
-  int x = (int)v + (minus ? -s : s);
-  x = x < 0 ? 0 : x;
-  x = x > 255 ? 255 : x;
-  return (uint32_t)x;
+// Packed 16-bit lanes: channels 0 and 2 of a pixel are (pix & 0x00FF00FF),
+// channels 1 and 3 are ((pix >> 8) & 0x00FF00FF); every quantity of the
+// index search fits 16 bits (interpolation sums within +-16352, channel
+// differences within +-255), so v_pk_* and v_dot2 give the exact integers.
+typedef short s16x2 __attribute__((ext_vector_type(2)));
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ u16x2 as_u16x2(uint32_t v) { return __builtin_bit_cast(u16x2, v); }
+__device__ __forceinline__ s16x2 as_s16x2(uint32_t v) { return __builtin_bit_cast(s16x2, v); }
+__device__ __forceinline__ s16x2 as_s16x2(u16x2 v) { return __builtin_bit_cast(s16x2, v); }
+
+// One endpoint's neighbour: every channel moved by delta = k1 - bit * k2
+// (channel pairs; bit k of the draw's top half is channel k's), clamped to
+// 0..255.
+__device__ __forceinline__ uint32_t step_endpoint(uint32_t p, uint32_t h, s16x2 k1_02,
+                                                  s16x2 k1_13, s16x2 k2_02, s16x2 k2_13) {
+  const uint32_t b02 = ((h >> 16) & 1u) | ((h >> 2) & 0x10000u);
+  const uint32_t b13 = ((h >> 17) & 1u) | ((h >> 3) & 0x10000u);
+  const s16x2 lo = {0, 0}, hi = {255, 255};
+  s16x2 n02 = as_s16x2(p & 0x00FF00FFu) + (k1_02 - as_s16x2(b02) * k2_02);
+  s16x2 n13 = as_s16x2((p >> 8) & 0x00FF00FFu) + (k1_13 - as_s16x2(b13) * k2_13);
+  n02 = __builtin_elementwise_min(__builtin_elementwise_max(n02, lo), hi);
+  n13 = __builtin_elementwise_min(__builtin_elementwise_max(n13, lo), hi);
+  return __builtin_bit_cast(uint32_t, n02) | (__builtin_bit_cast(uint32_t, n13) << 8);
 }
 
 // PickBestNeighboringEndpoints (Compressor.cpp:426-498) on integer endpoints.
+// A channel's bit of the draw chooses its direction: without p-bits +step or
+// -step; with them the p-bit flips, and an endpoint whose p-bit was 0 moves
+// by -step or 0, one whose p-bit was 1 by 0 or +step.
 __device__ __forceinline__ void pick_neighbor(const Fit &f, Rng &rng, uint32_t p1, uint32_t p2,
                                               int cur_pbc, uint32_t &np1, uint32_t &np2,
                                               int &npbc, uint32_t vp1, uint32_t vp2, int vpbc) {
-  int step[4];
-  step[0] = step[1] = step[2] = 1 << (8 - f.color_prec);
-  step[3] = 1 << (8 - f.alpha_prec);
-  if (f.mode < 4) step[(f.rot + 3) % 4] = 0;
+  // channel steps; the opaque modes' alpha (channel 3) stays
+  const uint32_t cs = 1u << (8 - f.color_prec);
+  const uint32_t as = f.mode < 4 ? 0u : 1u << (8 - f.alpha_prec);
+  const uint32_t s02 = cs | (cs << 16), s13 = cs | (as << 16);
   const bool has_pb = f.pbit_type != PB_NONE;
   if (has_pb) npbc = f.pbit_type == PB_SHARED ? (cur_pbc + 1) % 2 : 3 - cur_pbc;
+  const s16x2 k2_02 = as_s16x2(has_pb ? s02 : s02 << 1);
+  const s16x2 k2_13 = as_s16x2(has_pb ? s13 : s13 << 1);
   bool visited = true;
   int guard = -1;
   while (visited && ++guard < 16) {
 #pragma unroll
     for (int pt = 0; pt < 2; pt++) {
       const uint32_t p = pt ? p1 : p2;
-      const uint32_t dirv = rng.next16() % 16;
-      uint32_t np = 0;
-      if (has_pb) {
-        const int oldp = pbc_bit(f.pbit_type, cur_pbc, pt);
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-          const bool bit = (dirv >> k) & 1;
-          uint32_t c = chan(p, k);
-          if (bit && oldp == 0) c = step_channel(c, step[k], true);
-          else if (!bit && oldp == 1) c = step_channel(c, step[k], false);
-          np |= c << (8 * k);
-        }
-      } else {
-#pragma unroll
-        for (int k = 0; k < 4; k++)
-          np |= step_channel(chan(p, k), step[k], (dirv >> k) & 1) << (8 * k);
-      }
+      const bool up = !has_pb || pbc_bit(f.pbit_type, cur_pbc, pt) == 1;
+      const uint32_t np = step_endpoint(p, rng.next(), as_s16x2(up ? s02 : 0u),
+                                        as_s16x2(up ? s13 : 0u), k2_02, k2_13);
       if (pt) np1 = np;
       else np2 = np;
     }
@@ -1454,44 +1468,54 @@ __device__ __forceinline__ void wg_enqueue(Work &w, bool valid, int type, uint32
   if (valid) w.queue[(size_t)type * w.qcap + s_base[type] + local] = id;
 }
 
-// Packed 16-bit lanes: channels 0 and 2 of a pixel are (pix & 0x00FF00FF),
-// channels 1 and 3 are ((pix >> 8) & 0x00FF00FF); every quantity of the
-// index search fits 16 bits (interpolation sums <= 255 * 64 + 32, channel
-// differences within +-255), so v_pk_* and v_dot2 give the exact integers.
-typedef short s16x2 __attribute__((ext_vector_type(2)));
-typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ u16x2 as_u16x2(uint32_t v) { return __builtin_bit_cast(u16x2, v); }
-__device__ __forceinline__ s16x2 as_s16x2(uint32_t v) { return __builtin_bit_cast(s16x2, v); }
-__device__ __forceinline__ s16x2 as_s16x2(u16x2 v) { return __builtin_bit_cast(s16x2, v); }
-
 // Weight of the second endpoint at index j for nb = 4, 8, 16 entries:
 // (64 j + (nb - 1) / 2) / (nb - 1) by a multiply-shift, equal to
 // kInterpolationValues (Compressor.cpp:159-168); bc7_upload_tables checks
-// every entry on the host before the kernels run.
+// every entry on the host before the kernels run.  weight_word holds the
+// weight in its high half, where the packed multiply of interp_err reads it
+// without a shift.
 struct WeightFn {
-  uint32_t h, m;
+  uint32_t m, b;
 };
 __host__ __device__ __forceinline__ WeightFn weight_fn(int nb) {
-  if (nb == 4) return {1u, 21846u};
-  if (nb == 8) return {3u, 9363u};
-  return {7u, 4370u};
+  if (nb == 4) return {64u * 21846u, 21846u};
+  if (nb == 8) return {64u * 9363u, 3u * 9363u};
+  return {64u * 4370u, 7u * 4370u};
+}
+__host__ __device__ __forceinline__ uint32_t weight_word(WeightFn fn, uint32_t j) {
+  // j < 16: with the masks the compiler sees both factors below 2^24 and
+  // uses the full-rate 24-bit multiply-add
+  return (fn.m & 0xFFFFFFu) * (j & 0xFFFFFFu) + fn.b;
 }
 __host__ __device__ __forceinline__ uint32_t weight_of(WeightFn fn, uint32_t j) {
-  // j < 16: with the mask the compiler sees both factors below 2^24 and
-  // uses the full-rate 24-bit multiply
-  return ((64u * (j & 15u) + fn.h) * fn.m) >> 16;
+  return weight_word(fn, j) >> 16;
 }
 
-// Per-subset constants of one annealing step.  The interpolated value is
-// (e1 * (64 - w) + e2 * w + 32) >> 6 = (64 e1 + 32 + (e2 - e1) * w) >> 6, so
-// 64 e1 + 32 and the difference suffice.
+// A texel as the pixel pass reads it: 64 times its channel pairs (each 16-bit
+// lane at most 64 * 255 = 16320).  The interpolated value of an index weight
+// w is (e1 (64 - w) + e2 w + 32) >> 6 = (64 e1 + 32 + (e2 - e1) w) >> 6, so
+// with the texel scaled by 64 its difference to the texel is one shift of
+// one sum, and the texel's projection is 64 times the integer one.
+__device__ __forceinline__ uint32_t pair02x64(uint32_t pix) { return (pix & 0x00FF00FFu) << 6; }
+__device__ __forceinline__ uint32_t pair13x64(uint32_t pix) {
+  return ((pix >> 8) & 0x00FF00FFu) << 6;
+}
+
+// a . b + c in the three-operand form of the instruction: asked to saturate
+// (every sum here is far from the 32-bit range) the compiler cannot take the
+// accumulating two-operand form, which needs its start value moved into place
+// first (three moves per pixel in the pixel pass).
+__device__ __forceinline__ int dot2(s16x2 a, s16x2 b, int c) {
+  return __builtin_amdgcn_sdot2(a, b, c, true);
+}
+
+// Per-subset constants of one annealing step.
 struct SubConst {
-  uint32_t a02, a13;  // 64 * endpoint 1 + 32, channel pairs (see interp_err)
+  uint32_t a02, a13;  // 64 * endpoint 1 + 32, channel pairs
   uint32_t d02, d13;  // endpoint 2 - endpoint 1 (signed pairs)
-  int ad;             // endpoint 1 . (endpoint 2 - endpoint 1)
-  int l;              // squared endpoint distance, 1 when the endpoints are equal
-  float rl;           // 1 / l from below (see pixel_bounds)
+  uint32_t q02, q13;  // the projection axis (d, or d seen through a rotation)
+  int ad;             // -64 * endpoint 1 . (endpoint 2 - endpoint 1)
+  float rl;           // 1 / (64 l), l the squared endpoint distance (see pixel_bounds)
 };
 
 __device__ __forceinline__ SubConst sub_const(uint32_t e1, uint32_t e2) {
@@ -1500,116 +1524,129 @@ __device__ __forceinline__ SubConst sub_const(uint32_t e1, uint32_t e2) {
   const uint32_t b02 = e2 & 0x00FF00FFu, b13 = (e2 >> 8) & 0x00FF00FFu;
   c.d02 = __builtin_bit_cast(uint32_t, as_s16x2(b02) - as_s16x2(a02));
   c.d13 = __builtin_bit_cast(uint32_t, as_s16x2(b13) - as_s16x2(a13));
+  c.q02 = c.d02;
+  c.q13 = c.d13;
   // each 16-bit lane: 64 a + 32 <= 16352
   c.a02 = (a02 << 6) + 0x00200020u;
   c.a13 = (a13 << 6) + 0x00200020u;
   // endpoint 1's projection on the axis, subtracted from each pixel's
-  c.ad = __builtin_amdgcn_sdot2(as_s16x2(a02), as_s16x2(c.d02),
-                                __builtin_amdgcn_sdot2(as_s16x2(a13), as_s16x2(c.d13), 0, false),
-                                false);
-  const int l = __builtin_amdgcn_sdot2(as_s16x2(c.d02), as_s16x2(c.d02),
-                                       __builtin_amdgcn_sdot2(as_s16x2(c.d13),
-                                                              as_s16x2(c.d13), 0, false),
-                                       false);
+  c.ad = -64 * dot2(as_s16x2(a02), as_s16x2(c.d02), dot2(as_s16x2(a13), as_s16x2(c.d13), 0));
+  const int l = dot2(as_s16x2(c.d02), as_s16x2(c.d02), dot2(as_s16x2(c.d13), as_s16x2(c.d13), 0));
   // equal endpoints give d = 0 for every pixel, so l = 1 yields index 0
-  c.l = l > 0 ? l : 1;
-  // v_rcp_f32 is within 1 ulp (2^-23); scaled by 1 - 2^-20 the product
-  // num * rl stays strictly below num / l for num > 0
-  c.rl = __builtin_amdgcn_rcpf((float)c.l) * (1.0f - 0x1p-20f);
+  const float lf = (float)(l > 0 ? l : 1);
+  // v_rcp_f32 is within 1 ulp; one Newton step makes it the correctly
+  // rounded 1 / l for every l <= 4 * 255^2 (checked for starts within 2 ulp)
+  const float r = __builtin_amdgcn_rcpf(lf);
+  c.rl = __builtin_fmaf(__builtin_fmaf(-lf, r, 1.0f), r, r) * 0x1p-6f;
   return c;
 }
 
-// Squared error of the pixel pairs against index weight w1: each lane
-// computes (64 e1 + 32 + (e2 - e1) w1) >> 6, where (e2 - e1) w1 lies within
-// +-255 * 64 and the sum is 64 times an interpolant in 0..255 plus 32 (at
-// most 16352), so signed 16-bit lanes hold every intermediate exactly.
-__device__ __forceinline__ uint32_t interp_err(uint32_t p02, uint32_t p13, const SubConst &c,
-                                               uint32_t w1) {
-  const s16x2 W = {(short)w1, (short)w1};
-  const s16x2 S = {6, 6};
-  const s16x2 i02 = (as_s16x2(c.d02) * W + as_s16x2(c.a02)) >> S;
-  const s16x2 i13 = (as_s16x2(c.d13) * W + as_s16x2(c.a13)) >> S;
-  const s16x2 e02 = as_s16x2(p02) - i02;
-  const s16x2 e13 = as_s16x2(p13) - i13;
-  return (uint32_t)__builtin_amdgcn_sdot2(e02, e02, __builtin_amdgcn_sdot2(e13, e13, 0, false),
-                                          false);
+// The projection axis of a rotation mode (ptmode = rotation + 1).  Its
+// points are the texels with channel r - 1 replaced by alpha (r > 0) and
+// alpha 255 (point_of), so a point's projection is the texel's on a permuted
+// axis (alpha taking channel r - 1's component, that channel none) plus
+// 255 times the axis' alpha component.  sel02 / sel13: v_perm_b32 selectors
+// over (d02, d13), identity without a rotation.
+__device__ __forceinline__ void rotation_selectors(int ptmode, uint32_t &sel02, uint32_t &sel13) {
+  // bytes 0-3 of the selector index d13, 4-7 d02, 0x0c a zero byte
+  sel02 = 0x07060504u;
+  sel13 = 0x03020100u;
+  if (ptmode == 1) sel13 = 0x0c0c0100u;
+  if (ptmode == 2) {
+    sel02 = 0x07060c0cu;
+    sel13 = 0x05040100u;
+  }
+  if (ptmode == 3) sel13 = 0x01000c0cu;
+  if (ptmode == 4) {
+    sel02 = 0x0c0c0504u;
+    sel13 = 0x07060100u;
+  }
+}
+__device__ __forceinline__ void rotate_axis(SubConst &c, int ptmode, uint32_t sel02,
+                                            uint32_t sel13) {
+  c.q02 = __builtin_amdgcn_perm(c.d02, c.d13, sel02);
+  c.q13 = __builtin_amdgcn_perm(c.d02, c.d13, sel13);
+  const int da = (int)c.d13 >> 16;
+  c.ad += ptmode ? 64 * 255 * da : 0;
 }
 
-// QuantizedError's per-pixel index search (RGBAEndpoints.cpp:240-300) for
-// pixel pix (projected as pt), without branches: both neighbouring indices
-// are scored and the second kept only when it exists and is strictly better;
-// equal endpoints give index 0.  Returns the error, the index in *best.
+// Difference of the pixel pairs (64 p) to the interpolant of index weight
+// word ww, (64 e1 + 32 - 64 p + (e2 - e1) w) >> 6 = interpolant - p: z holds
+// 64 e1 + 32 - 64 p, and the sum lies within +-16352, so signed 16-bit lanes
+// hold it exactly.
+__device__ __forceinline__ s16x2 interp_diff(s16x2 z, uint32_t d, uint32_t ww) {
+  const s16x2 w = as_s16x2(ww);
+  const s16x2 W = {w.y, w.y};
+  const s16x2 S = {6, 6};
+  return (as_s16x2(d) * W + z) >> S;
+}
+
+// QuantizedError's neighbouring indices (RGBAEndpoints.cpp:240-300) of a
+// pixel: j1 = floor(t), j2 = ceil(t), both clamped to the index range, of the
+// reference's t = fl(fl(d / l) * kf) (float, d the integer projection, l the
+// integer squared distance, kf = nb - 1).  Those equal the floor and ceiling
+// of the rational d kf / l: its distance to an integer, when nonzero, is at
+// least 1 / l >= 1 / (4 * 255^2) = 3.8e-6, more than the float error of at
+// most 2^-23 |t| <= 1.9e-6 for |t| <= 16 (larger |t| is clamped away), and
+// fl(fl(k / kf) kf) = k for every integer 0 <= k <= kf in {3, 7, 15} (checked
+// exhaustively).
 //
-// The reference takes j1 = floor(t), j2 = ceil(t) of t = fl(fl(d / l) * kf)
-// (float, d the integer projection, l the integer squared distance, kf =
-// nb - 1).  Those equal the floor and ceiling of the rational d kf / l: its
-// distance to an integer, when nonzero, is at least 1 / l >= 1 / (4 * 255^2)
-// = 3.8e-6, more than the float error of at most 2^-23 |t| <= 1.9e-6 for
-// |t| <= 16 (larger |t| is clamped away), and fl(fl(k / kf) kf) = k for every
-// integer 0 <= k <= kf in {3, 7, 15} (checked exhaustively).  So the quotient
-// is taken in integers: an estimate from a reciprocal, corrected by one step
-// with the exact remainder.  The estimate comes from below (rl < 1 / l with
-// a margin larger than the float errors, and num / l <= 15 * 510 / sqrt(l)
-// keeps its shortfall under 1), so for num >= 0 it is the quotient or one
-// less, and one upward step fixes it.  For num < 0 the index is 0 whatever
-// the estimate: j1 clamps to 0 and j2 <= j1.
-__device__ __forceinline__ void pixel_bounds(uint32_t pt, const SubConst &c, int nb, int &j1,
-                                             int &j2) {
-  const uint32_t t02 = pt & 0x00FF00FFu, t13 = (pt >> 8) & 0x00FF00FFu;
-  const int d = __builtin_amdgcn_sdot2(
-      as_s16x2(t02), as_s16x2(c.d02),
-      __builtin_amdgcn_sdot2(as_s16x2(t13), as_s16x2(c.d13), -c.ad, false),
-      false);
-  const int num = __mul24(d, nb - 1);  // |d| <= 4 * 255^2, so 24-bit operands suffice
-  int q = (int)floorf((float)num * c.rl);
-  int rem = num - __mul24(q, c.l);
-  const bool hi = rem >= c.l;
-  q += hi ? 1 : 0;
-  rem -= hi ? c.l : 0;
-  j1 = q < 0 ? 0 : (q > nb - 1 ? nb - 1 : q);
-  j2 = q + (rem != 0 ? 1 : 0);
-  j2 = j2 > nb - 1 ? nb - 1 : j2;
+// Here u = fl(64 d * rl) clamped to [0, 1] (64 d is below 2^24, so its
+// conversion is exact; a d below 0 or above l clamps to the end index), and
+// the floor and ceiling are truncations of fma(u, kf, 1.9e-6) and
+// fma(u, kf, 1 - 1.9e-6).  Exact for every l up to 4 * 255^2, d in 0..l and
+// kf: checked exhaustively at the steps of both functions of d, which are
+// monotone.  The pass is bound by VALU issue: an integer quotient corrected
+// with the exact remainder took 17 instructions per pixel where this takes 9;
+// with the texels kept as scaled pairs (no unpacking, one subtraction per
+// pair) and the rotation folded into the axis (no separate point) the pass
+// went from about 54 instructions per pixel to 33, and the 4096 x 4096
+// annealing from 46.0 to 34.3 ms (reference search) and 5.2 to 4.1 ms
+// (learned).
+constexpr float kIndexSlack = 1.9e-6f;
+
+__device__ __forceinline__ void pixel_bounds(uint32_t p02, uint32_t p13, const SubConst &c,
+                                             float kf, uint32_t &j1, uint32_t &j2) {
+  const int d = dot2(as_s16x2(p02), as_s16x2(c.q02), dot2(as_s16x2(p13), as_s16x2(c.q13), c.ad));
+  const float u = __builtin_amdgcn_fmed3f((float)d * c.rl, 0.0f, 1.0f);
+  j1 = (uint32_t)__builtin_fmaf(u, kf, kIndexSlack);
+  j2 = (uint32_t)__builtin_fmaf(u, kf, 1.0f - kIndexSlack);
 }
 
-__device__ __forceinline__ uint32_t pixel_err(uint32_t pix, uint32_t pt, const SubConst &c,
-                                              int nb, float kf, WeightFn wf, int *best) {
-  (void)kf;
-  const uint32_t p02 = pix & 0x00FF00FFu, p13 = (pix >> 8) & 0x00FF00FFu;
-  int j1, j2;
-  pixel_bounds(pt, c, nb, j1, j2);
-  const uint32_t e1 = interp_err(p02, p13, c, weight_of(wf, (uint32_t)j1));
-  const uint32_t e2 = interp_err(p02, p13, c, weight_of(wf, (uint32_t)j2));
-  const bool second = j2 > j1 && e2 < e1;
-  *best = second ? j2 : j1;
-  return second ? e2 : e1;
+// The per-pixel index search without branches: both neighbouring indices
+// are scored and the second kept only when strictly better (where the two
+// are the same index the errors are equal).  Returns the error, the index in
+// *best.  p02, p13: the texel's pairs times 64.
+__device__ __forceinline__ uint32_t pixel_err(uint32_t p02, uint32_t p13, const SubConst &c,
+                                              float kf, WeightFn wf, uint32_t *best) {
+  uint32_t j1, j2;
+  pixel_bounds(p02, p13, c, kf, j1, j2);
+  const s16x2 z02 = as_s16x2(c.a02) - as_s16x2(p02), z13 = as_s16x2(c.a13) - as_s16x2(p13);
+  const uint32_t w1 = weight_word(wf, j1), w2 = weight_word(wf, j2);
+  const s16x2 x02 = interp_diff(z02, c.d02, w1), x13 = interp_diff(z13, c.d13, w1);
+  const s16x2 y02 = interp_diff(z02, c.d02, w2), y13 = interp_diff(z13, c.d13, w2);
+  const uint32_t e1 = (uint32_t)dot2(x02, x02, dot2(x13, x13, 0));
+  const uint32_t e2 = (uint32_t)dot2(y02, y02, dot2(y13, y13, 0));
+  *best = e2 < e1 ? j2 : j1;
+  return e2 < e1 ? e2 : e1;
 }
 
-// The nonuniform metric's pixel pass (the metric is described above qerr_nu).
-// interp_err under the weights (pair lanes: .x channels 0 / 1, .y 2 / 3).
-__device__ __forceinline__ float interp_err_nu(uint32_t p02, uint32_t p13, const SubConst &c,
-                                               uint32_t w1, const Weights &m) {
-  const s16x2 W = {(short)w1, (short)w1};
-  const s16x2 S = {6, 6};
-  const s16x2 i02 = (as_s16x2(c.d02) * W + as_s16x2(c.a02)) >> S;
-  const s16x2 i13 = (as_s16x2(c.d13) * W + as_s16x2(c.a13)) >> S;
-  const s16x2 e02 = as_s16x2(p02) - i02;
-  const s16x2 e13 = as_s16x2(p13) - i13;
-  return werr(e02.x, e13.x, e02.y, e13.y, m);
-}
-
-// pixel_err under the weights: the same two neighbouring indices, the second
-// kept only when strictly better.
-__device__ __forceinline__ float pixel_err_nu(uint32_t pix, uint32_t pt, const SubConst &c,
-                                              int nb, WeightFn wf, const Weights &m,
-                                              int *best) {
-  const uint32_t p02 = pix & 0x00FF00FFu, p13 = (pix >> 8) & 0x00FF00FFu;
-  int j1, j2;
-  pixel_bounds(pt, c, nb, j1, j2);
-  const float e1 = interp_err_nu(p02, p13, c, weight_of(wf, (uint32_t)j1), m);
-  const float e2 = interp_err_nu(p02, p13, c, weight_of(wf, (uint32_t)j2), m);
-  const bool second = j2 > j1 && e2 < e1;
-  *best = second ? j2 : j1;
-  return second ? e2 : e1;
+// The nonuniform metric's pixel pass (the metric is described above qerr_nu):
+// the same two neighbouring indices, scored under the weights (pair lanes:
+// .x channels 0 / 1, .y 2 / 3), the second kept only when strictly better.
+__device__ __forceinline__ float pixel_err_nu(uint32_t p02, uint32_t p13, const SubConst &c,
+                                              float kf, WeightFn wf, const Weights &m,
+                                              uint32_t *best) {
+  uint32_t j1, j2;
+  pixel_bounds(p02, p13, c, kf, j1, j2);
+  const s16x2 z02 = as_s16x2(c.a02) - as_s16x2(p02), z13 = as_s16x2(c.a13) - as_s16x2(p13);
+  const uint32_t w1 = weight_word(wf, j1), w2 = weight_word(wf, j2);
+  const s16x2 x02 = interp_diff(z02, c.d02, w1), x13 = interp_diff(z13, c.d13, w1);
+  const s16x2 y02 = interp_diff(z02, c.d02, w2), y13 = interp_diff(z13, c.d13, w2);
+  const float e1 = werr(x02.x, x13.x, x02.y, x13.y, m);
+  const float e2 = werr(y02.x, y13.x, y02.y, y13.y, m);
+  *best = e2 < e1 ? j2 : j1;
+  return e2 < e1 ? e2 : e1;
 }
 
 __device__ __forceinline__ SubConst pick_sub(bool c, const SubConst &x, const SubConst &y) {
@@ -1619,7 +1656,8 @@ __device__ __forceinline__ SubConst pick_sub(bool c, const SubConst &x, const Su
   r.ad = c ? x.ad : y.ad;
   r.d02 = c ? x.d02 : y.d02;
   r.d13 = c ? x.d13 : y.d13;
-  r.l = c ? x.l : y.l;
+  r.q02 = c ? x.q02 : y.q02;
+  r.q13 = c ? x.q13 : y.q13;
   r.rl = c ? x.rl : y.rl;
   return r;
 }
@@ -1693,8 +1731,9 @@ __device__ __forceinline__ double shape_estimate(const uint32_t px[16], int shap
     const uint32_t s = ((m1 >> i) & 1u) ? 1u + ((m2 >> i) & 1u) : 0u;
     const SubConst k = NS == 2 ? pick_sub(s != 0, c[1], c[0])
                                : pick_sub(s == 0, c[0], pick_sub(s == 1, c[1], c[NS - 1]));
-    int best;
-    const uint32_t me = pixel_err(px[i], px[i], k, NB, (float)(NB - 1), wf, &best);
+    uint32_t best;
+    const uint32_t me =
+        pixel_err(pair02x64(px[i]), pair13x64(px[i]), k, (float)(NB - 1), wf, &best);
 #pragma unroll
     for (int t = 0; t < NS; t++) e[t] += s == (uint32_t)t ? me : 0u;
   }
@@ -1733,8 +1772,9 @@ __device__ __forceinline__ double shape_estimate_nu(const uint32_t px[16], int s
     const uint32_t s = ((m1 >> i) & 1u) ? 1u + ((m2 >> i) & 1u) : 0u;
     const SubConst k = NS == 2 ? pick_sub(s != 0, c[1], c[0])
                                : pick_sub(s == 0, c[0], pick_sub(s == 1, c[1], c[NS - 1]));
-    int best;
-    const float me = pixel_err_nu(px[i], px[i], k, NB, wf, m, &best);
+    uint32_t best;
+    const float me =
+        pixel_err_nu(pair02x64(px[i]), pair13x64(px[i]), k, (float)(NB - 1), wf, m, &best);
 #pragma unroll
     for (int t = 0; t < NS; t++) e[t] += s == (uint32_t)t ? me : 0.0f;
   }
@@ -1852,9 +1892,10 @@ __device__ __forceinline__ void masked_subset_errors(const uint32_t px[16], uint
       ka = pick_sub(sub == (uint32_t)t, ca[t], ka);
       kb = pick_sub(sub == (uint32_t)t, cb[t], kb);
     }
-    int best;
-    const uint32_t xa = pixel_err(px[i], px[i], ka, NB, (float)(NB - 1), wf, &best);
-    const uint32_t xb = TWO ? pixel_err(px[i], px[i], kb, NB, (float)(NB - 1), wf, &best) : 0u;
+    const uint32_t p02 = pair02x64(px[i]), p13 = pair13x64(px[i]);
+    uint32_t best;
+    const uint32_t xa = pixel_err(p02, p13, ka, (float)(NB - 1), wf, &best);
+    const uint32_t xb = TWO ? pixel_err(p02, p13, kb, (float)(NB - 1), wf, &best) : 0u;
 #pragma unroll
     for (int t = 0; t < NS; t++) {
       ea[t] += sub == (uint32_t)t ? xa : 0u;
@@ -2692,6 +2733,8 @@ __global__ void __launch_bounds__(64) setup_kernel(BlockRange r, Bc7Params prm, 
 // endpoints.  Lanes that finish take the next candidate from a wave-local
 // window of the global list, so the wave stays full.
 // ---------------------------------------------------------------------------
+constexpr int kRowWords = 37;  // a lane's LDS row: 32 texel words, 4 of index bits, odd
+
 struct Lane {
   bool has;
   uint32_t id;
@@ -2699,12 +2742,13 @@ struct Lane {
   int nsub, entry, shape;
   uint32_t sub2;       // subset of pixel i in bits 2i..2i+1
   int ptmode;
-  uint32_t *px;        // the block's 16 texels: this lane's row of LDS
-  uint32_t *pt;        // the points the RGB fit sees (rotation applied), same row
+  uint32_t sel02, sel13;  // rotation_selectors(ptmode)
+  uint32_t *px;        // this lane's row of LDS: the 16 texels (64 times their pairs
+                       // 02 and 13), then the index bits of subsets 1 and 2
   uint32_t active;
   uint32_t p1[3], p2[3], bp1[3], bp2[3], cur[3], best[3];
   int cpbc[3], bpbc[3], energy[3];
-  uint32_t key[3], ctr[3];
+  uint32_t rng[3];
   uint64_t idx;        // indices of all subsets (best so far)
   uint32_t extra;
   // nonuniform metric: the candidate's weights (its rotation applied), the
@@ -2726,20 +2770,29 @@ __device__ void lane_load(Lane &L, const BlockRange &r, const Bc7Params &prm, co
   L.entry = (st.info >> 17) & 7;
   set_fit(L.f, mode, rot, im);
   L.ptmode = kModes[mode].has_rot ? rot + 1 : 0;
+  rotation_selectors(L.ptmode, L.sel02, L.sel13);
   L.sub2 = 0;
-  for (int s = 1; s < L.nsub; s++) {
-    const uint32_t m = subset_mask(L.shape, L.nsub, s);
+#pragma unroll
+  for (int s = 1; s < 3; s++) {
+    const uint32_t m = s < L.nsub ? subset_mask(L.shape, L.nsub, s) : 0u;
+    uint32_t lo = 0, hi = 0;
 #pragma unroll
     for (int i = 0; i < 16; i++)
-      if ((m >> i) & 1) L.sub2 |= (uint32_t)s << (2 * i);
+      if ((m >> i) & 1) {
+        L.sub2 |= (uint32_t)s << (2 * i);
+        if (i < 8) lo |= 0xFu << (4 * i);
+        else hi |= 0xFu << (4 * (i - 8));
+      }
+    L.px[32 + 2 * (s - 1)] = lo;
+    L.px[33 + 2 * (s - 1)] = hi;
   }
   {
     uint32_t v[16];
     load_block(r, id_block(st.id), v);
 #pragma unroll
     for (int i = 0; i < 16; i++) {
-      L.px[i] = v[i];
-      L.pt[i] = point_of(v[i], L.ptmode);
+      L.px[2 * i] = pair02x64(v[i]);
+      L.px[2 * i + 1] = pair13x64(v[i]);
     }
   }
   const uint64_t bid = prm.block_id_base + r.first_block + id_block(st.id);
@@ -2750,8 +2803,7 @@ __device__ void lane_load(Lane &L, const BlockRange &r, const Bc7Params &prm, co
     L.cur[s] = L.best[s] = st.err[s];
     L.cpbc[s] = L.bpbc[s] = (st.pbc >> (2 * s)) & 3;
     L.energy[s] = 0;
-    L.ctr[s] = 0;
-    L.key[s] = fit_key(prm.seed, bid, cand_tag(mode, L.entry, s, rot, im));
+    L.rng[s] = fit_key(prm.seed, bid, cand_tag(mode, L.entry, s, rot, im));
   }
   L.idx = (uint64_t)st.idx_lo | ((uint64_t)st.idx_hi << 32);
   L.extra = st.extra_err;
@@ -2763,33 +2815,43 @@ __device__ void lane_load(Lane &L, const BlockRange &r, const Bc7Params &prm, co
   }
 }
 
+// The constants of subset code s (0 beyond NSUB): NSUB = 1 takes sc0.
+// ROT: whether a lane of the wave holds a rotation mode; without one every
+// axis is the endpoint difference itself, which saves the two selects.
+template <int NSUB, bool ROT>
+__device__ __forceinline__ SubConst pixel_const(uint32_t s, const SubConst &sc0,
+                                                const SubConst &sc1, const SubConst &sc2) {
+  SubConst c = NSUB == 1 ? sc0
+                         : (NSUB == 2 ? pick_sub(s != 0, sc1, sc0)
+                                      : pick_sub(s == 0, sc0, pick_sub(s == 1, sc1, sc2)));
+  if (NSUB > 1 && !ROT) {
+    c.q02 = c.d02;
+    c.q13 = c.d13;
+  }
+  return c;
+}
+
 // The 16-pixel pass for up to NSUB subsets: errors per subset and the
 // indices.  Every pixel is scored; errors of subsets that have stopped
 // annealing are not used.
-template <int NSUB>
+template <int NSUB, bool ROT>
 __device__ __forceinline__ void score_pixels(const Lane &L, const SubConst &sc0,
-                                             const SubConst &sc1, const SubConst &sc2, int nb,
-                                             float kf, WeightFn wf, uint32_t nerr[3],
-                                             uint64_t &nidx) {
+                                             const SubConst &sc1, const SubConst &sc2, float kf,
+                                             WeightFn wf, uint32_t nerr[3], uint64_t &nidx) {
+  uint32_t all = 0, idx[2] = {0, 0};
 #pragma unroll
   for (int i = 0; i < 16; i++) {
     const uint32_t s = NSUB == 1 ? 0u : (L.sub2 >> (2 * i)) & 3u;
-    const SubConst c = NSUB == 1 ? sc0
-                                 : (NSUB == 2 ? pick_sub(s != 0, sc1, sc0)
-                                              : pick_sub(s == 0, sc0, pick_sub(s == 1, sc1, sc2)));
-    const uint32_t pix = L.px[i];
-    const uint32_t pt = L.pt[i];
-    int best;
-    const uint32_t me = pixel_err(pix, pt, c, nb, kf, wf, &best);
-    if (NSUB == 1) {
-      nerr[0] += me;
-    } else {
-      nerr[0] += s == 0 ? me : 0u;
-      nerr[1] += s == 1 ? me : 0u;
-      if (NSUB == 3) nerr[2] += s == 2 ? me : 0u;
-    }
-    nidx |= (uint64_t)best << (4 * i);
+    const SubConst c = pixel_const<NSUB, ROT>(s, sc0, sc1, sc2);
+    uint32_t best;
+    const uint32_t me = pixel_err(L.px[2 * i], L.px[2 * i + 1], c, kf, wf, &best);
+    all += me;
+    if (NSUB > 1) nerr[1] += s == 1 ? me : 0u;
+    if (NSUB == 3) nerr[2] += s == 2 ? me : 0u;
+    idx[i >> 3] |= best << (4 * (i & 7));
   }
+  nerr[0] = all - nerr[1] - nerr[2];
+  nidx = (uint64_t)idx[0] | ((uint64_t)idx[1] << 32);
 }
 
 // The pixel pass under the nonuniform metric: float errors, each subset's
@@ -2797,16 +2859,15 @@ __device__ __forceinline__ void score_pixels(const Lane &L, const SubConst &sc0,
 // unchanged).
 template <int NSUB>
 __device__ __forceinline__ void score_pixels_nu(const Lane &L, const SubConst &sc0,
-                                                const SubConst &sc1, const SubConst &sc2, int nb,
-                                                WeightFn wf, float nerr[3], uint64_t &nidx) {
+                                                const SubConst &sc1, const SubConst &sc2,
+                                                float kf, WeightFn wf, float nerr[3],
+                                                uint64_t &nidx) {
 #pragma unroll
   for (int i = 0; i < 16; i++) {
     const uint32_t s = NSUB == 1 ? 0u : (L.sub2 >> (2 * i)) & 3u;
-    const SubConst c = NSUB == 1 ? sc0
-                                 : (NSUB == 2 ? pick_sub(s != 0, sc1, sc0)
-                                              : pick_sub(s == 0, sc0, pick_sub(s == 1, sc1, sc2)));
-    int best;
-    const float me = pixel_err_nu(L.px[i], L.pt[i], c, nb, wf, L.m, &best);
+    const SubConst c = pixel_const<NSUB, true>(s, sc0, sc1, sc2);
+    uint32_t best;
+    const float me = pixel_err_nu(L.px[2 * i], L.px[2 * i + 1], c, kf, wf, L.m, &best);
     nerr[0] += s == 0 ? me : 0.0f;
     if (NSUB > 1) nerr[1] += s == 1 ? me : 0.0f;
     if (NSUB == 3) nerr[2] += s == 2 ? me : 0.0f;
@@ -2821,15 +2882,13 @@ __device__ __forceinline__ void score_pixels_nu(const Lane &L, const SubConst &s
 template <int NSUB>
 __device__ __forceinline__ void score_pixels_group(const Lane &L, const SubConst &sc0,
                                                    const SubConst &sc1, const SubConst &sc2,
-                                                   int nb, float kf, WeightFn wf, uint32_t nerr[3],
+                                                   float kf, WeightFn wf, uint32_t nerr[3],
                                                    uint64_t &nidx, int G, int m) {
   for (int i = m; i < 16; i += G) {
     const uint32_t s = NSUB == 1 ? 0u : (L.sub2 >> (2 * i)) & 3u;
-    const SubConst c = NSUB == 1 ? sc0
-                                 : (NSUB == 2 ? pick_sub(s != 0, sc1, sc0)
-                                              : pick_sub(s == 0, sc0, pick_sub(s == 1, sc1, sc2)));
-    int best;
-    const uint32_t me = pixel_err(L.px[i], L.pt[i], c, nb, kf, wf, &best);
+    const SubConst c = pixel_const<NSUB, true>(s, sc0, sc1, sc2);
+    uint32_t best;
+    const uint32_t me = pixel_err(L.px[2 * i], L.px[2 * i + 1], c, kf, wf, &best);
     nerr[0] += s == 0 ? me : 0u;
     if (NSUB > 1) nerr[1] += s == 1 ? me : 0u;
     if (NSUB == 3) nerr[2] += s == 2 ? me : 0u;
@@ -2862,15 +2921,15 @@ __device__ bool lane_step(Lane &L, uint32_t q, int G = 1, int m = 0) {
     npbc[s] = 0;
     if (!((L.active >> s) & 1)) continue;
     Rng rng;
-    rng.key = L.key[s];
-    rng.ctr = L.ctr[s];
+    rng.x = L.rng[s];
     pick_neighbor(f, rng, L.p1[s], L.p2[s], L.cpbc[s], np1[s], np2[s], npbc[s], L.bp1[s],
                   L.bp2[s], L.bpbc[s]);
-    L.ctr[s] = rng.ctr;
-    e1[s] = to_pixel_tab(np1[s], f.qmask, pbc_bit(f.pbit_type, npbc[s], 0));
-    e2[s] = to_pixel_tab(np2[s], f.qmask, pbc_bit(f.pbit_type, npbc[s], 1));
+    L.rng[s] = rng.x;
+    e1[s] = to_pixel_tab(np1[s], f, pbc_bit(f.pbit_type, npbc[s], 0));
+    e2[s] = to_pixel_tab(np2[s], f, pbc_bit(f.pbit_type, npbc[s], 1));
   }
-  const SubConst sc0 = sub_const(e1[0], e2[0]);
+  SubConst sc0 = sub_const(e1[0], e2[0]);
+  rotate_axis(sc0, L.ptmode, L.sel02, L.sel13);
   const SubConst sc1 = sub_const(e1[1], e2[1]);
   const SubConst sc2 = sub_const(e1[2], e2[2]);
   uint32_t nerr[3] = {0, 0, 0};
@@ -2882,21 +2941,23 @@ __device__ bool lane_step(Lane &L, uint32_t q, int G = 1, int m = 0) {
   // candidates of one subset count
   if constexpr (NU) {
     float nerf[3] = {0.0f, 0.0f, 0.0f};
-    if (__ballot(L.nsub == 3)) score_pixels_nu<3>(L, sc0, sc1, sc2, nb, wf, nerf, nidx);
-    else if (__ballot(L.nsub == 2)) score_pixels_nu<2>(L, sc0, sc1, sc2, nb, wf, nerf, nidx);
-    else score_pixels_nu<1>(L, sc0, sc1, sc2, nb, wf, nerf, nidx);
+    if (__ballot(L.nsub == 3)) score_pixels_nu<3>(L, sc0, sc1, sc2, kf, wf, nerf, nidx);
+    else if (__ballot(L.nsub == 2)) score_pixels_nu<2>(L, sc0, sc1, sc2, kf, wf, nerf, nidx);
+    else score_pixels_nu<1>(L, sc0, sc1, sc2, kf, wf, nerf, nidx);
 #pragma unroll
     for (int s = 0; s < 3; s++) nerr[s] = __float_as_uint(nerf[s]);
   } else if (GROUPED) {
-    if (__ballot(L.nsub == 3)) score_pixels_group<3>(L, sc0, sc1, sc2, nb, kf, wf, nerr, nidx, G, m);
-    else if (__ballot(L.nsub == 2)) score_pixels_group<2>(L, sc0, sc1, sc2, nb, kf, wf, nerr, nidx, G, m);
-    else score_pixels_group<1>(L, sc0, sc1, sc2, nb, kf, wf, nerr, nidx, G, m);
+    if (__ballot(L.nsub == 3)) score_pixels_group<3>(L, sc0, sc1, sc2, kf, wf, nerr, nidx, G, m);
+    else if (__ballot(L.nsub == 2)) score_pixels_group<2>(L, sc0, sc1, sc2, kf, wf, nerr, nidx, G, m);
+    else score_pixels_group<1>(L, sc0, sc1, sc2, kf, wf, nerr, nidx, G, m);
+  } else if (!__ballot(L.nsub > 1)) {
+    score_pixels<1, true>(L, sc0, sc1, sc2, kf, wf, nerr, nidx);
+  } else if (__ballot(L.ptmode != 0)) {
+    score_pixels<3, true>(L, sc0, sc1, sc2, kf, wf, nerr, nidx);
   } else if (__ballot(L.nsub == 3)) {
-    score_pixels<3>(L, sc0, sc1, sc2, nb, kf, wf, nerr, nidx);
-  } else if (__ballot(L.nsub == 2)) {
-    score_pixels<2>(L, sc0, sc1, sc2, nb, kf, wf, nerr, nidx);
+    score_pixels<3, false>(L, sc0, sc1, sc2, kf, wf, nerr, nidx);
   } else {
-    score_pixels<1>(L, sc0, sc1, sc2, nb, kf, wf, nerr, nidx);
+    score_pixels<2, false>(L, sc0, sc1, sc2, kf, wf, nerr, nidx);
   }
 #pragma unroll
   for (int s = 0; s < 3; s++) {
@@ -2908,10 +2969,9 @@ __device__ bool lane_step(Lane &L, uint32_t q, int G = 1, int m = 0) {
       // frand() < exp(0.1 (cur - err) / temp).  Here err >= cur, so the
       // probability is at most 1 and a draw in [1, 3) never accepts.
       Rng rng;
-      rng.key = L.key[s];
-      rng.ctr = L.ctr[s];
+      rng.x = L.rng[s];
       const float rr = rng.frand();
-      L.ctr[s] = rng.ctr;
+      L.rng[s] = rng.x;
       if (rr < 1.0f) {
         // A single-precision estimate of the probability decides unless rr
         // lies within 1e-4 (relative) of it, which covers the estimate's
@@ -2944,10 +3004,9 @@ __device__ bool lane_step(Lane &L, uint32_t q, int G = 1, int m = 0) {
     }
     if (err < L.best[s]) {
       // indices of this subset's pixels
-      uint64_t m = 0;
-#pragma unroll
-      for (int i = 0; i < 16; i++)
-        if (((L.sub2 >> (2 * i)) & 3) == (uint32_t)s) m |= (uint64_t)0xF << (4 * i);
+      const uint64_t m1 = (uint64_t)L.px[32] | ((uint64_t)L.px[33] << 32);
+      const uint64_t m2 = (uint64_t)L.px[34] | ((uint64_t)L.px[35] << 32);
+      const uint64_t m = s == 0 ? ~(m1 | m2) : (s == 1 ? m1 : m2);
       L.idx = (L.idx & ~m) | (nidx & m);
       L.bp1[s] = np1[s];
       L.bp2[s] = np2[s];
@@ -3064,8 +3123,9 @@ anneal_kernel(BlockRange r, Bc7Params prm, Work w) {
   };
   const uint64_t lt = (1ull << lane) - 1ull;
   const uint32_t listed = *(volatile uint32_t *)&w.counters[w.alist ? 18 : 16];
-  // per lane 16 texels then 16 points, odd row stride: conflict-free
-  __shared__ uint32_t s_px[64 * 33];
+  // per lane 16 texels (two words each) and the subsets' index bits, odd row
+  // stride: conflict-free
+  __shared__ uint32_t s_px[64 * kRowWords];
   // Learned search: the list is in state order, and the set-up kernels
   // append the rotation modes' states last (counters[19] holds the first of
   // them): the list's rotation states are its suffix from rot_begin.  (The
@@ -3095,8 +3155,7 @@ anneal_kernel(BlockRange r, Bc7Params prm, Work w) {
     const int m = lane % kRotGroup;
     constexpr uint64_t leaders = group_leaders(kRotGroup);
     Lane T;
-    T.px = s_px + lane * 33;
-    T.pt = T.px + 16;
+    T.px = s_px + lane * kRowWords;
     T.has = false;
     uint32_t abase = 0, aend = 0;
     bool aexh = false;
@@ -3143,8 +3202,7 @@ anneal_kernel(BlockRange r, Bc7Params prm, Work w) {
   // Phase B: the other states, one lane each, from the end of the prefix
   const uint32_t total = rot_begin;
   Lane L;
-  L.px = s_px + lane * 33;
-  L.pt = L.px + 16;
+  L.px = s_px + lane * kRowWords;
   L.has = false;
   uint32_t wbase = 0, wend = 0;  // wave-local window of the list
   bool exhausted = false;
@@ -3219,8 +3277,7 @@ anneal_kernel(BlockRange r, Bc7Params prm, Work w) {
   T.has = false;
   if (g < na) {
     T = s_tail[g];
-    T.px = s_px + s_row[g] * 33;
-    T.pt = T.px + 16;
+    T.px = s_px + s_row[g] * kRowWords;
   }
   while (__ballot(T.has)) {
     for (int u = 0; u < UNROLL; u++) {
