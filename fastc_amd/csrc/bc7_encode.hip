@@ -1446,6 +1446,10 @@ __device__ __forceinline__ void load_block(const BlockRange &r, uint32_t rel, ui
   }
 }
 
+__device__ __forceinline__ uint32_t idx_at(uint32_t lo, uint32_t hi, int i) {
+  return i < 8 ? (lo >> (4 * i)) & 0xFu : (hi >> (4 * (i - 8))) & 0xFu;
+}
+
 // Key of one fit's annealing stream; shape entries 0..4 take bits 3-4 and 10.
 __device__ __forceinline__ uint32_t cand_tag(int mode, int entry, int subset, int rot, int im) {
   return (uint32_t)mode | ((uint32_t)(entry & 3) << 3) | ((uint32_t)subset << 5) |
@@ -2905,6 +2909,26 @@ __device__ __forceinline__ void score_pixels_group(const Lane &L, const SubConst
   nidx = (uint64_t)lo | ((uint64_t)hi << 32);
 }
 
+// AcceptNewEndpointError (Compressor.cpp:524-536) for err >= cur: accept when
+// frand() < exp(0.1 (cur - err) / temp), temp = energy / (q - 1).  The
+// probability is at most 1, so a draw rr in [1, 3) never accepts.
+__device__ __forceinline__ bool accept_worse(float rr, float cf, float ef, int q, int energy) {
+  if (!(rr < 1.0f)) return false;
+  // A single-precision estimate of the probability decides unless rr
+  // lies within 1e-4 (relative) of it, which covers the estimate's
+  // error; then the double expression of the reference decides.  The
+  // uniform metric's errors are integers below 2^24, so their float
+  // difference is exact; the nonuniform metric's are floats, whose
+  // difference has a relative error of at most 2^-23 where it is not
+  // exact, well inside the margin.
+  const float pf = __expf(__fdividef(0.1f * (cf - ef) * (float)(q - 1), (float)energy));
+  if (rr != 0.0f && rr < pf * 0.9999f) return true;
+  if (rr != 0.0f && rr > pf * 1.0001f) return false;
+  const float temp = (float)energy / (float)(q - 1);
+  const double pr = exp(((double)0.1f * ((double)cf - (double)ef)) / (double)temp);
+  return (double)rr < pr;
+}
+
 // One annealing step of every active subset.  Returns true when the
 // candidate is finished.  With GROUPED, the lanes of an aligned group of G
 // hold the same candidate and share the pixel pass (member m); every other
@@ -2965,36 +2989,12 @@ __device__ bool lane_step(Lane &L, uint32_t q, int G = 1, int m = 0) {
     const uint32_t err = nerr[s];
     bool accept = err < L.cur[s];
     if (!accept) {
-      // AcceptNewEndpointError (Compressor.cpp:524-536): accept when
-      // frand() < exp(0.1 (cur - err) / temp).  Here err >= cur, so the
-      // probability is at most 1 and a draw in [1, 3) never accepts.
       Rng rng;
       rng.x = L.rng[s];
       const float rr = rng.frand();
       L.rng[s] = rng.x;
-      if (rr < 1.0f) {
-        // A single-precision estimate of the probability decides unless rr
-        // lies within 1e-4 (relative) of it, which covers the estimate's
-        // error; then the double expression of the reference decides.  The
-        // uniform metric's errors are integers below 2^24, so their float
-        // difference is exact; the nonuniform metric's are floats, whose
-        // difference has a relative error of at most 2^-23 where it is not
-        // exact, well inside the margin.
-        const float cf = NU ? __uint_as_float(L.cur[s]) : (float)L.cur[s];
-        const float ef = NU ? __uint_as_float(err) : (float)err;
-        const float diff = cf - ef;
-        const float pf =
-            __expf(__fdividef(0.1f * diff * (float)((int)q - 1), (float)L.energy[s]));
-        if (rr != 0.0f && rr < pf * 0.9999f) {
-          accept = true;
-        } else if (!(rr != 0.0f && rr > pf * 1.0001f)) {
-          const float temp = (float)L.energy[s] / (float)((int)q - 1);
-          const double cd = NU ? (double)cf : (double)L.cur[s];
-          const double ed = NU ? (double)ef : (double)err;
-          const double pr = exp(((double)0.1f * (cd - ed)) / (double)temp);
-          accept = (double)rr < pr;
-        }
-      }
+      accept = accept_worse(rr, NU ? __uint_as_float(L.cur[s]) : (float)L.cur[s],
+                            NU ? __uint_as_float(err) : (float)err, (int)q, L.energy[s]);
     }
     if (accept) {
       L.cur[s] = err;
@@ -3296,6 +3296,261 @@ anneal_kernel(BlockRange r, Bc7Params prm, Work w) {
 }
 
 // ---------------------------------------------------------------------------
+// Kernel 3b: the same annealing with one lane per pixel.  A row of 16 lanes
+// holds one candidate; a lane holds its own pixel and the state of its own
+// subset only (every lane of a subset computes the same step), so a step is
+// one pixel's work plus three row sums instead of sixteen pixels' work for
+// up to three subsets: about a quarter of the instructions, and of the
+// latency, of a step of the one-lane form.  A wave advances four candidates
+// where the one-lane form advances 64, so per candidate the step costs about
+// four times more issue: this form is for lists that leave the chip idle,
+// where the longest chain sets the time.
+// ---------------------------------------------------------------------------
+// kQuant's rows for the annealing's precisions (0, 4..8 bits) and p-bits, in
+// LDS: an L1 hit of the global table costs a step several times more latency.
+constexpr int kSpreadQuantRows = 6 * 2;
+__device__ __forceinline__ uint32_t spread_quant_row(int bits) {
+  return (uint32_t)(bits ? bits - 3 : 0) * 512u;
+}
+__device__ __forceinline__ void spread_quant_load(uint8_t *lds) {
+  uint32_t *dst = reinterpret_cast<uint32_t *>(lds);
+  for (int t = threadIdx.x; t < kSpreadQuantRows * 64; t += blockDim.x) {
+    const int row = t >> 6, bits = row < 2 ? 0 : (row >> 1) + 3, pb = row & 1;
+    dst[t] = reinterpret_cast<const uint32_t *>(kQuant)[(bits * 3 + pb + 1) * 64 + (t & 63)];
+  }
+}
+
+// Sum over the 16 lanes of a row (every lane of the wave active).
+__device__ __forceinline__ uint32_t row_sum(uint32_t v) {
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xf, 0xf, true);  // row_ror:8
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x124, 0xf, 0xf, true);
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x122, 0xf, 0xf, true);
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x121, 0xf, 0xf, true);
+  return v;
+}
+
+// COUNT: the work counters of anneal_kernel, in the same units.
+template <bool COUNT>
+__global__ void __launch_bounds__(256) anneal_spread_kernel(BlockRange r, Bc7Params prm, Work w) {
+  __shared__ __align__(4) uint8_t s_quant[kSpreadQuantRows * 256];
+  spread_quant_load(s_quant);
+  __syncthreads();
+  const int lane = threadIdx.x & 63, px = lane & 15, row0 = lane & 48;
+  const uint32_t total = *(volatile uint32_t *)&w.counters[w.alist ? 18 : 16];
+  const int q = (int)prm.quality;
+  constexpr uint64_t kRowLeaders = group_leaders(16);
+  uint32_t n_ref = 0, n_gpu = 0;  // COUNT
+  // the candidate (the same in the row)
+  bool has = false;
+  uint32_t id = 0, info = 0, extra = 0;
+  // its constants
+  uint32_t s02 = 0, s13 = 0, k2_02 = 0, k2_13 = 0, qc = 0, qa = 0, sel02 = 0, sel13 = 0;
+  uint32_t flip = 0, nopb = 0, sh = 0;
+  int ptmode = 0, nsub = 1;
+  float kf = 0.0f;
+  WeightFn wf = {0, 0};
+  // this lane's pixel, its subset and that subset's state
+  uint32_t p02 = 0, p13 = 0, sub = 0, bidx = 0;
+  bool active = false;
+  uint32_t p1 = 0, p2 = 0, bp1 = 0, bp2 = 0, cur = 0, best = 0, cpbc = 0, bpbc = 0, x = 0;
+  int energy = 0;
+  bool exhausted = total == 0;
+  for (;;) {
+    // idle rows take the next candidates, from the end of the list (the
+    // rotation modes, whose chains are the longest, first)
+    uint64_t hasm = __ballot(has);
+    const uint64_t need = ~hasm & kRowLeaders;
+    if (need && !exhausted) {
+      const uint32_t want = (uint32_t)__popcll(need);
+      uint32_t base = 0;
+      if (lane == 0) base = atomicAdd(&w.counters[17], want);
+      base = __shfl(base, 0);
+      if (base >= total || total - base <= want) exhausted = true;
+      const uint32_t item = base + (uint32_t)__popcll(need & ((1ull << row0) - 1ull));
+      if (!has && item < total) {
+        const uint32_t at = total - 1u - item;
+        const AState &st = w.astate[w.alist ? w.alist[at] : at];
+        has = true;
+        id = st.id;
+        info = st.info;
+        extra = st.extra_err;
+        const int mode = info & 7, rot = (info >> 3) & 3, im = (info >> 5) & 1;
+        const int shape = (info >> 8) & 63;
+        nsub = (info >> 6) & 3;
+        Fit f;
+        set_fit(f, mode, rot, im);
+        ptmode = kModes[mode].has_rot ? rot + 1 : 0;
+        rotation_selectors(ptmode, sel02, sel13);
+        const uint32_t cs = 1u << (8 - f.color_prec);
+        const uint32_t as = mode < 4 ? 0u : 1u << (8 - f.alpha_prec);
+        const bool has_pb = f.pbit_type != PB_NONE;
+        s02 = cs | (cs << 16);
+        s13 = cs | (as << 16);
+        k2_02 = has_pb ? s02 : s02 << 1;
+        k2_13 = has_pb ? s13 : s13 << 1;
+        nopb = has_pb ? 0u : 1u;
+        flip = f.pbit_type == PB_SHARED ? 1u : (has_pb ? 3u : 0u);
+        sh = f.pbit_type == PB_NOTSHARED ? 1u : 0u;
+        qc = spread_quant_row(f.color_prec);
+        qa = spread_quant_row(f.alpha_prec);
+        const int nb = 1 << f.nbits_idx;
+        kf = (float)(nb - 1);
+        wf = weight_fn(nb);
+        sub = 0;
+        if (nsub == 2) sub = (kShape2[shape] >> px) & 1u;
+        if (nsub == 3) sub = subset_of(kShape3[shape][0], kShape3[shape][1], px);
+        const uint32_t rel = id_block(id), b = r.first_block + rel;
+        const uint32_t bx = b % r.blocks_wide, by = b / r.blocks_wide;
+        const uint32_t pix =
+            r.img[(size_t)(by * 4 + (px >> 2)) * r.width + bx * 4 + (px & 3)];
+        p02 = pair02x64(pix);
+        p13 = pair13x64(pix);
+        p1 = bp1 = st.p1[sub];
+        p2 = bp2 = st.p2[sub];
+        cur = best = st.err[sub];
+        cpbc = bpbc = (st.pbc >> (2 * sub)) & 3u;
+        bidx = idx_at(st.idx_lo, st.idx_hi, px);
+        energy = 0;
+        active = (info >> (14 + sub)) & 1u;
+        x = fit_key(prm.seed, prm.block_id_base + b,
+                    cand_tag(mode, (int)((info >> 17) & 7), (int)sub, rot, im));
+      }
+      hasm = __ballot(has);
+    }
+    if (!hasm) break;
+    const bool multi = __ballot(nsub > 1) != 0;  // stale in rows without a candidate: harmless
+    for (int u = 0; u < 4; u++) {
+      if constexpr (COUNT) {
+        const uint64_t act = __ballot(active);
+        n_ref += active ? 1u : 0u;
+        n_gpu += (px == 0 && ((act >> row0) & 0xFFFFull)) ? 16u : 0u;
+      }
+      // the neighbour (pick_neighbor): draws for endpoint 2, then 1
+      uint32_t np1 = 0, np2 = 0;
+      const uint32_t npbc = cpbc ^ flip;
+      const uint32_t up2 = ((cpbc >> sh) & 1u) | nopb, up1 = (cpbc & 1u) | nopb;
+      const s16x2 k02 = as_s16x2(k2_02), k13 = as_s16x2(k2_13);
+      bool again = true;
+      for (int tries = 0; tries < 16; tries++) {
+        if (again) {
+          Rng rng;
+          rng.x = x;
+          np2 = step_endpoint(p2, rng.next(), as_s16x2(up2 ? s02 : 0u), as_s16x2(up2 ? s13 : 0u),
+                              k02, k13);
+          np1 = step_endpoint(p1, rng.next(), as_s16x2(up1 ? s02 : 0u), as_s16x2(up1 ? s13 : 0u),
+                              k02, k13);
+          x = rng.x;
+          again = active && np1 == bp1 && np2 == bp2 && npbc == bpbc;
+        }
+        if (!__ballot(again)) break;
+      }
+      // its error, this lane's pixel
+      const uint32_t o1 = ((npbc >> sh) & 1u) << 8, o2 = (npbc & 1u & (flip ? 1u : 0u)) << 8;
+      const uint8_t *c1 = s_quant + qc + o1, *c2 = s_quant + qc + o2;
+      const uint32_t e1 = (uint32_t)c1[chan(np1, 0)] | ((uint32_t)c1[chan(np1, 1)] << 8) |
+                          ((uint32_t)c1[chan(np1, 2)] << 16) |
+                          ((uint32_t)s_quant[qa + o1 + chan(np1, 3)] << 24);
+      const uint32_t e2 = (uint32_t)c2[chan(np2, 0)] | ((uint32_t)c2[chan(np2, 1)] << 8) |
+                          ((uint32_t)c2[chan(np2, 2)] << 16) |
+                          ((uint32_t)s_quant[qa + o2 + chan(np2, 3)] << 24);
+      SubConst sc = sub_const(e1, e2);
+      rotate_axis(sc, ptmode, sel02, sel13);
+      uint32_t j;
+      const uint32_t me = pixel_err(p02, p13, sc, kf, wf, &j);
+      // its subset's error
+      uint32_t err = row_sum(me);
+      if (multi) {
+        const uint32_t t1 = row_sum(sub == 1 ? me : 0u), t2 = row_sum(sub == 2 ? me : 0u);
+        err = sub == 0 ? err - t1 - t2 : (sub == 1 ? t1 : t2);
+      }
+      if (active) {
+        bool accept = err < cur;
+        if (!accept) {
+          Rng rng;
+          rng.x = x;
+          const float rr = rng.frand();
+          x = rng.x;
+          accept = accept_worse(rr, (float)cur, (float)err, q, energy);
+        }
+        if (accept) {
+          cur = err;
+          p1 = np1;
+          p2 = np2;
+          cpbc = npbc;
+        }
+        if (err < best) {
+          best = err;
+          bp1 = np1;
+          bp2 = np2;
+          bpbc = npbc;
+          bidx = j;
+          energy = 0;
+        }
+        energy++;
+        active = best > 0 && energy < q;
+      }
+    }
+    // finished rows write their records (lane_finish)
+    const uint64_t act = __ballot(active);
+    const bool done = has && ((act >> row0) & 0xFFFFull) == 0;
+    if (!__ballot(done)) continue;
+    // every lane of the wave takes part in the shuffles
+    const uint32_t pair = bidx | ((uint32_t)__shfl_xor((int)bidx, 1) << 4);
+    uint32_t sum = extra, pbcs = 0;
+    const uint64_t sub1 = __ballot(sub == 1) >> row0, sub2 = __ballot(sub == 2) >> row0;
+    const int first1 = __ffsll((unsigned long long)(sub1 & 0xFFFFull)) - 1;
+    const int first2 = __ffsll((unsigned long long)(sub2 & 0xFFFFull)) - 1;
+    const bool leader = px == 0 || px == first1 || px == first2;
+#pragma unroll
+    for (int s = 0; s < 3; s++) {
+      const int from = s == 0 ? 0 : (s == 1 ? first1 : first2);
+      const uint32_t e = (uint32_t)__shfl((int)best, row0 + (from & 15));
+      const uint32_t pb = (uint32_t)__shfl((int)bpbc, row0 + (from & 15));
+      if (from >= 0) {
+        sum += e;
+        pbcs |= pb << (2 * s);
+      }
+    }
+    if (done) {
+      CandRec *rc = &w.rec[id];
+      if (leader) {
+        const int mode = info & 7;
+        Fit f;
+        set_fit(f, mode, (info >> 3) & 3, (info >> 5) & 1);
+        const bool has_pb = f.pbit_type != PB_NONE;
+        uint32_t e1 = to_pixel_int(bp1, f.qmask, has_pb ? (int)((bpbc >> sh) & 1u) : -1);
+        uint32_t e2 = to_pixel_int(bp2, f.qmask, has_pb ? (int)(bpbc & 1u) : -1);
+        if (ptmode) {
+          e1 = (e1 & 0x00FFFFFFu) | (rc->px1[0] & 0xFF000000u);
+          e2 = (e2 & 0x00FFFFFFu) | (rc->px2[0] & 0xFF000000u);
+        }
+        rc->px1[sub] = e1;
+        rc->px2[sub] = e2;
+      }
+      if (!(px & 1)) reinterpret_cast<uint8_t *>(&rc->cidx_lo)[px >> 1] = (uint8_t)pair;
+      if (px == 0) {
+        rc->meta = (rc->meta & ~0x3Fu) | (rc->meta & 0x3Fu & ~((1u << (2 * nsub)) - 1u)) | pbcs |
+                   kMetaAnnealed;
+        rc->err = sum;
+      }
+      has = false;
+      active = false;
+    }
+  }
+  if constexpr (COUNT) {
+    unsigned long long a = n_ref, b = n_gpu;
+    for (int off = 32; off >= 1; off >>= 1) {
+      a += __shfl_xor(a, off);
+      b += __shfl_xor(b, off);
+    }
+    if (lane == 0) {
+      atomicAdd(&prm.work_counts[0], a);
+      atomicAdd(&prm.work_counts[1], b);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Kernel 4: choose the mode and write the block, one lane per block.
 // ---------------------------------------------------------------------------
 
@@ -3314,10 +3569,6 @@ struct BitWriter {
     pos += n;
   }
 };
-
-__device__ __forceinline__ uint32_t idx_at(uint32_t lo, uint32_t hi, int i) {
-  return i < 8 ? (lo >> (4 * i)) & 0xFu : (hi >> (4 * (i - 8))) & 0xFu;
-}
 
 // CompressOptimalColorBC7 (Compressor.cpp:1424-1458).
 __device__ void pack_solid(uint32_t pixel, uint32_t wm, BitWriter &w) {
@@ -3891,8 +4142,23 @@ hipError_t bc7_upload_tables(int device) {
   return hipSuccess;
 }
 
-void launch_anneal(uint32_t grid, const BlockRange &r, const Bc7Params &p, const bc7::Work &w,
-                   hipStream_t stream) {
+// Blocks up to which a call's annealing runs one lane per pixel.
+constexpr uint32_t kSpreadBlocks = 1u << 14, kSpreadBlocksLearned = 1u << 17;
+
+void launch_anneal(uint32_t grid, int cus, const BlockRange &r, const Bc7Params &p,
+                   const bc7::Work &w, hipStream_t stream) {
+  if (!w.nu_total && r.num_blocks <= (w.alist ? kSpreadBlocksLearned : kSpreadBlocks)) {
+    // workgroups of 16 rows, no more than the candidates could use
+    uint32_t groups = (r.num_blocks * (uint32_t)bc7::kMaxCands + 15) / 16;
+    if (groups > (uint32_t)cus * 6u) groups = (uint32_t)cus * 6u;
+    if (p.work_counts)
+      hipLaunchKernelGGL(bc7::anneal_spread_kernel<true>, dim3(groups), dim3(256), 0, stream, r,
+                         p, w);
+    else
+      hipLaunchKernelGGL(bc7::anneal_spread_kernel<false>, dim3(groups), dim3(256), 0, stream, r,
+                         p, w);
+    return;
+  }
   if (p.work_counts && !w.nu_total)  // the counting instance (both searches)
     hipLaunchKernelGGL((bc7::anneal_kernel<4, 3, false, true>), dim3(grid), dim3(64), 0, stream,
                        r, p, w);
@@ -4114,7 +4380,7 @@ hipError_t bc7_encode(const BlockRange &r, const Bc7Params &p, const Bc7Scratch 
                          (const uint32_t *)w.aid, (const uint32_t *)w.counters,
                          (const uint32_t *)w.sel, cerr, q0err, (const uint32_t *)chunk_count,
                          alist);
-      launch_anneal(persistent, r, p, wa, stream);
+      launch_anneal(persistent, g_num_cus[dev], r, p, wa, stream);
       timing_end(t, kTagBc7Anneal, stream);
     }
     t = timing_begin(stream);
@@ -4136,7 +4402,7 @@ hipError_t bc7_encode(const BlockRange &r, const Bc7Params &p, const Bc7Scratch 
   }
   if (p.quality > 0) {
     t = timing_begin(stream);
-    launch_anneal(persistent, r, p, w, stream);
+    launch_anneal(persistent, g_num_cus[dev], r, p, w, stream);
     timing_end(t, kTagBc7Anneal, stream);
   }
   t = timing_begin(stream);
