@@ -454,16 +454,6 @@ __device__ __forceinline__ uint32_t qmask_of(int color_prec, int alpha_prec) {
   return m;
 }
 
-// to_pixel_int for the fit's mask: a load per channel from kQuant in place
-// of the comparisons and shifts (the annealing step quantises both endpoints
-// of every subset).  The mask's bits per channel are the fit's precisions.
-__device__ __forceinline__ uint32_t to_pixel_tab(uint32_t p, const Fit &f, int pbit) {
-  const uint32_t pb = (uint32_t)(pbit + 1) * 256u;
-  const uint32_t cb = (uint32_t)f.color_prec * 768u + pb, ab = (uint32_t)f.alpha_prec * 768u + pb;
-  return (uint32_t)kQuant[cb + chan(p, 0)] | ((uint32_t)kQuant[cb + chan(p, 1)] << 8) |
-         ((uint32_t)kQuant[cb + chan(p, 2)] << 16) | ((uint32_t)kQuant[ab + chan(p, 3)] << 24);
-}
-
 // CompressSingleColor (Compressor.cpp:252-353) through the precomputed
 // per-value endpoint table.  Returns the per-pixel error; under the
 // nonuniform metric (NU) its float bit pattern, weighted by the unrotated
@@ -697,37 +687,6 @@ __device__ __forceinline__ uint32_t step_endpoint(uint32_t p, uint32_t h, s16x2 
   n02 = __builtin_elementwise_min(__builtin_elementwise_max(n02, lo), hi);
   n13 = __builtin_elementwise_min(__builtin_elementwise_max(n13, lo), hi);
   return __builtin_bit_cast(uint32_t, n02) | (__builtin_bit_cast(uint32_t, n13) << 8);
-}
-
-// PickBestNeighboringEndpoints (Compressor.cpp:426-498) on integer endpoints.
-// A channel's bit of the draw chooses its direction: without p-bits +step or
-// -step; with them the p-bit flips, and an endpoint whose p-bit was 0 moves
-// by -step or 0, one whose p-bit was 1 by 0 or +step.
-__device__ __forceinline__ void pick_neighbor(const Fit &f, Rng &rng, uint32_t p1, uint32_t p2,
-                                              int cur_pbc, uint32_t &np1, uint32_t &np2,
-                                              int &npbc, uint32_t vp1, uint32_t vp2, int vpbc) {
-  // channel steps; the opaque modes' alpha (channel 3) stays
-  const uint32_t cs = 1u << (8 - f.color_prec);
-  const uint32_t as = f.mode < 4 ? 0u : 1u << (8 - f.alpha_prec);
-  const uint32_t s02 = cs | (cs << 16), s13 = cs | (as << 16);
-  const bool has_pb = f.pbit_type != PB_NONE;
-  if (has_pb) npbc = f.pbit_type == PB_SHARED ? (cur_pbc + 1) % 2 : 3 - cur_pbc;
-  const s16x2 k2_02 = as_s16x2(has_pb ? s02 : s02 << 1);
-  const s16x2 k2_13 = as_s16x2(has_pb ? s13 : s13 << 1);
-  bool visited = true;
-  int guard = -1;
-  while (visited && ++guard < 16) {
-#pragma unroll
-    for (int pt = 0; pt < 2; pt++) {
-      const uint32_t p = pt ? p1 : p2;
-      const bool up = !has_pb || pbc_bit(f.pbit_type, cur_pbc, pt) == 1;
-      const uint32_t np = step_endpoint(p, rng.next(), as_s16x2(up ? s02 : 0u),
-                                        as_s16x2(up ? s13 : 0u), k2_02, k2_13);
-      if (pt) np1 = np;
-      else np2 = np;
-    }
-    visited = np1 == vp1 && np2 == vp2 && npbc == vpbc;
-  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1487,9 +1446,15 @@ __host__ __device__ __forceinline__ WeightFn weight_fn(int nb) {
   return {64u * 4370u, 7u * 4370u};
 }
 __host__ __device__ __forceinline__ uint32_t weight_word(WeightFn fn, uint32_t j) {
-  // j < 16: with the masks the compiler sees both factors below 2^24 and
-  // uses the full-rate 24-bit multiply-add
-  return (fn.m & 0xFFFFFFu) * (j & 0xFFFFFFu) + fn.b;
+#if defined(__HIP_DEVICE_COMPILE__)
+  // both factors are below 2^24: the full-rate 24-bit multiply-add, which
+  // the compiler only finds where it can see the factors' ranges
+  uint32_t w;
+  asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(w) : "v"(j), "v"(fn.m), "v"(fn.b));
+  return w;
+#else
+  return fn.m * j + fn.b;
+#endif
 }
 __host__ __device__ __forceinline__ uint32_t weight_of(WeightFn fn, uint32_t j) {
   return weight_word(fn, j) >> 16;
@@ -2734,25 +2699,185 @@ __global__ void __launch_bounds__(64) setup_kernel(BlockRange r, Bc7Params prm, 
 // Compressor.cpp:583-624), persistent.  A lane owns one candidate and
 // advances every still-annealing subset of it by one step per iteration; the
 // 16 pixels are scored in one pass, each against its own subset's
-// endpoints.  Lanes that finish take the next candidate from a wave-local
-// window of the global list, so the wave stays full.
+// endpoints.  Finished lanes wait until kRefillLanes of the wave are idle and
+// then take the next candidates together, from a wave-local window of the
+// global list.
 // ---------------------------------------------------------------------------
 constexpr int kRowWords = 37;  // a lane's LDS row: 32 texel words, 4 of index bits, odd
 
+// What a step needs of the candidate's mode, in one word:
+//   colour step 5 bits | alpha step 5 << 5 | p-bit flip 2 << 10 |
+//   first p-bit's shift 1 << 12 | no p-bits 1 << 13 |
+//   colour and alpha rows of the quantisation table 3 << 14, 3 << 17 |
+//   index bits 3 << 20
+// The endpoints' p-bits are those of the combination c (GetPBitCombo,
+// CompressionMode.h:243-250): (c >> shift) & 1 and c & 1; the next
+// combination tried is c ^ flip.
+__device__ __forceinline__ uint32_t step_cfg_pack(const Fit &f) {
+  const bool has_pb = f.pbit_type != PB_NONE;
+  const uint32_t cs = 1u << (8 - f.color_prec);
+  // the opaque modes' alpha (channel 3) stays
+  const uint32_t as = f.mode < 4 ? 0u : 1u << (8 - f.alpha_prec);
+  const uint32_t flip = f.pbit_type == PB_SHARED ? 1u : (has_pb ? 3u : 0u);
+  const uint32_t qa = f.alpha_prec ? (uint32_t)f.alpha_prec - 3u : 0u;
+  return cs | (as << 5) | (flip << 10) | ((f.pbit_type == PB_NOTSHARED ? 1u : 0u) << 12) |
+         ((has_pb ? 0u : 1u) << 13) | (((uint32_t)f.color_prec - 3u) << 14) | (qa << 17) |
+         ((uint32_t)f.nbits_idx << 20);
+}
+
+struct StepCfg {
+  uint32_t s02, s13, k2_02, k2_13, flip, sh, nopb, qc, qa;
+  float kf;
+  WeightFn wf;
+};
+
+__device__ __forceinline__ StepCfg step_cfg(uint32_t c) {
+  StepCfg k;
+  const uint32_t cs = c & 31u, as = (c >> 5) & 31u;
+  k.flip = (c >> 10) & 3u;
+  k.sh = (c >> 12) & 1u;
+  k.nopb = (c >> 13) & 1u;
+  k.s02 = cs | (cs << 16);
+  k.s13 = cs | (as << 16);
+  k.k2_02 = k.s02 << k.nopb;
+  k.k2_13 = k.s13 << k.nopb;
+  k.qc = ((c >> 14) & 7u) << 9;
+  k.qa = ((c >> 17) & 7u) << 9;
+  const int nb = 1 << ((c >> 20) & 7u);
+  k.kf = (float)(nb - 1);
+  k.wf = weight_fn(nb);
+  return k;
+}
+
+// The quantisation table's rows (kQuant) for the annealing's precisions (0,
+// 4..8 bits) and p-bits, in LDS: row (bits ? bits - 3 : 0) * 2 + p-bit.
+constexpr int kStepQuantBytes = 6 * 2 * 256;
+__device__ __forceinline__ void step_quant_load(uint8_t *lds) {
+  uint32_t *dst = reinterpret_cast<uint32_t *>(lds);
+  for (int t = threadIdx.x; t < kStepQuantBytes / 4; t += blockDim.x) {
+    const int row = t >> 6, bits = row < 2 ? 0 : (row >> 1) + 3, pb = row & 1;
+    dst[t] = reinterpret_cast<const uint32_t *>(kQuant)[(bits * 3 + pb + 1) * 64 + (t & 63)];
+  }
+}
+// An endpoint quantised with its p-bit (ToPixel).
+__device__ __forceinline__ uint32_t step_quant(const uint8_t *lds, const StepCfg &k, uint32_t p,
+                                               uint32_t pbit) {
+  const uint8_t *c = lds + (k.qc + (pbit << 8)), *a = lds + (k.qa + (pbit << 8));
+  return (uint32_t)c[chan(p, 0)] | ((uint32_t)c[chan(p, 1)] << 8) |
+         ((uint32_t)c[chan(p, 2)] << 16) | ((uint32_t)a[chan(p, 3)] << 24);
+}
+
+// The reference's acceptance expression.  A call, not inlined: inlined, the
+// exponential's constants are hoisted out of the annealing loop and cost it
+// some 20 registers for a branch that is hardly ever taken.
+__device__ __attribute__((noinline)) bool accept_exact(float rr, float cf, float ef, int q,
+                                                       int energy) {
+  const float temp = (float)energy / (float)(q - 1);
+  return (double)rr < exp(((double)0.1f * ((double)cf - (double)ef)) / (double)temp);
+}
+
+// AcceptNewEndpointError (Compressor.cpp:524-536) for err >= cur: accept when
+// frand() < exp(0.1 (cur - err) / temp), temp = energy / (q - 1).  The
+// probability is at most 1, so a draw rr in [1, 3) never accepts.
+//
+// A single-precision estimate of the probability decides unless rr lies
+// within 1e-4 (relative) of it, which covers the estimate's error (the
+// hardware reciprocal and exponential are within a few 2^-23 of theirs, and
+// where the exponent is large enough to magnify its own rounding past the
+// margin the probability is below every nonzero draw, 2^-16 at least); then
+// the double expression of the reference decides.  The uniform metric's
+// errors are integers below 2^24, so their float difference is exact; the
+// nonuniform metric's are floats, whose difference has a relative error of at
+// most 2^-23 where it is not exact, well inside the margin.  At energy 0 and
+// equal errors both forms are NaN, which never accepts.
+__device__ __forceinline__ bool accept_worse(float rr, float cf, float ef, int q, int energy) {
+  const float pf =
+      __expf(0.1f * (cf - ef) * ((float)(q - 1) * __builtin_amdgcn_rcpf((float)energy)));
+  const bool low = rr < pf * 0.9999f, high = rr > pf * 1.0001f;
+  bool accept = (rr != 0.0f) & low & (rr < 1.0f);
+  if ((rr < 1.0f) & ((rr == 0.0f) | !(low | high))) {
+    accept = accept_exact(rr, cf, ef, q, energy);
+  }
+  return accept;
+}
+
+// One subset's annealing state.
+struct SubState {
+  uint32_t p1, p2, bp1, bp2, cur, best, cpbc, bpbc, x;  // x: its random stream (Rng)
+  int energy;
+};
+
+// PickBestNeighboringEndpoints (Compressor.cpp:426-498) on integer endpoints.
+// A channel's bit of the draw chooses its direction: without p-bits +step or
+// -step; with them the p-bits flip, and an endpoint whose p-bit was 0 moves
+// by -step or 0, one whose p-bit was 1 by 0 or +step.  Up to 16 draws while
+// the neighbour is the best state itself (`live` lanes only); every lane of
+// the wave takes part.
+__device__ __forceinline__ void pick_neighbor(const StepCfg &k, bool live, SubState &t,
+                                              uint32_t &np1, uint32_t &np2, uint32_t &npbc) {
+  npbc = t.cpbc ^ k.flip;
+  const uint32_t up2 = ((t.cpbc >> k.sh) & 1u) | k.nopb, up1 = (t.cpbc & 1u) | k.nopb;
+  auto draw = [&]() {
+    // endpoint 2's draw comes first
+    Rng rng;
+    rng.x = t.x;
+    np2 = step_endpoint(t.p2, rng.next(), as_s16x2(up2 ? k.s02 : 0u),
+                        as_s16x2(up2 ? k.s13 : 0u), as_s16x2(k.k2_02), as_s16x2(k.k2_13));
+    np1 = step_endpoint(t.p1, rng.next(), as_s16x2(up1 ? k.s02 : 0u),
+                        as_s16x2(up1 ? k.s13 : 0u), as_s16x2(k.k2_02), as_s16x2(k.k2_13));
+    t.x = rng.x;
+  };
+  draw();
+  bool again = live & (np1 == t.bp1) & (np2 == t.bp2) & (npbc == t.bpbc);
+  for (int tries = 1; __ballot(again) && tries < 16; tries++) {
+    if (again) {
+      draw();
+      again = (np1 == t.bp1) & (np2 == t.bp2);
+    }
+  }
+}
+
+// The rest of a step, once the neighbour's error is known: acceptance and
+// the best state (Compressor.cpp:590-624).  Returns whether the best state
+// was replaced; live becomes false when the subset has finished.
+template <bool NU = false>
+__device__ __forceinline__ bool finish_step(SubState &t, bool &live, uint32_t err, uint32_t np1,
+                                            uint32_t np2, uint32_t npbc, int q) {
+  // the acceptance draw, made only where the error is not below cur
+  Rng rng;
+  rng.x = t.x;
+  const float rr = rng.frand();
+  const bool lower = err < t.cur;
+  const bool accept =
+      live & (lower | accept_worse(rr, NU ? __uint_as_float(t.cur) : (float)t.cur,
+                                   NU ? __uint_as_float(err) : (float)err, q, t.energy));
+  t.x = lower ? t.x : rng.x;
+  t.cur = accept ? err : t.cur;
+  t.p1 = accept ? np1 : t.p1;
+  t.p2 = accept ? np2 : t.p2;
+  t.cpbc = accept ? npbc : t.cpbc;
+  const bool better = live & (err < t.best);
+  t.best = better ? err : t.best;
+  t.bp1 = better ? np1 : t.bp1;
+  t.bp2 = better ? np2 : t.bp2;
+  t.bpbc = better ? npbc : t.bpbc;
+  t.energy = better ? 1 : t.energy + 1;
+  live = live & (t.best > 0) & (t.energy < q);
+  return better;
+}
+
 struct Lane {
   bool has;
-  uint32_t id;
-  Fit f;
-  int nsub, entry, shape;
-  uint32_t sub2;       // subset of pixel i in bits 2i..2i+1
+  uint32_t id, info;   // AState's
+  uint32_t cfg;        // step_cfg_pack
+  int nsub;
+  uint32_t m12;        // masks of the pixels of subsets 1 and 2 (<< 16)
   int ptmode;
   uint32_t sel02, sel13;  // rotation_selectors(ptmode)
   uint32_t *px;        // this lane's row of LDS: the 16 texels (64 times their pairs
                        // 02 and 13), then the index bits of subsets 1 and 2
-  uint32_t active;
-  uint32_t p1[3], p2[3], bp1[3], bp2[3], cur[3], best[3];
-  int cpbc[3], bpbc[3], energy[3];
-  uint32_t rng[3];
+  uint32_t active;     // subsets still annealing
+  SubState t0, t1, t2; // per subset
   uint64_t idx;        // indices of all subsets (best so far)
   uint32_t extra;
   // nonuniform metric: the candidate's weights (its rotation applied), the
@@ -2763,32 +2888,36 @@ struct Lane {
   double extra_nu;
 };
 
+// The low 8 bits of m as a mask of nibbles.
+__device__ __forceinline__ uint32_t nibble_mask(uint32_t m) {
+  uint32_t x = m & 0xFFu;
+  x = (x | (x << 12)) & 0x000F000Fu;
+  x = (x | (x << 6)) & 0x03030303u;
+  x = (x | (x << 3)) & 0x11111111u;
+  return (x << 4) - x;
+}
+
 template <bool NU = false>
-__device__ void lane_load(Lane &L, const BlockRange &r, const Bc7Params &prm, const AState &st) {
+__device__ __forceinline__ void lane_load(Lane &L, const BlockRange &r, const Bc7Params &prm, const AState &st) {
   L.has = true;
   L.id = st.id;
+  L.info = st.info;
   const int mode = st.info & 7, rot = (st.info >> 3) & 3, im = (st.info >> 5) & 1;
+  const int shape = (st.info >> 8) & 63, entry = (st.info >> 17) & 7;
   L.nsub = (st.info >> 6) & 3;
-  L.shape = (st.info >> 8) & 63;
   L.active = (st.info >> 14) & 7;
-  L.entry = (st.info >> 17) & 7;
-  set_fit(L.f, mode, rot, im);
+  Fit f;
+  set_fit(f, mode, rot, im);
+  L.cfg = step_cfg_pack(f);
   L.ptmode = kModes[mode].has_rot ? rot + 1 : 0;
   rotation_selectors(L.ptmode, L.sel02, L.sel13);
-  L.sub2 = 0;
+  L.m12 = 0;
 #pragma unroll
   for (int s = 1; s < 3; s++) {
-    const uint32_t m = s < L.nsub ? subset_mask(L.shape, L.nsub, s) : 0u;
-    uint32_t lo = 0, hi = 0;
-#pragma unroll
-    for (int i = 0; i < 16; i++)
-      if ((m >> i) & 1) {
-        L.sub2 |= (uint32_t)s << (2 * i);
-        if (i < 8) lo |= 0xFu << (4 * i);
-        else hi |= 0xFu << (4 * (i - 8));
-      }
-    L.px[32 + 2 * (s - 1)] = lo;
-    L.px[33 + 2 * (s - 1)] = hi;
+    const uint32_t m = s < L.nsub ? subset_mask(shape, L.nsub, s) : 0u;
+    L.m12 |= m << (16 * (s - 1));
+    L.px[32 + 2 * (s - 1)] = nibble_mask(m);
+    L.px[33 + 2 * (s - 1)] = nibble_mask(m >> 8);
   }
   {
     uint32_t v[16];
@@ -2800,15 +2929,17 @@ __device__ void lane_load(Lane &L, const BlockRange &r, const Bc7Params &prm, co
     }
   }
   const uint64_t bid = prm.block_id_base + r.first_block + id_block(st.id);
-#pragma unroll
-  for (int s = 0; s < 3; s++) {
-    L.p1[s] = L.bp1[s] = st.p1[s];
-    L.p2[s] = L.bp2[s] = st.p2[s];
-    L.cur[s] = L.best[s] = st.err[s];
-    L.cpbc[s] = L.bpbc[s] = (st.pbc >> (2 * s)) & 3;
-    L.energy[s] = 0;
-    L.rng[s] = fit_key(prm.seed, bid, cand_tag(mode, L.entry, s, rot, im));
-  }
+  auto start = [&](SubState &t, int s) {
+    t.p1 = t.bp1 = st.p1[s];
+    t.p2 = t.bp2 = st.p2[s];
+    t.cur = t.best = st.err[s];
+    t.cpbc = t.bpbc = (st.pbc >> (2 * s)) & 3u;
+    t.energy = 0;
+    t.x = fit_key(prm.seed, bid, cand_tag(mode, entry, s, rot, im));
+  };
+  start(L.t0, 0);
+  start(L.t1, 1);
+  start(L.t2, 2);
   L.idx = (uint64_t)st.idx_lo | ((uint64_t)st.idx_hi << 32);
   L.extra = st.extra_err;
   if constexpr (NU) {
@@ -2819,15 +2950,15 @@ __device__ void lane_load(Lane &L, const BlockRange &r, const Bc7Params &prm, co
   }
 }
 
-// The constants of subset code s (0 beyond NSUB): NSUB = 1 takes sc0.
+// The constants of pixel i: those of its subset (NSUB = 1 takes sc0).
 // ROT: whether a lane of the wave holds a rotation mode; without one every
 // axis is the endpoint difference itself, which saves the two selects.
 template <int NSUB, bool ROT>
-__device__ __forceinline__ SubConst pixel_const(uint32_t s, const SubConst &sc0,
+__device__ __forceinline__ SubConst pixel_const(bool in1, bool in2, const SubConst &sc0,
                                                 const SubConst &sc1, const SubConst &sc2) {
-  SubConst c = NSUB == 1 ? sc0
-                         : (NSUB == 2 ? pick_sub(s != 0, sc1, sc0)
-                                      : pick_sub(s == 0, sc0, pick_sub(s == 1, sc1, sc2)));
+  SubConst c = sc0;
+  if (NSUB > 1) c = pick_sub(in1, sc1, c);
+  if (NSUB > 2) c = pick_sub(in2, sc2, c);
   if (NSUB > 1 && !ROT) {
     c.q02 = c.d02;
     c.q13 = c.d13;
@@ -2841,222 +2972,146 @@ __device__ __forceinline__ SubConst pixel_const(uint32_t s, const SubConst &sc0,
 template <int NSUB, bool ROT>
 __device__ __forceinline__ void score_pixels(const Lane &L, const SubConst &sc0,
                                              const SubConst &sc1, const SubConst &sc2, float kf,
-                                             WeightFn wf, uint32_t nerr[3], uint64_t &nidx) {
-  uint32_t all = 0, idx[2] = {0, 0};
+                                             WeightFn wf, uint32_t &n0, uint32_t &n1,
+                                             uint32_t &n2, uint64_t &nidx) {
+  uint32_t all = 0, lo = 0, hi = 0;
+  n1 = n2 = 0;
 #pragma unroll
   for (int i = 0; i < 16; i++) {
-    const uint32_t s = NSUB == 1 ? 0u : (L.sub2 >> (2 * i)) & 3u;
-    const SubConst c = pixel_const<NSUB, ROT>(s, sc0, sc1, sc2);
+    const bool in1 = NSUB > 1 && (L.m12 & (1u << i)) != 0;
+    const bool in2 = NSUB > 2 && (L.m12 & (1u << (16 + i))) != 0;
+    const SubConst c = pixel_const<NSUB, ROT>(in1, in2, sc0, sc1, sc2);
     uint32_t best;
     const uint32_t me = pixel_err(L.px[2 * i], L.px[2 * i + 1], c, kf, wf, &best);
     all += me;
-    if (NSUB > 1) nerr[1] += s == 1 ? me : 0u;
-    if (NSUB == 3) nerr[2] += s == 2 ? me : 0u;
-    idx[i >> 3] |= best << (4 * (i & 7));
+    if (NSUB > 1) n1 += in1 ? me : 0u;
+    if (NSUB > 2) n2 += in2 ? me : 0u;
+    if (i < 8) lo |= best << (4 * i);
+    else hi |= best << (4 * (i - 8));
   }
-  nerr[0] = all - nerr[1] - nerr[2];
-  nidx = (uint64_t)idx[0] | ((uint64_t)idx[1] << 32);
+  n0 = all - n1 - n2;
+  nidx = (uint64_t)lo | ((uint64_t)hi << 32);
 }
 
 // The pixel pass under the nonuniform metric: float errors, each subset's
 // summed in pixel order (adding 0 to the other subsets' sums leaves them
 // unchanged).
-template <int NSUB>
 __device__ __forceinline__ void score_pixels_nu(const Lane &L, const SubConst &sc0,
                                                 const SubConst &sc1, const SubConst &sc2,
-                                                float kf, WeightFn wf, float nerr[3],
-                                                uint64_t &nidx) {
+                                                float kf, WeightFn wf, float &n0, float &n1,
+                                                float &n2, uint64_t &nidx) {
+  n0 = n1 = n2 = 0.0f;
+  nidx = 0;
 #pragma unroll
   for (int i = 0; i < 16; i++) {
-    const uint32_t s = NSUB == 1 ? 0u : (L.sub2 >> (2 * i)) & 3u;
-    const SubConst c = pixel_const<NSUB, true>(s, sc0, sc1, sc2);
+    const bool in1 = (L.m12 & (1u << i)) != 0, in2 = (L.m12 & (1u << (16 + i))) != 0;
+    const SubConst c = pixel_const<3, true>(in1, in2, sc0, sc1, sc2);
     uint32_t best;
     const float me = pixel_err_nu(L.px[2 * i], L.px[2 * i + 1], c, kf, wf, L.m, &best);
-    nerr[0] += s == 0 ? me : 0.0f;
-    if (NSUB > 1) nerr[1] += s == 1 ? me : 0.0f;
-    if (NSUB == 3) nerr[2] += s == 2 ? me : 0.0f;
+    n0 += in1 || in2 ? 0.0f : me;
+    n1 += in1 ? me : 0.0f;
+    n2 += in2 ? me : 0.0f;
     nidx |= (uint64_t)best << (4 * i);
   }
 }
 
-// The same pass split over a group of G lanes (G = 2, 4, 8 or 16, aligned in
-// the wave) that hold the same candidate: member m scores pixels m, m + G,
-// ...; the sums and index bits are combined over the group.  The per-subset
-// errors are integers, so the split does not change them.
-template <int NSUB>
-__device__ __forceinline__ void score_pixels_group(const Lane &L, const SubConst &sc0,
-                                                   const SubConst &sc1, const SubConst &sc2,
-                                                   float kf, WeightFn wf, uint32_t nerr[3],
-                                                   uint64_t &nidx, int G, int m) {
-  for (int i = m; i < 16; i += G) {
-    const uint32_t s = NSUB == 1 ? 0u : (L.sub2 >> (2 * i)) & 3u;
-    const SubConst c = pixel_const<NSUB, true>(s, sc0, sc1, sc2);
-    uint32_t best;
-    const uint32_t me = pixel_err(L.px[2 * i], L.px[2 * i + 1], c, kf, wf, &best);
-    nerr[0] += s == 0 ? me : 0u;
-    if (NSUB > 1) nerr[1] += s == 1 ? me : 0u;
-    if (NSUB == 3) nerr[2] += s == 2 ? me : 0u;
-    nidx |= (uint64_t)best << (4 * i);
-  }
-  uint32_t lo = (uint32_t)nidx, hi = (uint32_t)(nidx >> 32);
-  for (int off = 1; off < G; off <<= 1) {
-    nerr[0] += __shfl_xor(nerr[0], off);
-    if (NSUB > 1) nerr[1] += __shfl_xor(nerr[1], off);
-    if (NSUB == 3) nerr[2] += __shfl_xor(nerr[2], off);
-    lo |= __shfl_xor(lo, off);
-    hi |= __shfl_xor(hi, off);
-  }
-  nidx = (uint64_t)lo | ((uint64_t)hi << 32);
-}
-
-// AcceptNewEndpointError (Compressor.cpp:524-536) for err >= cur: accept when
-// frand() < exp(0.1 (cur - err) / temp), temp = energy / (q - 1).  The
-// probability is at most 1, so a draw rr in [1, 3) never accepts.
-__device__ __forceinline__ bool accept_worse(float rr, float cf, float ef, int q, int energy) {
-  if (!(rr < 1.0f)) return false;
-  // A single-precision estimate of the probability decides unless rr
-  // lies within 1e-4 (relative) of it, which covers the estimate's
-  // error; then the double expression of the reference decides.  The
-  // uniform metric's errors are integers below 2^24, so their float
-  // difference is exact; the nonuniform metric's are floats, whose
-  // difference has a relative error of at most 2^-23 where it is not
-  // exact, well inside the margin.
-  const float pf = __expf(__fdividef(0.1f * (cf - ef) * (float)(q - 1), (float)energy));
-  if (rr != 0.0f && rr < pf * 0.9999f) return true;
-  if (rr != 0.0f && rr > pf * 1.0001f) return false;
-  const float temp = (float)energy / (float)(q - 1);
-  const double pr = exp(((double)0.1f * ((double)cf - (double)ef)) / (double)temp);
-  return (double)rr < pr;
-}
-
-// One annealing step of every active subset.  Returns true when the
-// candidate is finished.  With GROUPED, the lanes of an aligned group of G
-// hold the same candidate and share the pixel pass (member m); every other
-// part of the step runs identically in each of them.
-template <bool GROUPED = false, bool NU = false>
-__device__ bool lane_step(Lane &L, uint32_t q, int G = 1, int m = 0) {
-  const Fit &f = L.f;
-  const int nb = 1 << f.nbits_idx;
-  uint32_t np1[3], np2[3], e1[3], e2[3];
-  int npbc[3];
-#pragma unroll
-  for (int s = 0; s < 3; s++) {
-    np1[s] = np2[s] = e1[s] = e2[s] = 0;
-    npbc[s] = 0;
-    if (!((L.active >> s) & 1)) continue;
-    Rng rng;
-    rng.x = L.rng[s];
-    pick_neighbor(f, rng, L.p1[s], L.p2[s], L.cpbc[s], np1[s], np2[s], npbc[s], L.bp1[s],
-                  L.bp2[s], L.bpbc[s]);
-    L.rng[s] = rng.x;
-    e1[s] = to_pixel_tab(np1[s], f, pbc_bit(f.pbit_type, npbc[s], 0));
-    e2[s] = to_pixel_tab(np2[s], f, pbc_bit(f.pbit_type, npbc[s], 1));
-  }
-  SubConst sc0 = sub_const(e1[0], e2[0]);
-  rotate_axis(sc0, L.ptmode, L.sel02, L.sel13);
-  const SubConst sc1 = sub_const(e1[1], e2[1]);
-  const SubConst sc2 = sub_const(e1[2], e2[2]);
-  uint32_t nerr[3] = {0, 0, 0};
-  uint64_t nidx = 0;
-  const float kf = (float)(nb - 1);
-  const WeightFn wf = weight_fn(nb);
-  // the widest subset count among the wave's running lanes picks the path
-  // (a wave-uniform branch): the list is ordered by mode, so most waves hold
-  // candidates of one subset count
+// One annealing step of every active subset, for waves whose running
+// candidates have at most NSUB subsets.  Every lane of the wave takes part.
+template <int NSUB, bool ROT, bool NU>
+__device__ __forceinline__ void lane_step_n(Lane &L, const uint8_t *quant, int q) {
+  const StepCfg k = step_cfg(L.cfg);
+  struct Next {
+    uint32_t p1 = 0, p2 = 0, pbc = 0, err = 0;
+  } n0, n1, n2;
+  auto propose = [&](SubState &t, int s, Next &n) {
+    pick_neighbor(k, (L.active >> s) & 1u, t, n.p1, n.p2, n.pbc);
+    return sub_const(step_quant(quant, k, n.p1, (n.pbc >> k.sh) & 1u),
+                     step_quant(quant, k, n.p2, n.pbc & 1u));
+  };
+  SubConst sc0 = propose(L.t0, 0, n0), sc1 = sc0, sc2 = sc0;
+  if (ROT) rotate_axis(sc0, L.ptmode, L.sel02, L.sel13);
+  if (NSUB > 1) sc1 = propose(L.t1, 1, n1);
+  if (NSUB > 2) sc2 = propose(L.t2, 2, n2);
+  uint64_t nidx;
   if constexpr (NU) {
-    float nerf[3] = {0.0f, 0.0f, 0.0f};
-    if (__ballot(L.nsub == 3)) score_pixels_nu<3>(L, sc0, sc1, sc2, kf, wf, nerf, nidx);
-    else if (__ballot(L.nsub == 2)) score_pixels_nu<2>(L, sc0, sc1, sc2, kf, wf, nerf, nidx);
-    else score_pixels_nu<1>(L, sc0, sc1, sc2, kf, wf, nerf, nidx);
-#pragma unroll
-    for (int s = 0; s < 3; s++) nerr[s] = __float_as_uint(nerf[s]);
-  } else if (GROUPED) {
-    if (__ballot(L.nsub == 3)) score_pixels_group<3>(L, sc0, sc1, sc2, kf, wf, nerr, nidx, G, m);
-    else if (__ballot(L.nsub == 2)) score_pixels_group<2>(L, sc0, sc1, sc2, kf, wf, nerr, nidx, G, m);
-    else score_pixels_group<1>(L, sc0, sc1, sc2, kf, wf, nerr, nidx, G, m);
-  } else if (!__ballot(L.nsub > 1)) {
-    score_pixels<1, true>(L, sc0, sc1, sc2, kf, wf, nerr, nidx);
-  } else if (__ballot(L.ptmode != 0)) {
-    score_pixels<3, true>(L, sc0, sc1, sc2, kf, wf, nerr, nidx);
-  } else if (__ballot(L.nsub == 3)) {
-    score_pixels<3, false>(L, sc0, sc1, sc2, kf, wf, nerr, nidx);
+    float e0, e1, e2;
+    score_pixels_nu(L, sc0, sc1, sc2, k.kf, k.wf, e0, e1, e2, nidx);
+    n0.err = __float_as_uint(e0);
+    n1.err = __float_as_uint(e1);
+    n2.err = __float_as_uint(e2);
   } else {
-    score_pixels<2, false>(L, sc0, sc1, sc2, kf, wf, nerr, nidx);
+    score_pixels<NSUB, ROT>(L, sc0, sc1, sc2, k.kf, k.wf, n0.err, n1.err, n2.err, nidx);
   }
-#pragma unroll
-  for (int s = 0; s < 3; s++) {
-    if (!((L.active >> s) & 1)) continue;
-    const uint32_t err = nerr[s];
-    bool accept = err < L.cur[s];
-    if (!accept) {
-      Rng rng;
-      rng.x = L.rng[s];
-      const float rr = rng.frand();
-      L.rng[s] = rng.x;
-      accept = accept_worse(rr, NU ? __uint_as_float(L.cur[s]) : (float)L.cur[s],
-                            NU ? __uint_as_float(err) : (float)err, (int)q, L.energy[s]);
-    }
-    if (accept) {
-      L.cur[s] = err;
-      L.p1[s] = np1[s];
-      L.p2[s] = np2[s];
-      L.cpbc[s] = npbc[s];
-    }
-    if (err < L.best[s]) {
-      // indices of this subset's pixels
-      const uint64_t m1 = (uint64_t)L.px[32] | ((uint64_t)L.px[33] << 32);
-      const uint64_t m2 = (uint64_t)L.px[34] | ((uint64_t)L.px[35] << 32);
-      const uint64_t m = s == 0 ? ~(m1 | m2) : (s == 1 ? m1 : m2);
-      L.idx = (L.idx & ~m) | (nidx & m);
-      L.bp1[s] = np1[s];
-      L.bp2[s] = np2[s];
-      L.bpbc[s] = npbc[s];
-      L.best[s] = err;
-      L.energy[s] = 0;
-    }
-    L.energy[s]++;
-    if (!(L.best[s] > 0 && L.energy[s] < (int)q)) L.active &= ~(1u << s);
+  // index bits of the subsets whose best state is replaced
+  const uint64_t m1 = NSUB > 1 ? (uint64_t)L.px[32] | ((uint64_t)L.px[33] << 32) : 0;
+  const uint64_t m2 = NSUB > 2 ? (uint64_t)L.px[34] | ((uint64_t)L.px[35] << 32) : 0;
+  uint64_t taken = 0;
+  auto finish = [&](SubState &t, int s, const Next &n, uint64_t mine) {
+    bool live = (L.active >> s) & 1u;
+    const uint32_t was = live ? 1u << s : 0u;
+    const bool better = finish_step<NU>(t, live, n.err, n.p1, n.p2, n.pbc, q);
+    taken |= better ? mine : 0ull;
+    if (!live) L.active &= ~was;
+  };
+  finish(L.t0, 0, n0, ~(m1 | m2));
+  if (NSUB > 1) finish(L.t1, 1, n1, m1);
+  if (NSUB > 2) finish(L.t2, 2, n2, m2);
+  L.idx = (L.idx & ~taken) | (nidx & taken);
+}
+
+// The widest subset count among the wave's running lanes picks the compiled
+// step (a wave-uniform branch): the list is ordered by mode, so most waves
+// hold candidates of one subset count.
+template <bool NU>
+__device__ __forceinline__ void lane_step(Lane &L, const uint8_t *quant, int q) {
+  if constexpr (NU) {
+    lane_step_n<3, true, true>(L, quant, q);
+  } else {
+    const bool run = L.active != 0;
+    if (!__ballot(run && L.nsub > 1)) lane_step_n<1, true, false>(L, quant, q);
+    else if (__ballot(run && L.ptmode != 0)) lane_step_n<3, true, false>(L, quant, q);
+    else if (__ballot(run && L.nsub == 3)) lane_step_n<3, false, false>(L, quant, q);
+    else lane_step_n<2, false, false>(L, quant, q);
   }
-  return L.active == 0;
 }
 
 template <bool NU = false>
-__device__ void lane_finish(Lane &L, Work &w) {
+__device__ __forceinline__ void lane_finish(Lane &L, Work &w) {
   CandRec *rc = &w.rec[L.id];
-  const Fit &f = L.f;
+  Fit f;
+  set_fit(f, L.info & 7, (L.info >> 3) & 3, (L.info >> 5) & 1);
   uint32_t total = L.extra;
   // nonuniform metric: the reference's double total, subsets in order, then
   // the alpha term of a rotation mode (Compressor.cpp:918, 1300-1371)
   double tnu = 0.0;
   uint32_t pbcs = rc->meta & 0x3Fu;
-  for (int s = 0; s < L.nsub; s++) {
-    const uint32_t bp1 = s == 0 ? L.bp1[0] : (s == 1 ? L.bp1[1] : L.bp1[2]);
-    const uint32_t bp2 = s == 0 ? L.bp2[0] : (s == 1 ? L.bp2[1] : L.bp2[2]);
-    const int pb = s == 0 ? L.bpbc[0] : (s == 1 ? L.bpbc[1] : L.bpbc[2]);
-    const uint32_t be = s == 0 ? L.best[0] : (s == 1 ? L.best[1] : L.best[2]);
-    total += be;
+  auto put = [&](const SubState &t, int s) {
+    if (s >= L.nsub) return;
+    total += t.best;
     if constexpr (NU) {
-      double e = (double)__uint_as_float(be);
+      double e = (double)__uint_as_float(t.best);
       if ((L.scf >> s) & 1) {
-        int n = 0;
-#pragma unroll
-        for (int i = 0; i < 16; i++) n += ((L.sub2 >> (2 * i)) & 3) == (uint32_t)s ? 1 : 0;
-        e = (double)n * e;
+        const int n1 = __popc(L.m12 & 0xFFFFu), n2 = __popc(L.m12 >> 16);
+        e = (double)(s == 0 ? 16 - n1 - n2 : (s == 1 ? n1 : n2)) * e;
       }
       tnu += e;
     }
+    const int pb = (int)t.bpbc;
     const int pb0 = f.pbit_type == PB_NONE ? -1 : pbc_bit(f.pbit_type, pb, 0);
     const int pb1 = f.pbit_type == PB_NONE ? -1 : pbc_bit(f.pbit_type, pb, 1);
-    uint32_t e1 = to_pixel_int(bp1, f.qmask, pb0);
-    uint32_t e2 = to_pixel_int(bp2, f.qmask, pb1);
-    if (kModes[f.mode].has_rot) {
+    uint32_t e1 = to_pixel_int(t.bp1, f.qmask, pb0);
+    uint32_t e2 = to_pixel_int(t.bp2, f.qmask, pb1);
+    if (L.ptmode) {
       e1 = (e1 & 0x00FFFFFFu) | (rc->px1[0] & 0xFF000000u);
       e2 = (e2 & 0x00FFFFFFu) | (rc->px2[0] & 0xFF000000u);
     }
     rc->px1[s] = e1;
     rc->px2[s] = e2;
     pbcs = (pbcs & ~(3u << (2 * s))) | ((uint32_t)pb << (2 * s));
-  }
+  };
+  put(L.t0, 0);
+  put(L.t1, 1);
+  put(L.t2, 2);
   rc->cidx_lo = (uint32_t)L.idx;
   rc->cidx_hi = (uint32_t)(L.idx >> 32);
   rc->meta = (rc->meta & ~0x3Fu) | pbcs | kMetaAnnealed;
@@ -3064,462 +3119,266 @@ __device__ void lane_finish(Lane &L, Work &w) {
   if constexpr (NU) w.nu_total[L.id] = tnu + L.extra_nu;
 }
 
-// A wave with at most this many candidates left after the list is used up
-// finishes them in lane groups.
-constexpr int kTailLanes = 16;
-// Lanes per candidate for the rotation modes (4 and 5), whose annealing
-// chains are the longest (hundreds to over a thousand steps against tens for
-// the other modes): run one lane each, they would set the launch's length.
-// Pairs split the pixel pass in two; every member repeats the rest of the
-// step, so larger groups shorten a step less than they cost (measured: 4
-// and 8 lanes slower overall).
-constexpr int kRotGroup = 2;
+// A candidate in the middle of its annealing, handed from the one-lane form
+// to the one-lane-per-pixel form.
+struct TailState {
+  uint32_t id, info;  // info: AState's, with the subsets still annealing
+  uint32_t extra, pbc;  // pbc: 2 bits per subset, current then (<< 6) best
+  uint32_t p1[3], p2[3], bp1[3], bp2[3], cur[3], best[3], energy[3], x[3];
+  uint32_t idx_lo, idx_hi;
+  uint32_t pad[2];
+};
+static_assert(sizeof(TailState) == 128, "TailState");
+
+__device__ __forceinline__ void lane_hand_over(const Lane &L, TailState &o) {
+  o.id = L.id;
+  o.info = (L.info & ~(7u << 14)) | (L.active << 14);
+  o.extra = L.extra;
+  uint32_t pbc = 0;
+  auto put = [&](const SubState &t, int s) {
+    o.p1[s] = t.p1;
+    o.p2[s] = t.p2;
+    o.bp1[s] = t.bp1;
+    o.bp2[s] = t.bp2;
+    o.cur[s] = t.cur;
+    o.best[s] = t.best;
+    o.energy[s] = (uint32_t)t.energy;
+    o.x[s] = t.x;
+    pbc |= (t.cpbc << (2 * s)) | (t.bpbc << (6 + 2 * s));
+  };
+  put(L.t0, 0);
+  put(L.t1, 1);
+  put(L.t2, 2);
+  o.pbc = pbc;
+  o.idx_lo = (uint32_t)L.idx;
+  o.idx_hi = (uint32_t)(L.idx >> 32);
+}
+
+// Idle lanes of a wave at which it loads new candidates: loading and
+// finishing cost a whole wave's issue however few lanes do it, idle lanes
+// waste their share of every step.  Measured at 4096 x 4096: 4 lanes 28.1 ms
+// (reference search) and 3.29 ms (learned), 8 28.5 and 3.31, 12 28.9 and 3.36,
+// 16 29.4 and 3.39; looking after every step and loading at one idle lane:
+// 33.8 and 4.0.
+constexpr int kRefillLanes = 4;
 // The wave mask of each group's first lane (lanes 0, g, 2g, ...).
 constexpr uint64_t group_leaders(int g, int lane = 0) {
   return lane >= 64 ? 0ull : (1ull << lane) | group_leaders(g, lane + g);
 }
-static_assert(group_leaders(2) == 0x5555555555555555ull && group_leaders(4) == 0x1111111111111111ull,
-              "group leaders");
+static_assert(group_leaders(16) == 0x0001000100010001ull, "group leaders");
 
-// UNROLL annealing steps run between refills of finished lanes.
-// WAVES: the minimum waves per SIMD the register allocation must allow.  3
-// (168 VGPRs, a small spill) suits both searches since the annealing step's
-// quantisation became table loads (before, the learned search ran alike at 2
-// and 3 waves per SIMD: 7.66 and 7.70 ms; now 6.08 and 5.78 ms).
-// NU: the nonuniform metric (float errors; the tail below, which splits a
-// candidate's pixel sums over lanes, would change their order and is not
-// used: the lanes finish their own candidates).
-// COUNT: also count the work into prm.work_counts: [0] the QuantizedError
-// point evaluations the reference's annealing makes (each step of a subset
-// scores that subset's points, Compressor.cpp:583-624), [1] the pixel scores
-// this kernel makes (16 per step of a candidate, whichever subsets are
-// still annealing).
-template <int UNROLL, int WAVES, bool NU = false, bool COUNT = false>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WAVES)))
-anneal_kernel(BlockRange r, Bc7Params prm, Work w) {
-  const int lane = threadIdx.x;
-  unsigned long long n_ref = 0, n_gpu = 0;  // COUNT
-  auto count_step = [&](const Lane &x) {
-    // points of the subsets still annealing: the subset codes' low and high
-    // bits give the sizes of subsets 1 and 2
-    const uint32_t lo = x.sub2 & 0x55555555u, hi = (x.sub2 >> 1) & 0x55555555u;
-    const uint32_t n1 = (uint32_t)__popc(lo & ~hi), n2 = (uint32_t)__popc(hi & ~lo);
-    const uint32_t n0 = 16u - n1 - n2;
-    n_ref += ((x.active & 1u) ? n0 : 0u) + ((x.active & 2u) ? n1 : 0u) +
-             ((x.active & 4u) ? n2 : 0u);
-    n_gpu += 16u;
-  };
-  auto flush_counts = [&]() {
-    if constexpr (COUNT) {
-      for (int off = 32; off >= 1; off >>= 1) {
-        n_ref += __shfl_xor(n_ref, off);
-        n_gpu += __shfl_xor(n_gpu, off);
-      }
-      if (lane == 0) {
-        atomicAdd(&prm.work_counts[0], n_ref);
-        atomicAdd(&prm.work_counts[1], n_gpu);
-      }
-    }
-  };
-  const uint64_t lt = (1ull << lane) - 1ull;
-  const uint32_t listed = *(volatile uint32_t *)&w.counters[w.alist ? 18 : 16];
-  // per lane 16 texels (two words each) and the subsets' index bits, odd row
-  // stride: conflict-free
-  __shared__ uint32_t s_px[64 * kRowWords];
-  // Learned search: the list is in state order, and the set-up kernels
-  // append the rotation modes' states last (counters[19] holds the first of
-  // them): the list's rotation states are its suffix from rot_begin.  (The
-  // full search's list is mostly rotation states, whose grouped steps would
-  // cost more than its short tail: it runs them one lane each.)
-  uint32_t rot_begin = listed;
-  if (!NU && w.alist) {
-    const uint32_t first_rot = *(volatile uint32_t *)&w.counters[19];
-    uint32_t lo = 0, hi = listed;  // first list entry >= first_rot
-    while (lo < hi) {
-      const uint32_t mid = (lo + hi) >> 1;
-      if (w.alist[mid] < first_rot) lo = mid + 1;
-      else hi = mid;
-    }
-    rot_begin = lo;
-  }
-  // Phase A, in the first eighth of the launch (a quarter of the waves that
-  // fit at once): the rotation states in groups of kRotGroup lanes that
-  // share each step's pixel pass (every member holds the same state and
-  // texels), fetched from the end of the suffix.  A group that finishes
-  // takes the next; once the suffix is used up the wave's groups finish
-  // theirs and the wave joins phase B.  The other waves start on phase B at
-  // once, so the longest chains run from the start, with shorter steps,
-  // while the rest of the list proceeds beside them.
-  if (!NU && rot_begin < listed && blockIdx.x < (gridDim.x + 7) / 8) {
-    const uint32_t nrot = listed - rot_begin;
-    const int m = lane % kRotGroup;
-    constexpr uint64_t leaders = group_leaders(kRotGroup);
-    Lane T;
-    T.px = s_px + lane * kRowWords;
-    T.has = false;
-    uint32_t abase = 0, aend = 0;
-    bool aexh = false;
-    for (;;) {
-      for (;;) {
-        const uint64_t need = __ballot(!T.has) & leaders;
-        if (!need || aexh) break;
-        if (abase >= aend) {
-          uint32_t b0 = 0;
-          if (lane == 0) b0 = atomicAdd(&w.counters[21], 16u);
-          b0 = __shfl(b0, 0);
-          if (b0 >= nrot) {
-            aexh = true;
-            break;
-          }
-          abase = b0;
-          aend = min(b0 + 16u, nrot);
-        }
-        const uint32_t avail = aend - abase;
-        // rank of this lane's group among the groups that need a state
-        const uint64_t below = (1ull << (lane & ~(kRotGroup - 1))) - 1ull;
-        const uint32_t rank = (uint32_t)__popcll(need & below);
-        const bool wants = ((need >> (lane & ~(kRotGroup - 1))) & 1) != 0;
-        if (wants && !T.has && rank < avail) {
-          const uint32_t item = listed - 1u - (abase + rank);
-          lane_load<NU>(T, r, prm, w.astate[w.alist ? w.alist[item] : item]);
-        }
-        abase += min(avail, (uint32_t)__popcll(need));
-      }
-      if (!__ballot(T.has)) break;
-      for (int u = 0; u < UNROLL; u++) {
-        if (T.has) {
-          if constexpr (COUNT) {
-            if (m == 0) count_step(T);
-          }
-          if (lane_step<true>(T, prm.quality, kRotGroup, m)) {
-            if (m == 0) lane_finish(T, w);
-            T.has = false;
-          }
-        }
-      }
-    }
-  }
-  // Phase B: the other states, one lane each, from the end of the prefix
-  const uint32_t total = rot_begin;
-  Lane L;
-  L.px = s_px + lane * kRowWords;
-  L.has = false;
-  uint32_t wbase = 0, wend = 0;  // wave-local window of the list
-  bool exhausted = false;
-  for (;;) {
-    // the list is used up and few candidates remain: the tail below
-    if (!NU && exhausted && __popcll(__ballot(L.has)) <= kTailLanes) break;
-    // refill idle lanes from the window, fetching a new window when needed
-    for (;;) {
-      const uint64_t need = __ballot(!L.has);
-      if (!need || exhausted) break;
-      if (wbase >= wend) {
-        uint32_t b0 = 0;
-        if (lane == 0) b0 = atomicAdd(&w.counters[17], 64u);
-        b0 = __shfl(b0, 0);
-        if (b0 >= total) {
-          exhausted = true;
-          break;
-        }
-        wbase = b0;
-        wend = min(b0 + 64u, total);
-      }
-      const uint32_t avail = wend - wbase;
-      const uint32_t rank = (uint32_t)__popcll(need & lt);
-      if (!L.has && rank < avail) {
-        // the list runs from its end: the set-up kernels append modes 0, 2,
-        // 3, 7, 6, 1, 4, 5.  The rotation modes' candidates anneal the
-        // longest, so the full search starts with them; then come the
-        // numerous mode-1 candidates, and the short mode-7 chains are among
-        // the last loaded, which keeps the tail of the launch short
-        const uint32_t item = total - 1u - (wbase + rank);
-        lane_load<NU>(L, r, prm, w.astate[w.alist ? w.alist[item] : item]);
-      }
-      wbase += min(avail, (uint32_t)__popcll(need));
-    }
-    if (!__ballot(L.has)) break;
-    for (int u = 0; u < UNROLL; u++) {
-      if (L.has) {
-        if constexpr (COUNT) count_step(L);
-        if (lane_step<false, NU>(L, prm.quality)) {
-          lane_finish<NU>(L, w);
-          L.has = false;
-        }
-      }
-    }
-  }
-  if constexpr (NU) {
-    flush_counts();
-    return;
-  }
-  // Tail: the wave's last candidates (at most kTailLanes) each get a group
-  // of G lanes that share the pixel pass of every step, so the longest
-  // anneals, which set the launch's length, run up to G times fewer
-  // instructions per step.  Their texels stay in the LDS rows of the lanes
-  // that loaded them.
-  const uint64_t act = __ballot(L.has);
-  const int na = __popcll(act);
-  if (na == 0) {
-    flush_counts();
-    return;
-  }
-  __shared__ Lane s_tail[kTailLanes];
-  __shared__ uint32_t s_row[kTailLanes];
-  if (L.has) {
-    const int k = __popcll(act & lt);
-    s_tail[k] = L;
-    s_row[k] = (uint32_t)lane;
-  }
-  __syncthreads();
-  const int G = na <= 4 ? 16 : (na <= 8 ? 8 : 4);
-  const int g = lane / G, m = lane % G;
-  Lane T;
-  T.has = false;
-  if (g < na) {
-    T = s_tail[g];
-    T.px = s_px + s_row[g] * kRowWords;
-  }
-  while (__ballot(T.has)) {
-    for (int u = 0; u < UNROLL; u++) {
-      if (T.has) {
-        if constexpr (COUNT) {
-          if (m == 0) count_step(T);  // the group scores the 16 pixels once
-        }
-        if (lane_step<true>(T, prm.quality, G, m)) {
-          if (m == 0) lane_finish(T, w);
-          T.has = false;
-        }
-      }
-    }
-  }
-  flush_counts();
-}
+// Groups still running at which a wave of the four-lane form hands over.
+constexpr int kHandGroups = 4;
 
 // ---------------------------------------------------------------------------
-// Kernel 3b: the same annealing with one lane per pixel.  A row of 16 lanes
-// holds one candidate; a lane holds its own pixel and the state of its own
-// subset only (every lane of a subset computes the same step), so a step is
-// one pixel's work plus three row sums instead of sixteen pixels' work for
-// up to three subsets: about a quarter of the instructions, and of the
-// latency, of a step of the one-lane form.  A wave advances four candidates
-// where the one-lane form advances 64, so per candidate the step costs about
-// four times more issue: this form is for lists that leave the chip idle,
-// where the longest chain sets the time.
+// The same annealing with G lanes per candidate.  G = 16: a row of 16 lanes
+// holds one candidate, a lane its own pixel and the state of its own subset
+// only (every lane of a subset computes the same step), so a step is one
+// pixel's work plus three row sums instead of sixteen pixels' work for up to
+// three subsets: about a quarter of the instructions, and of the latency, of
+// a step of the one-lane form.  A wave advances four candidates where the
+// one-lane form advances 64, so per candidate a step costs about four times
+// more issue: this form is for lists that leave the chip idle, where the
+// longest chain sets the time.  G = 4: candidates of one subset only, four
+// pixels a lane, between the two in both respects.
 // ---------------------------------------------------------------------------
-// kQuant's rows for the annealing's precisions (0, 4..8 bits) and p-bits, in
-// LDS: an L1 hit of the global table costs a step several times more latency.
-constexpr int kSpreadQuantRows = 6 * 2;
-__device__ __forceinline__ uint32_t spread_quant_row(int bits) {
-  return (uint32_t)(bits ? bits - 3 : 0) * 512u;
-}
-__device__ __forceinline__ void spread_quant_load(uint8_t *lds) {
-  uint32_t *dst = reinterpret_cast<uint32_t *>(lds);
-  for (int t = threadIdx.x; t < kSpreadQuantRows * 64; t += blockDim.x) {
-    const int row = t >> 6, bits = row < 2 ? 0 : (row >> 1) + 3, pb = row & 1;
-    dst[t] = reinterpret_cast<const uint32_t *>(kQuant)[(bits * 3 + pb + 1) * 64 + (t & 63)];
+// Sum over the G lanes of a group (every lane of the wave active).
+template <int G>
+__device__ __forceinline__ uint32_t group_sum(uint32_t v) {
+  if (G == 16) {
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xf, 0xf, true);  // row_ror:8
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x124, 0xf, 0xf, true);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x122, 0xf, 0xf, true);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x121, 0xf, 0xf, true);
+  } else {
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4e, 0xf, 0xf, true);  // quad 2,3,0,1
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xb1, 0xf, 0xf, true);  // quad 1,0,3,2
   }
-}
-
-// Sum over the 16 lanes of a row (every lane of the wave active).
-__device__ __forceinline__ uint32_t row_sum(uint32_t v) {
-  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xf, 0xf, true);  // row_ror:8
-  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x124, 0xf, 0xf, true);
-  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x122, 0xf, 0xf, true);
-  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x121, 0xf, 0xf, true);
   return v;
 }
 
-// COUNT: the work counters of anneal_kernel, in the same units.
-template <bool COUNT>
-__global__ void __launch_bounds__(256) anneal_spread_kernel(BlockRange r, Bc7Params prm, Work w) {
-  __shared__ __align__(4) uint8_t s_quant[kSpreadQuantRows * 256];
-  spread_quant_load(s_quant);
-  __syncthreads();
-  const int lane = threadIdx.x & 63, px = lane & 15, row0 = lane & 48;
-  const uint32_t total = *(volatile uint32_t *)&w.counters[w.alist ? 18 : 16];
+// Runs the candidates [begin, end) of a list, taken from its end through
+// *fetch, until none is left.  SRC: kFromList (the annealing states),
+// kFromTail (the candidates handed over in `tail`) or kFromListHand (the
+// annealing states; once they are used up a wave with few groups running
+// hands them over through `tail` and returns).
+// Called by whole waves.  COUNT: the work counters of anneal_kernel.
+enum { kFromList = 0, kFromTail = 1, kFromListHand = 2 };
+
+template <int G, int SRC, bool COUNT>
+__device__ __forceinline__ void spread_run(const BlockRange &r, const Bc7Params &prm,
+                                           const Work &w, TailState *tail, const uint8_t *quant,
+                                           uint32_t begin, uint32_t end, uint32_t *fetch,
+                                           unsigned long long &n_ref, unsigned long long &n_gpu) {
+  static_assert(G == 16 || G == 4, "lanes per candidate");
+  constexpr int P = 16 / G;  // pixels per lane
+  constexpr bool kTail = SRC == kFromTail;
+  constexpr uint64_t kLeaders = group_leaders(G);
+  constexpr uint64_t kGroup = (1ull << G) - 1ull;
+  const int lane = threadIdx.x & 63, m = lane & (G - 1), lead = lane & ~(G - 1);
   const int q = (int)prm.quality;
-  constexpr uint64_t kRowLeaders = group_leaders(16);
-  uint32_t n_ref = 0, n_gpu = 0;  // COUNT
-  // the candidate (the same in the row)
+  const uint32_t total = end - begin;
+  // the candidate (the same in the group) and its constants
   bool has = false;
-  uint32_t id = 0, info = 0, extra = 0;
-  // its constants
-  uint32_t s02 = 0, s13 = 0, k2_02 = 0, k2_13 = 0, qc = 0, qa = 0, sel02 = 0, sel13 = 0;
-  uint32_t flip = 0, nopb = 0, sh = 0;
+  uint32_t id = 0, info = 0, extra = 0, sel02 = 0, sel13 = 0;
   int ptmode = 0, nsub = 1;
-  float kf = 0.0f;
-  WeightFn wf = {0, 0};
-  // this lane's pixel, its subset and that subset's state
-  uint32_t p02 = 0, p13 = 0, sub = 0, bidx = 0;
+  StepCfg k = step_cfg(0);
+  // this lane's pixels m * P .., their subset and that subset's state
+  uint32_t p02[P] = {}, p13[P] = {}, sub = 0, bidx = 0;
   bool active = false;
-  uint32_t p1 = 0, p2 = 0, bp1 = 0, bp2 = 0, cur = 0, best = 0, cpbc = 0, bpbc = 0, x = 0;
-  int energy = 0;
+  SubState t = {};
   bool exhausted = total == 0;
   for (;;) {
-    // idle rows take the next candidates, from the end of the list (the
+    // idle groups take the next candidates, from the end of the list (the
     // rotation modes, whose chains are the longest, first)
-    uint64_t hasm = __ballot(has);
-    const uint64_t need = ~hasm & kRowLeaders;
+    uint64_t hasm = __ballot(has) & kLeaders;
+    const uint64_t need = ~hasm & kLeaders;
     if (need && !exhausted) {
       const uint32_t want = (uint32_t)__popcll(need);
       uint32_t base = 0;
-      if (lane == 0) base = atomicAdd(&w.counters[17], want);
+      if (lane == 0) base = atomicAdd(fetch, want);
       base = __shfl(base, 0);
       if (base >= total || total - base <= want) exhausted = true;
-      const uint32_t item = base + (uint32_t)__popcll(need & ((1ull << row0) - 1ull));
+      const uint32_t item = base + (uint32_t)__popcll(need & ((1ull << lead) - 1ull));
       if (!has && item < total) {
-        const uint32_t at = total - 1u - item;
-        const AState &st = w.astate[w.alist ? w.alist[at] : at];
+        const uint32_t at = end - 1u - item;
+        const TailState *ts = kTail ? tail + at : nullptr;
+        const AState *st = kTail ? nullptr : w.astate + (w.alist ? w.alist[at] : at);
         has = true;
-        id = st.id;
-        info = st.info;
-        extra = st.extra_err;
+        id = kTail ? ts->id : st->id;
+        info = kTail ? ts->info : st->info;
+        extra = kTail ? ts->extra : st->extra_err;
         const int mode = info & 7, rot = (info >> 3) & 3, im = (info >> 5) & 1;
         const int shape = (info >> 8) & 63;
-        nsub = (info >> 6) & 3;
         Fit f;
         set_fit(f, mode, rot, im);
+        k = step_cfg(step_cfg_pack(f));
         ptmode = kModes[mode].has_rot ? rot + 1 : 0;
         rotation_selectors(ptmode, sel02, sel13);
-        const uint32_t cs = 1u << (8 - f.color_prec);
-        const uint32_t as = mode < 4 ? 0u : 1u << (8 - f.alpha_prec);
-        const bool has_pb = f.pbit_type != PB_NONE;
-        s02 = cs | (cs << 16);
-        s13 = cs | (as << 16);
-        k2_02 = has_pb ? s02 : s02 << 1;
-        k2_13 = has_pb ? s13 : s13 << 1;
-        nopb = has_pb ? 0u : 1u;
-        flip = f.pbit_type == PB_SHARED ? 1u : (has_pb ? 3u : 0u);
-        sh = f.pbit_type == PB_NOTSHARED ? 1u : 0u;
-        qc = spread_quant_row(f.color_prec);
-        qa = spread_quant_row(f.alpha_prec);
-        const int nb = 1 << f.nbits_idx;
-        kf = (float)(nb - 1);
-        wf = weight_fn(nb);
-        sub = 0;
-        if (nsub == 2) sub = (kShape2[shape] >> px) & 1u;
-        if (nsub == 3) sub = subset_of(kShape3[shape][0], kShape3[shape][1], px);
+        if (G == 16) {
+          nsub = (info >> 6) & 3;
+          sub = 0;
+          if (nsub == 2) sub = (kShape2[shape] >> m) & 1u;
+          if (nsub == 3) sub = subset_of(kShape3[shape][0], kShape3[shape][1], m);
+        }
         const uint32_t rel = id_block(id), b = r.first_block + rel;
         const uint32_t bx = b % r.blocks_wide, by = b / r.blocks_wide;
-        const uint32_t pix =
-            r.img[(size_t)(by * 4 + (px >> 2)) * r.width + bx * 4 + (px & 3)];
-        p02 = pair02x64(pix);
-        p13 = pair13x64(pix);
-        p1 = bp1 = st.p1[sub];
-        p2 = bp2 = st.p2[sub];
-        cur = best = st.err[sub];
-        cpbc = bpbc = (st.pbc >> (2 * sub)) & 3u;
-        bidx = idx_at(st.idx_lo, st.idx_hi, px);
-        energy = 0;
+        const uint32_t *src =
+            r.img + (size_t)(by * 4 + (m * P >> 2)) * r.width + bx * 4 + ((m * P) & 3);
+#pragma unroll
+        for (int i = 0; i < P; i++) {
+          const uint32_t pix = src[i];
+          p02[i] = pair02x64(pix);
+          p13[i] = pair13x64(pix);
+        }
         active = (info >> (14 + sub)) & 1u;
-        x = fit_key(prm.seed, prm.block_id_base + b,
-                    cand_tag(mode, (int)((info >> 17) & 7), (int)sub, rot, im));
+        const uint32_t pbc = kTail ? ts->pbc : st->pbc;
+        t.p1 = kTail ? ts->p1[sub] : st->p1[sub];
+        t.p2 = kTail ? ts->p2[sub] : st->p2[sub];
+        t.bp1 = kTail ? ts->bp1[sub] : t.p1;
+        t.bp2 = kTail ? ts->bp2[sub] : t.p2;
+        t.cur = kTail ? ts->cur[sub] : st->err[sub];
+        t.best = kTail ? ts->best[sub] : t.cur;
+        t.cpbc = (pbc >> (2 * sub)) & 3u;
+        t.bpbc = kTail ? (pbc >> (6 + 2 * sub)) & 3u : t.cpbc;
+        t.energy = kTail ? (int)ts->energy[sub] : 0;
+        t.x = kTail ? ts->x[sub]
+                    : fit_key(prm.seed, prm.block_id_base + b,
+                              cand_tag(mode, (int)((info >> 17) & 7), (int)sub, rot, im));
+        const uint64_t idx = kTail ? (uint64_t)ts->idx_lo | ((uint64_t)ts->idx_hi << 32)
+                                   : (uint64_t)st->idx_lo | ((uint64_t)st->idx_hi << 32);
+        bidx = (uint32_t)(idx >> (4 * P * m)) & ((1u << (4 * P)) - 1u);
       }
-      hasm = __ballot(has);
+      hasm = __ballot(has) & kLeaders;
     }
     if (!hasm) break;
-    const bool multi = __ballot(nsub > 1) != 0;  // stale in rows without a candidate: harmless
+    if (SRC == kFromListHand && exhausted && __popcll(hasm) <= kHandGroups) {
+      uint32_t base = 0;
+      if (lane == 0) base = atomicAdd(&w.counters[22], (uint32_t)__popcll(hasm));
+      base = __shfl(base, 0);
+      if (has) {
+        TailState &o = tail[base + (uint32_t)__popcll(hasm & ((1ull << lead) - 1ull))];
+        if (m == 0) {
+          o.id = id;
+          o.info = info;  // one subset, still active
+          o.extra = extra;
+          o.pbc = t.cpbc | (t.bpbc << 6);
+          o.p1[0] = t.p1;
+          o.p2[0] = t.p2;
+          o.bp1[0] = t.bp1;
+          o.bp2[0] = t.bp2;
+          o.cur[0] = t.cur;
+          o.best[0] = t.best;
+          o.energy[0] = (uint32_t)t.energy;
+          o.x[0] = t.x;
+        }
+        reinterpret_cast<uint16_t *>(&o.idx_lo)[m] = (uint16_t)bidx;
+      }
+      break;
+    }
+    // stale in rows without a candidate: harmless
+    const bool multi = G == 16 && __ballot(nsub > 1) != 0;
     for (int u = 0; u < 4; u++) {
       if constexpr (COUNT) {
         const uint64_t act = __ballot(active);
-        n_ref += active ? 1u : 0u;
-        n_gpu += (px == 0 && ((act >> row0) & 0xFFFFull)) ? 16u : 0u;
+        n_ref += active ? (unsigned)P : 0u;
+        n_gpu += (m == 0 && ((act >> lead) & kGroup)) ? 16u : 0u;
       }
-      // the neighbour (pick_neighbor): draws for endpoint 2, then 1
-      uint32_t np1 = 0, np2 = 0;
-      const uint32_t npbc = cpbc ^ flip;
-      const uint32_t up2 = ((cpbc >> sh) & 1u) | nopb, up1 = (cpbc & 1u) | nopb;
-      const s16x2 k02 = as_s16x2(k2_02), k13 = as_s16x2(k2_13);
-      bool again = true;
-      for (int tries = 0; tries < 16; tries++) {
-        if (again) {
-          Rng rng;
-          rng.x = x;
-          np2 = step_endpoint(p2, rng.next(), as_s16x2(up2 ? s02 : 0u), as_s16x2(up2 ? s13 : 0u),
-                              k02, k13);
-          np1 = step_endpoint(p1, rng.next(), as_s16x2(up1 ? s02 : 0u), as_s16x2(up1 ? s13 : 0u),
-                              k02, k13);
-          x = rng.x;
-          again = active && np1 == bp1 && np2 == bp2 && npbc == bpbc;
-        }
-        if (!__ballot(again)) break;
-      }
-      // its error, this lane's pixel
-      const uint32_t o1 = ((npbc >> sh) & 1u) << 8, o2 = (npbc & 1u & (flip ? 1u : 0u)) << 8;
-      const uint8_t *c1 = s_quant + qc + o1, *c2 = s_quant + qc + o2;
-      const uint32_t e1 = (uint32_t)c1[chan(np1, 0)] | ((uint32_t)c1[chan(np1, 1)] << 8) |
-                          ((uint32_t)c1[chan(np1, 2)] << 16) |
-                          ((uint32_t)s_quant[qa + o1 + chan(np1, 3)] << 24);
-      const uint32_t e2 = (uint32_t)c2[chan(np2, 0)] | ((uint32_t)c2[chan(np2, 1)] << 8) |
-                          ((uint32_t)c2[chan(np2, 2)] << 16) |
-                          ((uint32_t)s_quant[qa + o2 + chan(np2, 3)] << 24);
-      SubConst sc = sub_const(e1, e2);
+      uint32_t np1, np2, npbc;
+      pick_neighbor(k, active, t, np1, np2, npbc);
+      SubConst sc = sub_const(step_quant(quant, k, np1, (npbc >> k.sh) & 1u),
+                              step_quant(quant, k, np2, npbc & 1u));
       rotate_axis(sc, ptmode, sel02, sel13);
-      uint32_t j;
-      const uint32_t me = pixel_err(p02, p13, sc, kf, wf, &j);
+      uint32_t me = 0, nidx = 0;
+#pragma unroll
+      for (int i = 0; i < P; i++) {
+        uint32_t j;
+        me += pixel_err(p02[i], p13[i], sc, k.kf, k.wf, &j);
+        nidx |= j << (4 * i);
+      }
       // its subset's error
-      uint32_t err = row_sum(me);
+      uint32_t err = group_sum<G>(me);
       if (multi) {
-        const uint32_t t1 = row_sum(sub == 1 ? me : 0u), t2 = row_sum(sub == 2 ? me : 0u);
+        const uint32_t t1 = group_sum<G>(sub == 1 ? me : 0u);
+        const uint32_t t2 = group_sum<G>(sub == 2 ? me : 0u);
         err = sub == 0 ? err - t1 - t2 : (sub == 1 ? t1 : t2);
       }
-      if (active) {
-        bool accept = err < cur;
-        if (!accept) {
-          Rng rng;
-          rng.x = x;
-          const float rr = rng.frand();
-          x = rng.x;
-          accept = accept_worse(rr, (float)cur, (float)err, q, energy);
-        }
-        if (accept) {
-          cur = err;
-          p1 = np1;
-          p2 = np2;
-          cpbc = npbc;
-        }
-        if (err < best) {
-          best = err;
-          bp1 = np1;
-          bp2 = np2;
-          bpbc = npbc;
-          bidx = j;
-          energy = 0;
-        }
-        energy++;
-        active = best > 0 && energy < q;
-      }
+      if (finish_step(t, active, err, np1, np2, npbc, q)) bidx = nidx;
     }
-    // finished rows write their records (lane_finish)
+    // finished groups write their records (lane_finish)
     const uint64_t act = __ballot(active);
-    const bool done = has && ((act >> row0) & 0xFFFFull) == 0;
+    const bool done = has && ((act >> lead) & kGroup) == 0;
     if (!__ballot(done)) continue;
-    // every lane of the wave takes part in the shuffles
-    const uint32_t pair = bidx | ((uint32_t)__shfl_xor((int)bidx, 1) << 4);
-    uint32_t sum = extra, pbcs = 0;
-    const uint64_t sub1 = __ballot(sub == 1) >> row0, sub2 = __ballot(sub == 2) >> row0;
-    const int first1 = __ffsll((unsigned long long)(sub1 & 0xFFFFull)) - 1;
-    const int first2 = __ffsll((unsigned long long)(sub2 & 0xFFFFull)) - 1;
-    const bool leader = px == 0 || px == first1 || px == first2;
+    uint32_t sum = extra + t.best, pbcs = t.bpbc, out = bidx;
+    bool leader = m == 0;
+    if (G == 16) {
+      // every lane of the wave takes part in the shuffles
+      out = bidx | ((uint32_t)__shfl_xor((int)bidx, 1) << 4);
+      const uint64_t sub1 = __ballot(sub == 1) >> lead, sub2 = __ballot(sub == 2) >> lead;
+      const int first1 = __ffsll((unsigned long long)(sub1 & kGroup)) - 1;
+      const int first2 = __ffsll((unsigned long long)(sub2 & kGroup)) - 1;
+      leader = m == 0 || m == first1 || m == first2;
+      sum = extra;
+      pbcs = 0;
 #pragma unroll
-    for (int s = 0; s < 3; s++) {
-      const int from = s == 0 ? 0 : (s == 1 ? first1 : first2);
-      const uint32_t e = (uint32_t)__shfl((int)best, row0 + (from & 15));
-      const uint32_t pb = (uint32_t)__shfl((int)bpbc, row0 + (from & 15));
-      if (from >= 0) {
-        sum += e;
-        pbcs |= pb << (2 * s);
+      for (int s = 0; s < 3; s++) {
+        const int from = s == 0 ? 0 : (s == 1 ? first1 : first2);
+        const uint32_t e = (uint32_t)__shfl((int)t.best, lead + (from & 15));
+        const uint32_t pb = (uint32_t)__shfl((int)t.bpbc, lead + (from & 15));
+        if (from >= 0) {
+          sum += e;
+          pbcs |= pb << (2 * s);
+        }
       }
     }
     if (done) {
       CandRec *rc = &w.rec[id];
       if (leader) {
-        const int mode = info & 7;
         Fit f;
-        set_fit(f, mode, (info >> 3) & 3, (info >> 5) & 1);
+        set_fit(f, info & 7, (info >> 3) & 3, (info >> 5) & 1);
         const bool has_pb = f.pbit_type != PB_NONE;
-        uint32_t e1 = to_pixel_int(bp1, f.qmask, has_pb ? (int)((bpbc >> sh) & 1u) : -1);
-        uint32_t e2 = to_pixel_int(bp2, f.qmask, has_pb ? (int)(bpbc & 1u) : -1);
+        uint32_t e1 = to_pixel_int(t.bp1, f.qmask, has_pb ? (int)((t.bpbc >> k.sh) & 1u) : -1);
+        uint32_t e2 = to_pixel_int(t.bp2, f.qmask, has_pb ? (int)(t.bpbc & 1u) : -1);
         if (ptmode) {
           e1 = (e1 & 0x00FFFFFFu) | (rc->px1[0] & 0xFF000000u);
           e2 = (e2 & 0x00FFFFFFu) | (rc->px2[0] & 0xFF000000u);
@@ -3527,27 +3386,162 @@ __global__ void __launch_bounds__(256) anneal_spread_kernel(BlockRange r, Bc7Par
         rc->px1[sub] = e1;
         rc->px2[sub] = e2;
       }
-      if (!(px & 1)) reinterpret_cast<uint8_t *>(&rc->cidx_lo)[px >> 1] = (uint8_t)pair;
-      if (px == 0) {
-        rc->meta = (rc->meta & ~0x3Fu) | (rc->meta & 0x3Fu & ~((1u << (2 * nsub)) - 1u)) | pbcs |
-                   kMetaAnnealed;
+      if (G == 4) reinterpret_cast<uint16_t *>(&rc->cidx_lo)[m] = (uint16_t)out;
+      else if (!(m & 1)) reinterpret_cast<uint8_t *>(&rc->cidx_lo)[m >> 1] = (uint8_t)out;
+      if (m == 0) {
+        rc->meta = (rc->meta & ~((1u << (2 * nsub)) - 1u)) | pbcs | kMetaAnnealed;
         rc->err = sum;
       }
       has = false;
       active = false;
     }
   }
-  if constexpr (COUNT) {
-    unsigned long long a = n_ref, b = n_gpu;
-    for (int off = 32; off >= 1; off >>= 1) {
-      a += __shfl_xor(a, off);
-      b += __shfl_xor(b, off);
+}
+
+__device__ __forceinline__ void add_counts(const Bc7Params &prm, unsigned long long a,
+                                           unsigned long long b) {
+  for (int off = 32; off >= 1; off >>= 1) {
+    a += __shfl_xor(a, off);
+    b += __shfl_xor(b, off);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    atomicAdd(&prm.work_counts[0], a);
+    atomicAdd(&prm.work_counts[1], b);
+  }
+}
+
+// TAIL: the candidates the one-lane form handed over (counters[22] of them);
+// otherwise the whole annealing list.
+template <bool TAIL, bool COUNT>
+__global__ void __launch_bounds__(256) anneal_spread_kernel(BlockRange r, Bc7Params prm, Work w,
+                                                            TailState *tail) {
+  __shared__ __align__(4) uint8_t s_quant[kStepQuantBytes];
+  step_quant_load(s_quant);
+  __syncthreads();
+  const uint32_t total = *(volatile uint32_t *)&w.counters[TAIL ? 22 : (w.alist ? 18 : 16)];
+  unsigned long long n_ref = 0, n_gpu = 0;
+  spread_run<16, TAIL ? kFromTail : kFromList, COUNT>(r, prm, w, tail, s_quant, 0, total,
+                                                      &w.counters[TAIL ? 23 : 17], n_ref, n_gpu);
+  if constexpr (COUNT) add_counts(prm, n_ref, n_gpu);
+}
+
+// unroll: annealing steps between looks at the idle lanes.
+// tail_lanes: once the list is used up, a wave with at most this many
+// running candidates hands them to anneal_spread_kernel (through `tail`),
+// whose steps are several times shorter; otherwise the longest anneals, which
+// set the launch's length, would run on in nearly empty waves.
+// NU: the nonuniform metric (float errors, whose sums have an order: the
+// lanes finish their own candidates).
+// COUNT: also count the work into prm.work_counts: [0] the QuantizedError
+// point evaluations the reference's annealing makes (each step of a subset
+// scores that subset's points, Compressor.cpp:583-624), [1] the pixel scores
+// this kernel makes (16 per step of a candidate, whichever subsets are
+// still annealing).
+template <int WAVES, bool NU = false, bool COUNT = false>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES)))
+anneal_kernel(BlockRange r, Bc7Params prm, Work w, uint32_t unroll, uint32_t tail_lanes,
+              uint32_t rot_groups, TailState *tail) {
+  const int lane = threadIdx.x & 63;
+  unsigned long long n_ref = 0, n_gpu = 0;  // COUNT
+  const uint64_t lt = (1ull << lane) - 1ull;
+  uint32_t total = *(volatile uint32_t *)&w.counters[w.alist ? 18 : 16];
+  // odd row stride: conflict-free
+  __shared__ uint32_t s_px[256 * kRowWords];
+  __shared__ __align__(4) uint8_t s_quant[kStepQuantBytes];
+  step_quant_load(s_quant);
+  __syncthreads();
+  // Learned search: the list is in state order, and the set-up kernels
+  // append the rotation modes' states last (counters[19] holds the first of
+  // them): the list's rotation states are its suffix.  Their chains are the
+  // longest by far (to 1410 steps, against a mean of 66 in mode 1), so the
+  // first rot_groups workgroups start on them at once, four lanes each, while
+  // the others run the rest.  (The reference search's list is mostly rotation
+  // states: one lane each is the cheapest form, and the list starts with
+  // them.)
+  if (!NU && rot_groups && w.alist) {
+    const uint32_t first_rot = *(volatile uint32_t *)&w.counters[19];
+    uint32_t lo = 0, hi = total;  // first list entry >= first_rot
+    while (lo < hi) {
+      const uint32_t mid = (lo + hi) >> 1;
+      if (w.alist[mid] < first_rot) lo = mid + 1;
+      else hi = mid;
     }
-    if (lane == 0) {
-      atomicAdd(&prm.work_counts[0], a);
-      atomicAdd(&prm.work_counts[1], b);
+    if (blockIdx.x < rot_groups)
+      spread_run<4, kFromListHand, COUNT>(r, prm, w, tail, s_quant, lo, total, &w.counters[21],
+                                          n_ref, n_gpu);
+    total = lo;
+  }
+  Lane L = {};  // lanes without a candidate step along on zeros
+  L.nsub = 1;
+  L.px = s_px + threadIdx.x * kRowWords;
+  uint32_t wbase = 0, wend = 0;  // wave-local window of the list
+  bool exhausted = false;
+  for (;;) {
+    const uint64_t running = __ballot(L.active != 0);
+    const int nrun = __popcll(running);
+    if (!exhausted ? 64 - nrun >= kRefillLanes : nrun == 0) {
+      if (L.has && L.active == 0) {
+        lane_finish<NU>(L, w);
+        L.has = false;
+      }
+      // refill idle lanes from the window, fetching a new window when needed
+      for (;;) {
+        const uint64_t need = __ballot(!L.has);
+        if (!need || exhausted) break;
+        if (wbase >= wend) {
+          uint32_t b0 = 0;
+          if (lane == 0) b0 = atomicAdd(&w.counters[17], 64u);
+          b0 = __shfl(b0, 0);
+          if (b0 >= total) {
+            exhausted = true;
+            break;
+          }
+          wbase = b0;
+          wend = min(b0 + 64u, total);
+        }
+        const uint32_t avail = wend - wbase;
+        const uint32_t rank = (uint32_t)__popcll(need & lt);
+        if (!L.has && rank < avail) {
+          // the list runs from its end: the set-up kernels append modes 0, 2,
+          // 3, 7, 6, 1, 4, 5.  The rotation modes' candidates anneal the
+          // longest, so the list starts with them; then come the numerous
+          // mode-1 candidates, and the short mode-7 chains are among the last
+          // loaded, which keeps the tail of the launch short
+          const uint32_t item = total - 1u - (wbase + rank);
+          lane_load<NU>(L, r, prm, w.astate[w.alist ? w.alist[item] : item]);
+        }
+        wbase += min(avail, (uint32_t)__popcll(need));
+      }
+      if (!__ballot(L.has)) break;
+    }
+    if (!NU && exhausted && __popcll(__ballot(L.active != 0)) <= (int)tail_lanes) {
+      if (L.has && L.active == 0) {
+        lane_finish(L, w);
+        L.has = false;
+      }
+      const uint64_t left = __ballot(L.has);
+      uint32_t base = 0;
+      if (lane == 0) base = atomicAdd(&w.counters[22], (uint32_t)__popcll(left));
+      base = __shfl(base, 0);
+      if (L.has) lane_hand_over(L, tail[base + (uint32_t)__popcll(left & lt)]);
+      break;
+    }
+    for (uint32_t u = 0; u < unroll; u++) {
+      if constexpr (COUNT) {
+        const int n1 = __popc(L.m12 & 0xFFFFu), n2 = __popc(L.m12 >> 16);
+        if (L.active) {
+          n_ref += ((L.active & 1u) ? 16 - n1 - n2 : 0) + ((L.active & 2u) ? n1 : 0) +
+                   ((L.active & 4u) ? n2 : 0);
+          n_gpu += 16u;
+        }
+      }
+      // keeps the texels' LDS reads inside the step: hoisted out of this loop
+      // they would take 32 registers and spill
+      asm volatile("" ::: "memory");
+      lane_step<NU>(L, s_quant, (int)prm.quality);
     }
   }
+  if constexpr (COUNT) add_counts(prm, n_ref, n_gpu);
 }
 
 // ---------------------------------------------------------------------------
@@ -4142,37 +4136,64 @@ hipError_t bc7_upload_tables(int device) {
   return hipSuccess;
 }
 
-// Blocks up to which a call's annealing runs one lane per pixel.
-constexpr uint32_t kSpreadBlocks = 1u << 14, kSpreadBlocksLearned = 1u << 17;
+// Blocks up to which a call's annealing runs one lane per pixel from the
+// start.  Its lists (about 7 states a block in the reference search, 1 in the
+// learned one) then leave the one-lane form too few waves, and the longest
+// chain sets the time: 508x380 (12065 blocks) anneals in 2.0 ms against 2.9,
+// 1000x1024 (64000) in 7.9 against 4.6; learned 1024x1024 in 1.15 against
+// 1.18, 2048x2048 in 3.0 against 1.5.
+constexpr uint32_t kSpreadBlocks = 1u << 14, kSpreadBlocksLearned = 1u << 16;
+// Running candidates at which a wave of the one-lane form hands over
+// (learned 4096x4096: 4..12 3.3 ms, 16 3.5, 24 3.6, never 3.8; reference
+// search 2048x2048: 9.5 to 9.7 at 4..24).
+constexpr uint32_t kTailLanes = 12;
+// One workgroup in kRotShare starts on the learned list's rotation states
+// (learned 4096x4096: 4 3.9 ms, 8 3.4, 12 3.3, 16 4.1).
+constexpr uint32_t kRotShare = 10;
+// Workgroups per CU of the one-lane-per-pixel form: five fit, but more waves
+// on a SIMD slow the longest chain (508x380: 6 2.12 ms, 4 2.04, 3 2.05).
+constexpr uint32_t kSpreadWgPerCu = 4;
 
-void launch_anneal(uint32_t grid, int cus, const BlockRange &r, const Bc7Params &p,
-                   const bc7::Work &w, hipStream_t stream) {
-  if (!w.nu_total && r.num_blocks <= (w.alist ? kSpreadBlocksLearned : kSpreadBlocks)) {
-    // workgroups of 16 rows, no more than the candidates could use
-    uint32_t groups = (r.num_blocks * (uint32_t)bc7::kMaxCands + 15) / 16;
-    if (groups > (uint32_t)cus * 6u) groups = (uint32_t)cus * 6u;
-    if (p.work_counts)
-      hipLaunchKernelGGL(bc7::anneal_spread_kernel<true>, dim3(groups), dim3(256), 0, stream, r,
-                         p, w);
-    else
-      hipLaunchKernelGGL(bc7::anneal_spread_kernel<false>, dim3(groups), dim3(256), 0, stream, r,
-                         p, w);
+// waves: persistent waves of the one-lane form.  tail: memory for tail_cap
+// candidates handed over.
+void launch_anneal(uint32_t waves, int cus, const BlockRange &r, const Bc7Params &p,
+                   const bc7::Work &w, bc7::TailState *tail, size_t tail_cap,
+                   hipStream_t stream) {
+  // workgroups of 16 rows, no more than the candidates could use
+  uint64_t spread = ((uint64_t)r.num_blocks * bc7::kMaxCands + 15) / 16;
+  if (spread > (uint64_t)cus * kSpreadWgPerCu) spread = (uint64_t)cus * kSpreadWgPerCu;
+  const dim3 sgrid((uint32_t)spread), grid((waves + 3) / 4), wg(256);
+  const uint32_t unroll = w.alist ? 4u : (p.anneal_unroll ? p.anneal_unroll : 1u);
+  if (w.nu_total) {  // nonuniform metric (the full search or given selections)
+    hipLaunchKernelGGL((bc7::anneal_kernel<1, true>), grid, wg, 0, stream, r, p, w, unroll, 0u,
+                       0u, (bc7::TailState *)nullptr);
     return;
   }
-  if (p.work_counts && !w.nu_total)  // the counting instance (both searches)
-    hipLaunchKernelGGL((bc7::anneal_kernel<4, 3, false, true>), dim3(grid), dim3(64), 0, stream,
-                       r, p, w);
-  else if (w.nu_total)  // nonuniform metric (the full search or given selections)
-    hipLaunchKernelGGL((bc7::anneal_kernel<4, 1, true>), dim3(grid), dim3(64), 0, stream, r, p,
-                       w);
-  else if (w.alist)  // learned search: four steps between refills
-    hipLaunchKernelGGL((bc7::anneal_kernel<4, 3>), dim3(grid), dim3(64), 0, stream, r, p, w);
-  else if (p.anneal_unroll >= 4)
-    hipLaunchKernelGGL((bc7::anneal_kernel<4, 3>), dim3(grid), dim3(64), 0, stream, r, p, w);
-  else if (p.anneal_unroll == 2)
-    hipLaunchKernelGGL((bc7::anneal_kernel<2, 3>), dim3(grid), dim3(64), 0, stream, r, p, w);
-  else
-    hipLaunchKernelGGL((bc7::anneal_kernel<1, 3>), dim3(grid), dim3(64), 0, stream, r, p, w);
+  if (r.num_blocks <= (w.alist ? kSpreadBlocksLearned : kSpreadBlocks)) {
+    if (p.work_counts)
+      hipLaunchKernelGGL((bc7::anneal_spread_kernel<false, true>), sgrid, wg, 0, stream, r, p, w,
+                         (bc7::TailState *)nullptr);
+    else
+      hipLaunchKernelGGL((bc7::anneal_spread_kernel<false, false>), sgrid, wg, 0, stream, r, p, w,
+                         (bc7::TailState *)nullptr);
+    return;
+  }
+  const size_t per_wave = tail_cap / ((size_t)grid.x * 4);
+  // each wave hands over at most kHandGroups rotation states and `lanes` others
+  const uint32_t room = per_wave > bc7::kHandGroups ? (uint32_t)per_wave - bc7::kHandGroups : 0u;
+  const uint32_t lanes = room < kTailLanes ? room : kTailLanes;
+  const uint32_t rots = w.alist && room ? (grid.x + kRotShare - 1) / kRotShare : 0u;
+  if (p.work_counts) {  // the counting instances (both searches)
+    hipLaunchKernelGGL((bc7::anneal_kernel<3, false, true>), grid, wg, 0, stream, r, p, w, unroll,
+                       lanes, rots, tail);
+    hipLaunchKernelGGL((bc7::anneal_spread_kernel<true, true>), sgrid, wg, 0, stream, r, p, w,
+                       tail);
+  } else {
+    hipLaunchKernelGGL((bc7::anneal_kernel<3>), grid, wg, 0, stream, r, p, w, unroll, lanes,
+                       rots, tail);
+    hipLaunchKernelGGL((bc7::anneal_spread_kernel<true, false>), sgrid, wg, 0, stream, r, p, w,
+                       tail);
+  }
 }
 
 hipError_t fill_u32(uint32_t *p, uint32_t n, uint32_t v, hipStream_t stream) {
@@ -4285,6 +4306,11 @@ hipError_t bc7_encode(const BlockRange &r, const Bc7Params &p, const Bc7Scratch 
   // candidate-error kernel: grid-stride, a few workgroups per CU
   const uint32_t err_grid = (uint32_t)g_num_cus[dev] * 8u;
   const bool guard = p.quality > 0 && p.q0_guard;
+  // the type queues are dead once the set-up (and the learned search's first
+  // error pass) is done: the annealing hands its tail over through them
+  bc7::TailState *tail = reinterpret_cast<bc7::TailState *>(w.queue);
+  const size_t tail_cap =
+      (size_t)w.qcap * bc7::kNumTypes * sizeof(uint32_t) / sizeof(bc7::TailState);
   int t = timing_begin(stream);
   hipLaunchKernelGGL(bc7::reset_kernel, dim3(1), dim3(64), 0, stream, w.counters, 64);
   hipLaunchKernelGGL(bc7::solid_scan_kernel, dim3(nchunks), dim3(256), 0, stream, r, s);
@@ -4380,7 +4406,7 @@ hipError_t bc7_encode(const BlockRange &r, const Bc7Params &p, const Bc7Scratch 
                          (const uint32_t *)w.aid, (const uint32_t *)w.counters,
                          (const uint32_t *)w.sel, cerr, q0err, (const uint32_t *)chunk_count,
                          alist);
-      launch_anneal(persistent, g_num_cus[dev], r, p, wa, stream);
+      launch_anneal(persistent, g_num_cus[dev], r, p, wa, tail, tail_cap, stream);
       timing_end(t, kTagBc7Anneal, stream);
     }
     t = timing_begin(stream);
@@ -4402,7 +4428,7 @@ hipError_t bc7_encode(const BlockRange &r, const Bc7Params &p, const Bc7Scratch 
   }
   if (p.quality > 0) {
     t = timing_begin(stream);
-    launch_anneal(persistent, g_num_cus[dev], r, p, w, stream);
+    launch_anneal(persistent, g_num_cus[dev], r, p, w, tail, tail_cap, stream);
     timing_end(t, kTagBc7Anneal, stream);
   }
   t = timing_begin(stream);
