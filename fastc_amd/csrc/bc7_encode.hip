@@ -546,6 +546,22 @@ __device__ __forceinline__ void unpack4f(uint32_t p, float v[4]) {
 // past the last unique point (:364-371).
 __device__ __forceinline__ void principal_axis(const uint32_t px[16], uint32_t smask, int ptmode, int n,
                                const float avg[4], float axis[4]) {
+  // the repeated points: equal to an earlier one of the subset.  Unrolled on
+  // register copies: the 120 comparisons take one instruction each (rolled,
+  // with two LDS reads apiece, they were a fifth of a fit's latency)
+  uint32_t dup = 0;
+  {
+    uint32_t pt[16];
+#pragma unroll
+    for (int i = 0; i < 16; i++) pt[i] = point_of(px[i], ptmode);
+#pragma unroll
+    for (int i = 1; i < 16; i++) {
+      bool seen = false;
+#pragma unroll
+      for (int j = 0; j < i; j++) seen = seen | (((smask >> j) & 1) && pt[j] == pt[i]);
+      dup |= seen ? 1u << i : 0u;
+    }
+  }
   // unique points in first-occurrence order; test u2.. as they appear
   int nu = 0;
   float u0[4], dir[4];
@@ -553,13 +569,8 @@ __device__ __forceinline__ void principal_axis(const uint32_t px[16], uint32_t s
   uint32_t u0p = 0;
 #pragma unroll 1
   for (int i = 0; i < 16; i++) {
-    if (!((smask >> i) & 1)) continue;
+    if (!(((smask & ~dup) >> i) & 1)) continue;
     const uint32_t pi = point_of(px[i], ptmode);
-    bool seen = false;
-#pragma unroll 1
-    for (int j = 0; j < i; j++)
-      if (((smask >> j) & 1) && point_of(px[j], ptmode) == pi) seen = true;
-    if (seen) continue;
     if (nu == 0) {
       u0p = pi;
       unpack4f(pi, u0);
@@ -741,15 +752,22 @@ __device__ __forceinline__ int nearest_centroid(const float c[NB][4], const floa
   return minb;
 }
 
+__device__ __forceinline__ void km_add(uint32_t *p, uint32_t v) {
+  __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+}
+
 // NU: the nonuniform metric, mu its unrotated weights (single colour), mr
 // the weights of this candidate's rotation (QuantizedError).
-// km: this lane's k-means accumulators in LDS (word (j * 5 + k) * 64 of
-// bucket j, k = 4 the count).
+// km: this lane's k-means accumulators in LDS, words (j * 3 + k) * 64 of
+// bucket j: the sums of channels 0 and 2 (<< 16), of 1 and 3, the count.  A sum
+// is at most 16 * 255, so 16 bits hold it, and integer sums are the reference's
+// float sums exactly; they are added in place without being read, where five
+// float sums a point took a read and a write each.
 template <int NB, bool NU = false>
 __device__ __forceinline__ void kmeans_setup(const Fit &f, uint32_t q, const uint32_t *sctab,
                              const uint32_t px[16], uint32_t smask, int ptmode, int n,
                              const float avg[4], SubStart &out,
-                             const Weights *mu, const Weights *mr, float *km) {
+                             const Weights *mu, const Weights *mr, uint32_t *km) {
   float axis[4];
   principal_axis(px, smask, ptmode, n, avg, axis);
   float mindp = FLT_MAX, maxdp = -FLT_MAX;
@@ -785,40 +803,41 @@ __device__ __forceinline__ void kmeans_setup(const Fit &f, uint32_t q, const uin
   bool fixed = false;
   int guard = 0;
   while (!fixed && guard++ < 4096) {
-    // every point into its nearest centroid's LDS sums, in point order, so
-    // each bucket adds its points in the order the reference's per-bucket
-    // loop does (Compressor.cpp:997-1009)
+    // every point into its nearest centroid's sums (Compressor.cpp:997-1009)
 #pragma unroll
-    for (int j = 0; j < NB * 5; j++) km[j * 64] = 0.0f;
+    for (int j = 0; j < NB * 3; j++) km[j * 64] = 0u;
 #pragma unroll 1
     for (int i = 0; i < 16; i++) {
       if (!((smask >> i) & 1)) continue;
+      const uint32_t pt = point_of(px[i], ptmode);
       float v[4];
-      unpack4f(point_of(px[i], ptmode), v);
-      float *b = km + nearest_centroid<NB>(c, v) * 5 * 64;
-#pragma unroll
-      for (int k = 0; k < 4; k++) b[k * 64] += v[k];
-      b[4 * 64] += 1.0f;
+      unpack4f(pt, v);
+      uint32_t *b = km + nearest_centroid<NB>(c, v) * 3 * 64;
+      km_add(b, pt & 0x00FF00FFu);
+      km_add(b + 64, (pt >> 8) & 0x00FF00FFu);
+      km_add(b + 2 * 64, 1u);
     }
     fixed = true;
 #pragma unroll
     for (int j = 0; j < NB; j++) {
-      const float cn = km[(j * 5 + 4) * 64];
+      const uint32_t k02 = km[(j * 3) * 64], k13 = km[(j * 3 + 1) * 64];
+      const uint32_t cn = km[(j * 3 + 2) * 64];
       float s[4];
       // sum / cn in float, correctly rounded, as a double product: the sum
       // is an integer below 2^13 and cn one of 1..16, so sum / cn is either
       // a float or, in lowest terms p / q with q odd, at least 2^-29
       // (relative) from every float rounding boundary, far beyond the
-      // product's 2^-52
-      const double inv = kInvCount[(int)cn];
-#pragma unroll
-      for (int k = 0; k < 4; k++)
-        s[k] = cn != 0.0f ? (float)((double)km[(j * 5 + k) * 64] * inv) : 0.0f;
+      // product's 2^-52 (kInvCount[0] is 0: an empty bucket's mean is 0)
+      const double inv = kInvCount[cn];
+      s[0] = (float)((double)(k02 & 0xFFFFu) * inv);
+      s[1] = (float)((double)(k13 & 0xFFFFu) * inv);
+      s[2] = (float)((double)(k02 >> 16) * inv);
+      s[3] = (float)((double)(k13 >> 16) * inv);
       if (s[0] != c[j][0] || s[1] != c[j][1] || s[2] != c[j][2] || s[3] != c[j][3])
         fixed = false;
 #pragma unroll
       for (int k = 0; k < 4; k++) c[j][k] = s[k];
-      cnt[j] = (uint32_t)cn;
+      cnt[j] = cn;
     }
   }
   int nfilled = 0, last = 0;
@@ -930,7 +949,7 @@ template <bool NU = false>
 __device__ __forceinline__ void subset_setup(const Fit &f, uint32_t q, const uint32_t *sctab,
                              const uint32_t px[16], uint32_t smask, int ptmode, int n,
                              const float avg[4], bool all_same, SubStart &out,
-                             const Weights *mu, const Weights *mr, float *km) {
+                             const Weights *mu, const Weights *mr, uint32_t *km) {
   if (all_same) {
     const int first = __ffs(smask) - 1;
     uint32_t pt = 0;
@@ -1251,17 +1270,71 @@ struct AState {
 // annealed (annealing lowers a fit's error by a few percent at most).
 constexpr unsigned long long kAnnealMarginDiv = 50;
 
+struct Work {
+  uint32_t *sel;          // per block
+  uint16_t *cdesc;        // per block x 16 candidate descriptors
+  CandRec *rec;           // per block x 16
+  uint32_t *queue;        // per-type candidate queues, kMaxPerType entries per block each
+  // [0..7] queue sizes, [8..15] set-up fetch, [16] annealing states of the
+  // modes without rotation, [17] anneal fetch, [18] learned annealing list
+  // size, [20] fallback blocks, [21] anneal fetch of the rotation states, [22]
+  // candidates handed over, [23] their fetch, [24] and [25] annealing states of
+  // modes 4 and 5
+  uint32_t *counters;
+  // the annealing states: those of the modes without rotation from the front,
+  // the rotation modes' at the back (state_map)
+  AState *astate;
+  uint32_t qcap;          // entries per type queue
+  uint32_t astate_cap;
+  // learned search: the annealing states to run (slots of astate, in
+  // order), counters[18] of them; null in the reference search
+  const uint32_t *alist;
+  // learned search: astate[i].id for every state (read when the list is
+  // built, without touching the 64-byte states); null in the reference search
+  uint32_t *aid;
+  // nonuniform metric: each candidate's total error, the double the
+  // reference compares (per block x kMaxCands); null under the uniform metric
+  double *nu_total;
+};
+
+// Annealing state i of the counters[16], [24] and [25]: its slot of astate.
+// The rotation modes come last, mode 5 after mode 4: the longer a mode's
+// chains, the earlier annealing starts on them (it runs from the end).  The
+// three regions cannot meet: mode 4's lies below room for every candidate of
+// mode 5, and a job's candidates all fit.
+// (Read once per kernel: the counters share a cache line with the annealing's
+// fetch counters, and loads of it between their atomics took the 508x380
+// annealing from 2.0 to 3.2 ms.)
+struct StateMap {
+  uint32_t front, c4, c5, base4, base5;
+  __device__ __forceinline__ uint32_t count() const { return front + c4 + c5; }
+  __device__ __forceinline__ uint32_t slot(uint32_t i) const {
+    if (i < front) return i;
+    i -= front;
+    return i < c4 ? base4 + i : base5 + (i - c4);
+  }
+};
+__device__ __forceinline__ StateMap state_map(const Work &w) {
+  const volatile uint32_t *c = w.counters;
+  StateMap m;
+  m.front = c[16];
+  m.c4 = c[24];
+  m.c5 = c[25];
+  m.base4 = w.astate_cap - c[7] - m.c4;  // below room for mode 5's whole queue
+  m.base5 = w.astate_cap - m.c5;
+  return m;
+}
+
 // Learned search: the list of annealing states that pass the margin, in
-// astate order (the set-up kernels append by mode, so annealing waves stay
-// uniform and the list's end holds the rotation modes).  An ordered
+// the order of state_map (for large jobs the set-up kernels append by mode, so
+// annealing waves stay uniform; the list's end holds the rotation modes).  An ordered
 // compaction over chunks of 4096 states: per-chunk counts, their exclusive
 // scan, then each chunk writes its passing states from its offset.
 constexpr uint32_t kListChunk = 4096;
 
 // Flags of the states cb + 256 k + t (k = 0..15) of thread t: bit k set when
 // the state passes the margin.  Adjacent lanes read adjacent states.
-__device__ __forceinline__ uint32_t list_flags(const uint32_t *aid, uint32_t total,
-                                               const uint32_t *sel,
+__device__ __forceinline__ uint32_t list_flags(const Work &w, const StateMap &sm,
                                                const unsigned long long *cerr,
                                                const unsigned long long *q0best, uint32_t cb,
                                                int t) {
@@ -1269,12 +1342,12 @@ __device__ __forceinline__ uint32_t list_flags(const uint32_t *aid, uint32_t tot
 #pragma unroll
   for (int k = 0; k < 16; k++) {
     const uint32_t i = cb + 256u * (uint32_t)k + (uint32_t)t;
-    if (i < total) {
-      const uint32_t id = aid[i];
+    if (i < sm.count()) {
+      const uint32_t id = w.aid[sm.slot(i)];
       const uint32_t rel = id_block(id);
       const unsigned long long best = q0best[rel];
       // a full-search block anneals every candidate
-      if (sel_full(sel[rel]) || cerr[id] <= best + best / kAnnealMarginDiv) flags |= 1u << k;
+      if (sel_full(w.sel[rel]) || cerr[id] <= best + best / kAnnealMarginDiv) flags |= 1u << k;
     }
   }
   return flags;
@@ -1302,16 +1375,14 @@ __device__ __forceinline__ uint32_t wg_exclusive_scan(uint32_t v, uint32_t *excl
   return all;
 }
 
-__global__ void __launch_bounds__(256) list_count_kernel(const uint32_t *aid, const uint32_t *counters,
-                                                         const uint32_t *sel,
-                                                         const unsigned long long *cerr,
+__global__ void __launch_bounds__(256) list_count_kernel(Work w, const unsigned long long *cerr,
                                                          const unsigned long long *q0best,
                                                          uint32_t *chunk_count) {
   __shared__ uint32_t s_wave[4];
-  const uint32_t total = counters[16];
+  const StateMap sm = state_map(w);
   const uint32_t cb = blockIdx.x * kListChunk;
-  if (cb >= total) return;  // whole workgroup
-  const uint32_t flags = list_flags(aid, total, sel, cerr, q0best, cb, threadIdx.x);
+  if (cb >= sm.count()) return;  // whole workgroup
+  const uint32_t flags = list_flags(w, sm, cerr, q0best, cb, threadIdx.x);
   uint32_t excl;
   const uint32_t all = wg_exclusive_scan((uint32_t)__popc(flags), &excl, s_wave);
   if (threadIdx.x == 0) chunk_count[blockIdx.x] = all;
@@ -1319,9 +1390,9 @@ __global__ void __launch_bounds__(256) list_count_kernel(const uint32_t *aid, co
 
 // One workgroup: exclusive scan of the chunk counts (at most 64 per thread),
 // the list length into counters[18].
-__global__ void __launch_bounds__(256) list_scan_kernel(uint32_t *counters, uint32_t *chunk_count) {
+__global__ void __launch_bounds__(256) list_scan_kernel(Work w, uint32_t *chunk_count) {
   __shared__ uint32_t s_wave[4];
-  const uint32_t nchunks = (counters[16] + kListChunk - 1) / kListChunk;
+  const uint32_t nchunks = (state_map(w).count() + kListChunk - 1) / kListChunk;
   const uint32_t per = (nchunks + 255) / 256;
   const uint32_t c0 = threadIdx.x * per;
   uint32_t sum = 0;
@@ -1333,19 +1404,17 @@ __global__ void __launch_bounds__(256) list_scan_kernel(uint32_t *counters, uint
     chunk_count[c] = excl;
     excl += v;
   }
-  if (threadIdx.x == 0) counters[18] = all;
+  if (threadIdx.x == 0) w.counters[18] = all;
 }
 
-__global__ void __launch_bounds__(256) list_write_kernel(const uint32_t *aid, const uint32_t *counters,
-                                                         const uint32_t *sel,
-                                                         const unsigned long long *cerr,
+__global__ void __launch_bounds__(256) list_write_kernel(Work w, const unsigned long long *cerr,
                                                          const unsigned long long *q0best,
                                                          const uint32_t *chunk_offset,
                                                          uint32_t *alist) {
-  const uint32_t total = counters[16];
+  const StateMap sm = state_map(w);
   const uint32_t cb = blockIdx.x * kListChunk;
-  if (cb >= total) return;  // whole workgroup
-  const uint32_t flags = list_flags(aid, total, sel, cerr, q0best, cb, threadIdx.x);
+  if (cb >= sm.count()) return;  // whole workgroup
+  const uint32_t flags = list_flags(w, sm, cerr, q0best, cb, threadIdx.x);
   // round k places the passing states cb + 256 k .. cb + 256 k + 255 in
   // order: rank within the wave by ballot, then the waves before it
   __shared__ uint32_t s_round[2][4];
@@ -1365,31 +1434,10 @@ __global__ void __launch_bounds__(256) list_write_kernel(const uint32_t *aid, co
     }
     if (f)
       alist[pos + before + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] =
-          cb + 256u * (uint32_t)k + (uint32_t)threadIdx.x;
+          sm.slot(cb + 256u * (uint32_t)k + (uint32_t)threadIdx.x);
     pos += all;
   }
 }
-
-struct Work {
-  uint32_t *sel;          // per block
-  uint16_t *cdesc;        // per block x 16 candidate descriptors
-  CandRec *rec;           // per block x 16
-  uint32_t *queue;        // per-type candidate queues, kMaxPerType entries per block each
-  uint32_t *counters;     // [0..7] queue sizes, [8..15] set-up fetch, [16] anneal size,
-                          // [17] anneal fetch, [18] learned annealing list size
-  AState *astate;
-  uint32_t qcap;          // entries per type queue
-  uint32_t astate_cap;
-  // learned search: the annealing states to run (indices into astate, in
-  // astate order), counters[18] of them; null in the reference search
-  const uint32_t *alist;
-  // learned search: astate[i].id for every state (read when the list is
-  // built, without touching the 64-byte states); null in the reference search
-  uint32_t *aid;
-  // nonuniform metric: each candidate's total error, the double the
-  // reference compares (per block x kMaxCands); null under the uniform metric
-  double *nu_total;
-};
 
 __device__ __forceinline__ void load_block(const BlockRange &r, uint32_t rel, uint32_t px[16]) {
   const uint32_t b = r.first_block + rel;
@@ -2470,6 +2518,39 @@ __global__ void __launch_bounds__(256, 2) rank_select_kernel(BlockRange r, Bc7Pa
 // ---------------------------------------------------------------------------
 // Kernel 2: candidate set-up, persistent over the type queues in order.
 // ---------------------------------------------------------------------------
+// One subset of a mode without rotation: its average, then its fit.  Returns
+// its pixel count.
+template <bool NU>
+__device__ __forceinline__ int fit_subset(const Fit &f, uint32_t quality, const uint32_t *sctab,
+                                          const uint32_t px[16], uint32_t smask, SubStart &ss,
+                                          const Weights *mu, uint32_t *km) {
+  const int n = __popc(smask);
+  uint32_t sum02 = 0, sum13 = 0;
+  bool same = true;
+  uint32_t firstp = 0;
+  bool have_first = false;
+#pragma unroll
+  for (int i = 0; i < 16; i++) {
+    if (!((smask >> i) & 1)) continue;
+    if (!have_first) {
+      firstp = px[i];
+      have_first = true;
+    }
+    same = same && px[i] == firstp;
+    sum02 += px[i] & 0x00FF00FFu;
+    sum13 += (px[i] >> 8) & 0x00FF00FFu;
+  }
+  // integer sums over n in 1..16: the double product is the correctly
+  // rounded quotient (as for the k-means means)
+  float avg[4];
+  avg[0] = (float)((double)(sum02 & 0xFFFFu) * kInvCount[n]);
+  avg[1] = (float)((double)(sum13 & 0xFFFFu) * kInvCount[n]);
+  avg[2] = (float)((double)(sum02 >> 16) * kInvCount[n]);
+  avg[3] = (float)((double)(sum13 >> 16) * kInvCount[n]);
+  subset_setup<NU>(f, quality, sctab, px, smask, 0, n, avg, same, ss, mu, mu, km);
+  return n;
+}
+
 // Quality-0 fit of one candidate: every subset's endpoints, indices and
 // error (CompressionMode::Compress, Compressor.cpp:1300-1371, without the
 // annealing), the record the pack kernel reads, and the annealing start
@@ -2487,7 +2568,7 @@ __device__ __forceinline__ uint32_t fit_candidate(const Cand &k, const uint32_t 
                                                   uint32_t quality, const uint32_t *sctab,
                                                   CandRec &rec, AState &st, uint32_t &total,
                                                   const Weights *mu, double *tot_nu,
-                                                  float *km) {
+                                                  uint32_t *km) {
   Fit f;
   const ModeAttr attr = MODE >= 0 ? kModeTab[MODE < 0 ? 0 : MODE] : kModes[k.mode];
   const int nsub = attr.subsets;
@@ -2548,29 +2629,11 @@ __device__ __forceinline__ uint32_t fit_candidate(const Cand &k, const uint32_t 
   } else {
 #pragma unroll 1
     for (int s = 0; s < nsub; s++) {
-      const uint32_t smask = subset_mask(k.shape, nsub, s);
-      const int n = __popc(smask);
-      float avg[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-      bool same = true;
-      uint32_t firstp = 0;
-      bool have_first = false;
-#pragma unroll
-      for (int i = 0; i < 16; i++) {
-        if (!((smask >> i) & 1)) continue;
-        if (!have_first) {
-          firstp = px[i];
-          have_first = true;
-        }
-        same = same && px[i] == firstp;
-#pragma unroll
-        for (int kk = 0; kk < 4; kk++) avg[kk] += (float)chan(px[i], kk);
-      }
-      // integer sums over n in 1..16: the double product is the correctly
-      // rounded quotient (as for the k-means means)
-#pragma unroll
-      for (int kk = 0; kk < 4; kk++) avg[kk] = (float)((double)avg[kk] * kInvCount[n]);
+      // keeps the texels' LDS reads inside the loop: hoisted, their channels
+      // take 80 registers
+      asm volatile("" ::: "memory");
       SubStart ss;
-      subset_setup<NU>(f, quality, sctab, px, smask, 0, n, avg, same, ss, mu, mu, km);
+      const int n = fit_subset<NU>(f, quality, sctab, px, subset_mask(k.shape, nsub, s), ss, mu, km);
       if constexpr (NU) {
         tnu += ss.sc ? (double)n * (double)__uint_as_float(ss.err)
                      : (double)__uint_as_float(ss.err);
@@ -2620,50 +2683,120 @@ constexpr int kSetupBuckets(int mode) {
   return mode == 6 ? 16 : ((mode == 0 || mode == 1 || mode == 4) ? 8 : 4);
 }
 
-template <int MODE, bool NU = false>
-__global__ void __launch_bounds__(64) setup_kernel(BlockRange r, Bc7Params prm, Work w,
-                                                   const uint32_t *sctab) {
-  const int lane = threadIdx.x;
-  __shared__ uint32_t s_px[64 * kPxStride];
-  // the k-means sums and counts, per bucket and channel a row of 64 lanes
-  __shared__ float s_km[kSetupBuckets(MODE) * 5 * 64];
-  {
-    constexpr int kTypeOf[8] = {0, 2, 1, 3, 6, 7, 5, 4};
-    const int t = kTypeOf[MODE];
-    const uint32_t count = *(volatile uint32_t *)&w.counters[t];
-    for (;;) {
-      uint32_t b0 = 0;
-      if (lane == 0) b0 = atomicAdd(&w.counters[8 + t], 64u);
-      b0 = __shfl(b0, 0);
-      if (b0 >= count) break;
-      const uint32_t item = b0 + lane;
-      if (item >= count) continue;
-      const uint32_t id = w.queue[(size_t)t * w.qcap + item];
-      const uint32_t rel = id_block(id);
-      const int c = (int)id_slot(id);
-      Cand k;
-      cand_from_desc(w.cdesc[(size_t)rel * kMaxCands + c], k);
-      // the lane's texels live in LDS: the fit reads them many times, and
-      // keeping them (and values derived from them) out of registers lets
-      // the loops below stay rolled
-      {
-        uint32_t v[16];
-        load_block(r, rel, v);
+// One wave takes batches of candidates of the mode's queue until it is used
+// up: one lane each, or with several subsets one adjacent lane per subset (64
+// candidates, or 32 or 21), whose fits run side by side.  (One lane for all
+// subsets took their fits' time one after another: 155 us for a batch of
+// mode 0.)  s_px: the lanes' texels; s_km: the k-means sums and counts, per
+// bucket a row of 64 lanes each.
+template <int MODE, bool NU>
+__device__ __forceinline__ void setup_run(const BlockRange &r, const Bc7Params &prm,
+                                          const Work &w, const uint32_t *sctab, uint32_t *s_px,
+                                          uint32_t *s_km) {
+  constexpr int kTypeOf[8] = {0, 2, 1, 3, 6, 7, 5, 4};
+  constexpr int t = kTypeOf[MODE], kSub = kModeTab[MODE].subsets, kBatch = 64 / kSub;
+  const int lane = threadIdx.x, sub = lane % kSub, lead = lane - sub;
+  const uint32_t count = *(volatile uint32_t *)&w.counters[t];
+  for (;;) {
+    uint32_t b0 = 0;
+    if (lane == 0) b0 = atomicAdd(&w.counters[8 + t], (uint32_t)kBatch);
+    b0 = __shfl(b0, 0);
+    if (b0 >= count) break;
+    const uint32_t item = b0 + (uint32_t)(lane / kSub);
+    const bool mine = lane < kBatch * kSub && item < count;
+    const uint32_t id = mine ? w.queue[(size_t)t * w.qcap + item] : 0u;
+    const uint32_t rel = id_block(id);
+    const int c = (int)id_slot(id);
+    Cand k;
+    cand_from_desc(mine ? w.cdesc[(size_t)rel * kMaxCands + c] : (uint16_t)MODE, k);
+    // the lane's texels live in LDS: the fit reads them many times, and
+    // keeping them (and values derived from them) out of registers lets
+    // the loops below stay rolled
+    uint32_t *px = s_px + lane * kPxStride;
+    if (mine) {
+      uint32_t v[16];
+      load_block(r, rel, v);
 #pragma unroll
-        for (int i = 0; i < 16; i++) s_px[lane * kPxStride + i] = v[i];
+      for (int i = 0; i < 16; i++) px[i] = v[i];
+    }
+    Weights mu;
+    if constexpr (NU) mu = params_weights(prm);
+    CandRec *out = &w.rec[(size_t)rel * kMaxCands + c];
+    if constexpr (kSub > 1) {
+      Fit f;
+      set_fit_attr(f, kModeTab[MODE], MODE, 0, 0);
+      SubStart ss = {};
+      int n = 0;
+      if (mine)
+        n = fit_subset<NU>(f, prm.quality, sctab, px, subset_mask(k.shape, kSub, sub), ss, &mu,
+                           s_km + lane);
+      const bool has_pb = f.pbit_type != PB_NONE;
+      const uint32_t e1 =
+          to_pixel_int(ss.p1, f.qmask, has_pb ? pbc_bit(f.pbit_type, ss.pbc, 0) : -1);
+      const uint32_t e2 =
+          to_pixel_int(ss.p2, f.qmask, has_pb ? pbc_bit(f.pbit_type, ss.pbc, 1) : -1);
+      // the candidate's record from its subsets' lanes (every lane of the
+      // wave takes part)
+      const uint32_t bits = (uint32_t)ss.pbc | ((ss.anneal ? 1u : 0u) << 2) |
+                            ((ss.sc ? 1u : 0u) << 3);
+      const int nerr = ss.sc ? n : 1;
+      const double terr = NU ? (double)nerr * (double)__uint_as_float(ss.err) : 0.0;
+      uint32_t total = 0, pbcs = 0, active = 0, scf = 0, lo = 0, hi = 0;
+      double tnu = 0.0;
+#pragma unroll
+      for (int s = 0; s < kSub; s++) {
+        const int from = (lead + s) & 63;
+        const uint32_t b = (uint32_t)__shfl((int)bits, from);
+        total += (uint32_t)__shfl((int)ss.err, from);
+        lo |= (uint32_t)__shfl((int)(uint32_t)ss.idx, from);
+        hi |= (uint32_t)__shfl((int)(uint32_t)(ss.idx >> 32), from);
+        pbcs |= (b & 3u) << (2 * s);
+        active |= ((b >> 2) & 1u) << s;
+        scf |= ((b >> 3) & 1u) << s;
+        if constexpr (NU) tnu += __shfl(terr, from);
       }
-      const uint32_t *px = s_px + lane * kPxStride;
+      uint32_t slot = 0;
+      if (mine && sub == 0 && active) slot = atomicAdd(&w.counters[16], 1u);
+      slot = (uint32_t)__shfl((int)slot, lead);
+      if (mine) {
+        out->px1[sub] = e1;
+        out->px2[sub] = e2;
+        if (sub == 0) {
+          if (kSub == 2) out->px1[2] = out->px2[2] = 0;
+          out->err = total;  // the quality-0 result; annealing overwrites active ones
+          out->cidx_lo = lo;
+          out->cidx_hi = hi;
+          out->aidx_lo = out->aidx_hi = 0;
+          out->meta = pbcs;
+          if constexpr (NU) w.nu_total[(size_t)rel * kMaxCands + c] = tnu;
+        }
+        if (active) {
+          AState &st = w.astate[slot];
+          st.p1[sub] = ss.p1;
+          st.p2[sub] = ss.p2;
+          st.err[sub] = ss.err;
+          if (sub == 0) {
+            st.id = id;
+            st.info = (uint32_t)MODE | ((uint32_t)kSub << 6) | ((uint32_t)k.shape << 8) |
+                      (active << 14) | ((uint32_t)k.entry << 17);
+            st.pbc = pbcs | (NU ? scf << 8 : 0u);
+            st.idx_lo = lo;
+            st.idx_hi = hi;
+            st.extra_err = 0;
+            st.pad = 0;
+            if (w.aid) w.aid[slot] = id;
+          }
+        }
+      }
+    } else if (mine) {
       CandRec rec;
-      AState st;
+      AState st = {};
       uint32_t total = 0;
       double tnu = 0.0;
-      Weights mu;
-      if constexpr (NU) mu = params_weights(prm);
-      const uint32_t active =
-          fit_candidate<MODE, NU>(k, px, prm.quality, sctab, rec, st, total, &mu, &tnu,
-                                  s_km + lane);
+      const uint32_t active = fit_candidate<MODE, NU>(k, px, prm.quality, sctab, rec, st, total,
+                                                      &mu, &tnu, s_km + lane);
       st.id = id;
-      w.rec[(size_t)rel * kMaxCands + c] = rec;
+      *out = rec;
       if constexpr (NU) w.nu_total[(size_t)rel * kMaxCands + c] = tnu;
       // mode 6, shape entry 0 followed by entry 1 (opaque blocks with two
       // shapes): the second slot gets the same fit and its own annealing state
@@ -2673,14 +2806,18 @@ __global__ void __launch_bounds__(64) setup_kernel(BlockRange r, Bc7Params prm, 
         twin = (d1 & 7) == 6 && ((d1 >> 12) & 7) == 1;
       }
       if (twin) {
-        w.rec[(size_t)rel * kMaxCands + c + 1] = rec;
+        out[1] = rec;
         if constexpr (NU) w.nu_total[(size_t)rel * kMaxCands + c + 1] = tnu;
       }
       if (active) {
         st.info = (uint32_t)k.mode | ((uint32_t)k.rot << 3) | ((uint32_t)k.im << 5) |
                   ((uint32_t)k.nsub << 6) | ((uint32_t)k.shape << 8) | (active << 14) |
                   ((uint32_t)k.entry << 17);
-        const uint32_t slot = atomicAdd(&w.counters[16], twin ? 2u : 1u);
+        uint32_t slot;
+        if (MODE == 5) slot = w.astate_cap - 1u - atomicAdd(&w.counters[25], 1u);
+        else if (MODE == 4)
+          slot = w.astate_cap - 1u - w.counters[kTypeOf[5]] - atomicAdd(&w.counters[24], 1u);
+        else slot = atomicAdd(&w.counters[16], twin ? 2u : 1u);
         w.astate[slot] = st;
         if (w.aid) w.aid[slot] = id;
         if (twin) {
@@ -2690,6 +2827,43 @@ __global__ void __launch_bounds__(64) setup_kernel(BlockRange r, Bc7Params prm, 
           if (w.aid) w.aid[slot + 1] = id + 1;
         }
       }
+    }
+  }
+}
+
+// Three waves per SIMD (168 registers) for every mode but 6, whose 16
+// centroids take 64 registers: mode 4 at two waves took 3.9 ms at 4096 x 4096
+// instead of 2.4.
+template <int MODE, bool NU = false>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MODE == 6 ? 2 : 3)))
+setup_kernel(BlockRange r, Bc7Params prm, Work w,
+                                                   const uint32_t *sctab) {
+  __shared__ uint32_t s_px[64 * kPxStride];
+  __shared__ uint32_t s_km[kSetupBuckets(MODE) * 3 * 64];
+  setup_run<MODE, NU>(r, prm, w, sctab, s_px, s_km);
+}
+
+// Every mode in one launch, for jobs that leave the chip idle: a batch of fits
+// takes 50 to 170 us whatever the job's size (one lane's serial fit), so
+// eight launches in a row add up where one lets the modes run side by side.
+// Consecutive workgroups start on different modes; the annealing states come
+// out in no order but the rotation modes' place.
+template <bool NU>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
+setup_all_kernel(BlockRange r, Bc7Params prm, Work w,
+                                                       const uint32_t *sctab) {
+  __shared__ uint32_t s_px[64 * kPxStride];
+  __shared__ uint32_t s_km[kSetupBuckets(6) * 3 * 64];
+  for (uint32_t k = 0; k < 8; k++) {
+    switch ((blockIdx.x + k) & 7u) {
+      case 0: setup_run<4, NU>(r, prm, w, sctab, s_px, s_km); break;
+      case 1: setup_run<0, NU>(r, prm, w, sctab, s_px, s_km); break;
+      case 2: setup_run<2, NU>(r, prm, w, sctab, s_px, s_km); break;
+      case 3: setup_run<1, NU>(r, prm, w, sctab, s_px, s_km); break;
+      case 4: setup_run<3, NU>(r, prm, w, sctab, s_px, s_km); break;
+      case 5: setup_run<7, NU>(r, prm, w, sctab, s_px, s_km); break;
+      case 6: setup_run<6, NU>(r, prm, w, sctab, s_px, s_km); break;
+      default: setup_run<5, NU>(r, prm, w, sctab, s_px, s_km); break;
     }
   }
 }
@@ -3214,6 +3388,7 @@ __device__ __forceinline__ void spread_run(const BlockRange &r, const Bc7Params 
   constexpr int P = 16 / G;  // pixels per lane
   constexpr bool kTail = SRC == kFromTail;
   constexpr uint64_t kLeaders = group_leaders(G);
+  const StateMap sm = state_map(w);
   constexpr uint64_t kGroup = (1ull << G) - 1ull;
   const int lane = threadIdx.x & 63, m = lane & (G - 1), lead = lane & ~(G - 1);
   const int q = (int)prm.quality;
@@ -3243,7 +3418,7 @@ __device__ __forceinline__ void spread_run(const BlockRange &r, const Bc7Params 
       if (!has && item < total) {
         const uint32_t at = end - 1u - item;
         const TailState *ts = kTail ? tail + at : nullptr;
-        const AState *st = kTail ? nullptr : w.astate + (w.alist ? w.alist[at] : at);
+        const AState *st = kTail ? nullptr : w.astate + (w.alist ? w.alist[at] : sm.slot(at));
         has = true;
         id = kTail ? ts->id : st->id;
         info = kTail ? ts->info : st->info;
@@ -3418,7 +3593,9 @@ __global__ void __launch_bounds__(256) anneal_spread_kernel(BlockRange r, Bc7Par
   __shared__ __align__(4) uint8_t s_quant[kStepQuantBytes];
   step_quant_load(s_quant);
   __syncthreads();
-  const uint32_t total = *(volatile uint32_t *)&w.counters[TAIL ? 22 : (w.alist ? 18 : 16)];
+  const uint32_t total = TAIL      ? *(volatile uint32_t *)&w.counters[22]
+                         : w.alist ? *(volatile uint32_t *)&w.counters[18]
+                                   : state_map(w).count();
   unsigned long long n_ref = 0, n_gpu = 0;
   spread_run<16, TAIL ? kFromTail : kFromList, COUNT>(r, prm, w, tail, s_quant, 0, total,
                                                       &w.counters[TAIL ? 23 : 17], n_ref, n_gpu);
@@ -3444,22 +3621,22 @@ anneal_kernel(BlockRange r, Bc7Params prm, Work w, uint32_t unroll, uint32_t tai
   const int lane = threadIdx.x & 63;
   unsigned long long n_ref = 0, n_gpu = 0;  // COUNT
   const uint64_t lt = (1ull << lane) - 1ull;
-  uint32_t total = *(volatile uint32_t *)&w.counters[w.alist ? 18 : 16];
+  const StateMap sm = state_map(w);
+  uint32_t total = w.alist ? *(volatile uint32_t *)&w.counters[18] : sm.count();
   // odd row stride: conflict-free
   __shared__ uint32_t s_px[256 * kRowWords];
   __shared__ __align__(4) uint8_t s_quant[kStepQuantBytes];
   step_quant_load(s_quant);
   __syncthreads();
-  // Learned search: the list is in state order, and the set-up kernels
-  // append the rotation modes' states last (counters[19] holds the first of
-  // them): the list's rotation states are its suffix.  Their chains are the
+  // Learned search: the list is in state order, so its rotation states (slots
+  // past the front's) are its suffix.  Their chains are the
   // longest by far (to 1410 steps, against a mean of 66 in mode 1), so the
   // first rot_groups workgroups start on them at once, four lanes each, while
   // the others run the rest.  (The reference search's list is mostly rotation
   // states: one lane each is the cheapest form, and the list starts with
   // them.)
   if (!NU && rot_groups && w.alist) {
-    const uint32_t first_rot = *(volatile uint32_t *)&w.counters[19];
+    const uint32_t first_rot = sm.front;
     uint32_t lo = 0, hi = total;  // first list entry >= first_rot
     while (lo < hi) {
       const uint32_t mid = (lo + hi) >> 1;
@@ -3508,7 +3685,7 @@ anneal_kernel(BlockRange r, Bc7Params prm, Work w, uint32_t unroll, uint32_t tai
           // mode-1 candidates, and the short mode-7 chains are among the last
           // loaded, which keeps the tail of the launch short
           const uint32_t item = total - 1u - (wbase + rank);
-          lane_load<NU>(L, r, prm, w.astate[w.alist ? w.alist[item] : item]);
+          lane_load<NU>(L, r, prm, w.astate[w.alist ? w.alist[item] : sm.slot(item)]);
         }
         wbase += min(avail, (uint32_t)__popcll(need));
       }
@@ -3939,7 +4116,7 @@ __global__ void __launch_bounds__(64) label_kernel(BlockRange r, int mode, uint3
                                                    const uint32_t *sctab,
                                                    unsigned long long *best, float *errs) {
   __shared__ uint32_t s_px[64 * kPxStride];
-  __shared__ float s_km[16 * 5 * 64];  // k-means sums and counts (up to 16 buckets)
+  __shared__ uint32_t s_km[16 * 3 * 64];  // k-means sums and counts (up to 16 buckets)
   const uint64_t items = (uint64_t)r.num_blocks * nslots;
   for (uint64_t item = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; item < items;
        item += (uint64_t)gridDim.x * blockDim.x) {
@@ -4017,9 +4194,6 @@ __global__ void __launch_bounds__(256) fill_kernel(uint32_t *p, uint32_t n, uint
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
 }
-
-// The annealing states appended so far (before the rotation modes' set-up).
-__global__ void mark_kernel(uint32_t *counters) { counters[19] = counters[16]; }
 
 __global__ void reset_kernel(uint32_t *counters, int n) {
   const int i = threadIdx.x;
@@ -4151,8 +4325,15 @@ constexpr uint32_t kTailLanes = 12;
 // (learned 4096x4096: 4 3.9 ms, 8 3.4, 12 3.3, 16 4.1).
 constexpr uint32_t kRotShare = 10;
 // Workgroups per CU of the one-lane-per-pixel form: five fit, but more waves
-// on a SIMD slow the longest chain (508x380: 6 2.12 ms, 4 2.04, 3 2.05).
-constexpr uint32_t kSpreadWgPerCu = 4;
+// on a SIMD slow the longest chain (508x380: 4 2.10 ms, 3 1.99, 2 1.83, 1 2.64;
+// learned 1024x1024: 4 1.10, 3 1.04, 2 0.97, 1 1.11).
+constexpr uint32_t kSpreadWgPerCu = 2;
+
+// Blocks up to which every mode's set-up runs in one launch (64x64: 0.89 ms of
+// eight launches, 0.17 of one; 508x380 1.07 and 0.72; learned 1024x1024 0.95
+// and 0.80, 2048x2048 1.35 and 1.26, but the merged launch mixes the modes in
+// the annealing list, which costs the one-lane form as much again).
+constexpr uint32_t kSetupAllBlocks = kSpreadBlocks, kSetupAllBlocksLearned = kSpreadBlocksLearned;
 
 // waves: persistent waves of the one-lane form.  tail: memory for tail_cap
 // candidates handed over.
@@ -4352,9 +4533,18 @@ hipError_t bc7_encode(const BlockRange &r, const Bc7Params &p, const Bc7Scratch 
     timing_end(t, kTagBc7Select, stream);
   }
   t = timing_begin(stream);
-  // annealing-state order: modes 0, 2, 3, 7, 6, 1, then the rotation modes 4
-  // and 5 (the mark between them records where they begin)
-  if (nu) {
+  if (n <= (learned ? kSetupAllBlocksLearned : kSetupAllBlocks)) {
+    const uint32_t waves = persistent < (uint32_t)g_num_cus[dev] * 8u
+                               ? (persistent + 7u) / 8u * 8u
+                               : (uint32_t)g_num_cus[dev] * 8u;
+    if (nu)
+      hipLaunchKernelGGL(bc7::setup_all_kernel<true>, dim3(waves), dim3(64), 0, stream, r, p, w,
+                         sct);
+    else
+      hipLaunchKernelGGL(bc7::setup_all_kernel<false>, dim3(waves), dim3(64), 0, stream, r, p, w,
+                         sct);
+  } else if (nu) {
+    // annealing-state order: modes 0, 2, 3, 7, 6, 1 in front, 5 and 4 behind
     hipLaunchKernelGGL((bc7::setup_kernel<0, true>), dim3(persistent), dim3(64), 0, stream, r,
                        p, w, sct);
     hipLaunchKernelGGL((bc7::setup_kernel<2, true>), dim3(persistent), dim3(64), 0, stream, r,
@@ -4367,7 +4557,6 @@ hipError_t bc7_encode(const BlockRange &r, const Bc7Params &p, const Bc7Scratch 
                        p, w, sct);
     hipLaunchKernelGGL((bc7::setup_kernel<1, true>), dim3(persistent), dim3(64), 0, stream, r,
                        p, w, sct);
-    hipLaunchKernelGGL(bc7::mark_kernel, dim3(1), dim3(1), 0, stream, w.counters);
     hipLaunchKernelGGL((bc7::setup_kernel<4, true>), dim3(persistent), dim3(64), 0, stream, r,
                        p, w, sct);
     hipLaunchKernelGGL((bc7::setup_kernel<5, true>), dim3(persistent), dim3(64), 0, stream, r,
@@ -4379,7 +4568,6 @@ hipError_t bc7_encode(const BlockRange &r, const Bc7Params &p, const Bc7Scratch 
     hipLaunchKernelGGL(bc7::setup_kernel<7>, dim3(persistent), dim3(64), 0, stream, r, p, w, sct);
     hipLaunchKernelGGL(bc7::setup_kernel<6>, dim3(persistent), dim3(64), 0, stream, r, p, w, sct);
     hipLaunchKernelGGL(bc7::setup_kernel<1>, dim3(persistent), dim3(64), 0, stream, r, p, w, sct);
-    hipLaunchKernelGGL(bc7::mark_kernel, dim3(1), dim3(1), 0, stream, w.counters);
     hipLaunchKernelGGL(bc7::setup_kernel<4>, dim3(persistent), dim3(64), 0, stream, r, p, w, sct);
     hipLaunchKernelGGL(bc7::setup_kernel<5>, dim3(persistent), dim3(64), 0, stream, r, p, w, sct);
   }
@@ -4397,15 +4585,11 @@ hipError_t bc7_encode(const BlockRange &r, const Bc7Params &p, const Bc7Scratch 
       t = timing_begin(stream);
       // ordered compaction of the annealing list (grid covers the largest list)
       const uint32_t nlist = (uint32_t)((nc + bc7::kListChunk - 1) / bc7::kListChunk);
-      hipLaunchKernelGGL(bc7::list_count_kernel, dim3(nlist), dim3(256), 0, stream,
-                         (const uint32_t *)w.aid, (const uint32_t *)w.counters,
-                         (const uint32_t *)w.sel, cerr, q0err, chunk_count);
-      hipLaunchKernelGGL(bc7::list_scan_kernel, dim3(1), dim3(256), 0, stream, w.counters,
-                         chunk_count);
-      hipLaunchKernelGGL(bc7::list_write_kernel, dim3(nlist), dim3(256), 0, stream,
-                         (const uint32_t *)w.aid, (const uint32_t *)w.counters,
-                         (const uint32_t *)w.sel, cerr, q0err, (const uint32_t *)chunk_count,
-                         alist);
+      hipLaunchKernelGGL(bc7::list_count_kernel, dim3(nlist), dim3(256), 0, stream, w, cerr,
+                         q0err, chunk_count);
+      hipLaunchKernelGGL(bc7::list_scan_kernel, dim3(1), dim3(256), 0, stream, w, chunk_count);
+      hipLaunchKernelGGL(bc7::list_write_kernel, dim3(nlist), dim3(256), 0, stream, w, cerr,
+                         q0err, (const uint32_t *)chunk_count, alist);
       launch_anneal(persistent, g_num_cus[dev], r, p, wa, tail, tail_cap, stream);
       timing_end(t, kTagBc7Anneal, stream);
     }
