@@ -659,11 +659,12 @@ __device__ __forceinline__ uint32_t fit_key(uint64_t seed, uint64_t block_id, ui
 }
 
 // x: key + (draws made) * 0x9E3779B9, kept as a running sum.
+constexpr uint32_t kRngStep = 0x9E3779B9u;
 struct Rng {
   uint32_t x;
   __device__ __forceinline__ uint32_t next() {
     const uint32_t h = mix32(x);
-    x += 0x9E3779B9u;
+    x += kRngStep;
     return h;
   }
   __device__ __forceinline__ uint32_t next16() { return next() >> 16; }
@@ -3013,18 +3014,18 @@ __device__ __forceinline__ void pick_neighbor(const StepCfg &k, bool live, SubSt
 
 // The rest of a step, once the neighbour's error is known: acceptance and
 // the best state (Compressor.cpp:590-624).  Returns whether the best state
-// was replaced; live becomes false when the subset has finished.
+// was replaced, and in `accept` whether the neighbour was taken; live becomes
+// false when the subset has finished.
 template <bool NU = false>
 __device__ __forceinline__ bool finish_step(SubState &t, bool &live, uint32_t err, uint32_t np1,
-                                            uint32_t np2, uint32_t npbc, int q) {
+                                            uint32_t np2, uint32_t npbc, int q, bool &accept) {
   // the acceptance draw, made only where the error is not below cur
   Rng rng;
   rng.x = t.x;
   const float rr = rng.frand();
   const bool lower = err < t.cur;
-  const bool accept =
-      live & (lower | accept_worse(rr, NU ? __uint_as_float(t.cur) : (float)t.cur,
-                                   NU ? __uint_as_float(err) : (float)err, q, t.energy));
+  accept = live & (lower | accept_worse(rr, NU ? __uint_as_float(t.cur) : (float)t.cur,
+                                        NU ? __uint_as_float(err) : (float)err, q, t.energy));
   t.x = lower ? t.x : rng.x;
   t.cur = accept ? err : t.cur;
   t.p1 = accept ? np1 : t.p1;
@@ -3223,7 +3224,8 @@ __device__ __forceinline__ void lane_step_n(Lane &L, const uint8_t *quant, int q
   auto finish = [&](SubState &t, int s, const Next &n, uint64_t mine) {
     bool live = (L.active >> s) & 1u;
     const uint32_t was = live ? 1u << s : 0u;
-    const bool better = finish_step<NU>(t, live, n.err, n.p1, n.p2, n.pbc, q);
+    bool accept;
+    const bool better = finish_step<NU>(t, live, n.err, n.p1, n.p2, n.pbc, q, accept);
     taken |= better ? mine : 0ull;
     if (!live) L.active &= ~was;
   };
@@ -3355,6 +3357,16 @@ constexpr int kHandGroups = 4;
 // more issue: this form is for lists that leave the chip idle, where the
 // longest chain sets the time.  G = 4: candidates of one subset only, four
 // pixels a lane, between the two in both respects.
+//
+// Looking ahead (G = 16): a wave left with one or two candidates, or given no
+// more (lists shorter than the waves), runs each with two or four rows.  A
+// step that is rejected leaves the state as it was but for three draws of the
+// random stream and the energy, so row k proposes and scores the k-th next
+// step as if the ones before it were rejected, and the first row where
+// something else happens (an acceptance, a repeated draw, the end) gives the
+// next state.  Modes 4 and 5 accept one step in five and one in four, the
+// others fewer than one in sixteen: four rows advance 2.8 and nearly 4 steps
+// at once.  The subsets are chains of their own and may advance differently.
 // ---------------------------------------------------------------------------
 // Sum over the G lanes of a group (every lane of the wave active).
 template <int G>
@@ -3372,7 +3384,7 @@ __device__ __forceinline__ uint32_t group_sum(uint32_t v) {
 }
 
 // Runs the candidates [begin, end) of a list, taken from its end through
-// *fetch, until none is left.  SRC: kFromList (the annealing states),
+// *fetch by `waves` waves, until none is left.  SRC: kFromList (the annealing states),
 // kFromTail (the candidates handed over in `tail`) or kFromListHand (the
 // annealing states; once they are used up a wave with few groups running
 // hands them over through `tail` and returns).
@@ -3382,7 +3394,8 @@ enum { kFromList = 0, kFromTail = 1, kFromListHand = 2 };
 template <int G, int SRC, bool COUNT>
 __device__ __forceinline__ void spread_run(const BlockRange &r, const Bc7Params &prm,
                                            const Work &w, TailState *tail, const uint8_t *quant,
-                                           uint32_t begin, uint32_t end, uint32_t *fetch,
+                                           uint32_t begin, uint32_t end, uint32_t waves,
+                                           uint32_t *fetch,
                                            unsigned long long &n_ref, unsigned long long &n_gpu) {
   static_assert(G == 16 || G == 4, "lanes per candidate");
   constexpr int P = 16 / G;  // pixels per lane
@@ -3390,7 +3403,7 @@ __device__ __forceinline__ void spread_run(const BlockRange &r, const Bc7Params 
   constexpr uint64_t kLeaders = group_leaders(G);
   const StateMap sm = state_map(w);
   constexpr uint64_t kGroup = (1ull << G) - 1ull;
-  const int lane = threadIdx.x & 63, m = lane & (G - 1), lead = lane & ~(G - 1);
+  const int lane = threadIdx.x & 63, m = lane & (G - 1);
   const int q = (int)prm.quality;
   const uint32_t total = end - begin;
   // the candidate (the same in the group) and its constants
@@ -3403,11 +3416,16 @@ __device__ __forceinline__ void spread_run(const BlockRange &r, const Bc7Params 
   bool active = false;
   SubState t = {};
   bool exhausted = total == 0;
+  // rows per candidate: 1, 2 or 4 (see above); lead: this lane's group of rows
+  int rpc = G == 16 && total <= 2 * waves ? (total <= waves ? 4 : 2) : 1;
+  int lead = lane & ~(G * rpc - 1);
   for (;;) {
     // idle groups take the next candidates, from the end of the list (the
     // rotation modes, whose chains are the longest, first)
-    uint64_t hasm = __ballot(has) & kLeaders;
-    const uint64_t need = ~hasm & kLeaders;
+    uint64_t leaders = kLeaders;
+    if (G == 16 && rpc > 1) leaders = rpc == 2 ? group_leaders(32) : 1ull;
+    uint64_t hasm = __ballot(has) & leaders;
+    const uint64_t need = ~hasm & leaders;
     if (need && !exhausted) {
       const uint32_t want = (uint32_t)__popcll(need);
       uint32_t base = 0;
@@ -3464,7 +3482,7 @@ __device__ __forceinline__ void spread_run(const BlockRange &r, const Bc7Params 
                                    : (uint64_t)st->idx_lo | ((uint64_t)st->idx_hi << 32);
         bidx = (uint32_t)(idx >> (4 * P * m)) & ((1u << (4 * P)) - 1u);
       }
-      hasm = __ballot(has) & kLeaders;
+      hasm = __ballot(has) & leaders;
     }
     if (!hasm) break;
     if (SRC == kFromListHand && exhausted && __popcll(hasm) <= kHandGroups) {
@@ -3491,20 +3509,69 @@ __device__ __forceinline__ void spread_run(const BlockRange &r, const Bc7Params 
       }
       break;
     }
+    if (G == 16 && rpc < 4 && exhausted) {
+      // few candidates left: give each more rows
+      const int n = __popcll(hasm);
+      const int wide = n == 1 ? 4 : (n == 2 ? 2 : 1);
+      if (wide > rpc) {
+        rpc = wide;
+        lead = lane & ~(G * rpc - 1);
+        // the first or the last running group's lane of the same pixel
+        const int first = __ffsll((unsigned long long)hasm) - 1;
+        const int last = 63 - __clzll((long long)hasm);
+        const int from = (lead == 0 ? first : last) + m;
+        auto take = [&](auto &v) { v = __shfl(v, from); };
+        take(id);
+        take(info);
+        take(extra);
+        take(sel02);
+        take(sel13);
+        take(ptmode);
+        take(nsub);
+        take(k.s02);
+        take(k.s13);
+        take(k.k2_02);
+        take(k.k2_13);
+        take(k.flip);
+        take(k.sh);
+        take(k.nopb);
+        take(k.qc);
+        take(k.qa);
+        take(k.kf);
+        take(k.wf.m);
+        take(k.wf.b);
+        take(p02[0]);
+        take(p13[0]);
+        take(sub);
+        take(bidx);
+        take(t.p1);
+        take(t.p2);
+        take(t.bp1);
+        take(t.bp2);
+        take(t.cur);
+        take(t.best);
+        take(t.cpbc);
+        take(t.bpbc);
+        take(t.x);
+        take(t.energy);
+        active = __shfl(active ? 1 : 0, from) != 0;
+        has = true;
+      }
+    }
     // stale in rows without a candidate: harmless
     const bool multi = G == 16 && __ballot(nsub > 1) != 0;
-    for (int u = 0; u < 4; u++) {
-      if constexpr (COUNT) {
-        const uint64_t act = __ballot(active);
-        n_ref += active ? (unsigned)P : 0u;
-        n_gpu += (m == 0 && ((act >> lead) & kGroup)) ? 16u : 0u;
-      }
+    // proposes a neighbour of v, scores it and finishes v's step; nidx: its
+    // indices.  Returns finish_step's result.
+    auto step = [&](SubState &v, bool &live, uint32_t &nidx, bool &accept, bool &again) {
       uint32_t np1, np2, npbc;
-      pick_neighbor(k, active, t, np1, np2, npbc);
+      const uint32_t x0 = v.x;
+      pick_neighbor(k, live, v, np1, np2, npbc);
+      again = v.x != x0 + 2u * kRngStep;
       SubConst sc = sub_const(step_quant(quant, k, np1, (npbc >> k.sh) & 1u),
                               step_quant(quant, k, np2, npbc & 1u));
       rotate_axis(sc, ptmode, sel02, sel13);
-      uint32_t me = 0, nidx = 0;
+      uint32_t me = 0;
+      nidx = 0;
 #pragma unroll
       for (int i = 0; i < P; i++) {
         uint32_t j;
@@ -3518,7 +3585,61 @@ __device__ __forceinline__ void spread_run(const BlockRange &r, const Bc7Params 
         const uint32_t t2 = group_sum<G>(sub == 2 ? me : 0u);
         err = sub == 0 ? err - t1 - t2 : (sub == 1 ? t1 : t2);
       }
-      if (finish_step(t, active, err, np1, np2, npbc, q)) bidx = nidx;
+      return finish_step(v, live, err, np1, np2, npbc, q, accept);
+    };
+    if (G == 4 || rpc == 1) {
+      for (int u = 0; u < 4; u++) {
+        if constexpr (COUNT) {
+          const uint64_t act = __ballot(active);
+          n_ref += active ? (unsigned)P : 0u;
+          n_gpu += (m == 0 && ((act >> lead) & kGroup)) ? 16u : 0u;
+        }
+        uint32_t nidx;
+        bool accept, again;
+        if (step(t, active, nidx, accept, again)) bidx = nidx;
+      }
+    } else {
+      const int row = (lane >> 4) & (rpc - 1);
+      const uint64_t rows = rpc == 4 ? kLeaders : 0x00010001ull;
+      for (int u = 0; u < 4; u++) {
+        // this row's step: `row` rejections ahead of t
+        SubState v = t;
+        v.x += (uint32_t)row * 3u * kRngStep;
+        v.energy += row;
+        bool live = active, accept, again;
+        uint32_t nidx;
+        const bool better = step(v, live, nidx, accept, again);
+        const uint64_t event = __ballot(active & (accept | again | !live));
+        // the first row of this lane's group with an event in its chain
+        const uint64_t mine = (event >> (lead + m)) & rows;
+        const int last = mine ? (__ffsll((unsigned long long)mine) - 1) >> 4 : rpc - 1;
+        if constexpr (COUNT) {
+          const uint64_t act = __ballot(active);
+          n_ref += active && row == 0 ? (unsigned)last + 1u : 0u;
+          n_gpu += (m == 0 && ((act >> lead) & kGroup)) ? 16u : 0u;
+        }
+        if (!event) {
+          t.x += (uint32_t)rpc * 3u * kRngStep;
+          t.energy += rpc;
+          continue;
+        }
+        const int from = lead + 16 * last + m;
+        uint32_t bits = v.cpbc | (v.bpbc << 2) | ((better ? nidx : bidx) << 4) |
+                        ((live ? 1u : 0u) << 8);
+        bits = __shfl(bits, from);
+        t.p1 = __shfl(v.p1, from);
+        t.p2 = __shfl(v.p2, from);
+        t.bp1 = __shfl(v.bp1, from);
+        t.bp2 = __shfl(v.bp2, from);
+        t.cur = __shfl(v.cur, from);
+        t.best = __shfl(v.best, from);
+        t.x = __shfl(v.x, from);
+        t.energy = __shfl(v.energy, from);
+        t.cpbc = bits & 3u;
+        t.bpbc = (bits >> 2) & 3u;
+        bidx = (bits >> 4) & 15u;
+        active = (bits >> 8) & 1u;
+      }
     }
     // finished groups write their records (lane_finish)
     const uint64_t act = __ballot(active);
@@ -3546,7 +3667,7 @@ __device__ __forceinline__ void spread_run(const BlockRange &r, const Bc7Params 
         }
       }
     }
-    if (done) {
+    if (done && (G == 4 || lane - lead < G)) {
       CandRec *rc = &w.rec[id];
       if (leader) {
         Fit f;
@@ -3567,9 +3688,8 @@ __device__ __forceinline__ void spread_run(const BlockRange &r, const Bc7Params 
         rc->meta = (rc->meta & ~((1u << (2 * nsub)) - 1u)) | pbcs | kMetaAnnealed;
         rc->err = sum;
       }
-      has = false;
-      active = false;
     }
+    if (done) has = active = false;
   }
 }
 
@@ -3598,7 +3718,8 @@ __global__ void __launch_bounds__(256) anneal_spread_kernel(BlockRange r, Bc7Par
                                    : state_map(w).count();
   unsigned long long n_ref = 0, n_gpu = 0;
   spread_run<16, TAIL ? kFromTail : kFromList, COUNT>(r, prm, w, tail, s_quant, 0, total,
-                                                      &w.counters[TAIL ? 23 : 17], n_ref, n_gpu);
+                                                      4 * gridDim.x, &w.counters[TAIL ? 23 : 17],
+                                                      n_ref, n_gpu);
   if constexpr (COUNT) add_counts(prm, n_ref, n_gpu);
 }
 
@@ -3644,8 +3765,8 @@ anneal_kernel(BlockRange r, Bc7Params prm, Work w, uint32_t unroll, uint32_t tai
       else hi = mid;
     }
     if (blockIdx.x < rot_groups)
-      spread_run<4, kFromListHand, COUNT>(r, prm, w, tail, s_quant, lo, total, &w.counters[21],
-                                          n_ref, n_gpu);
+      spread_run<4, kFromListHand, COUNT>(r, prm, w, tail, s_quant, lo, total, 4 * rot_groups,
+                                          &w.counters[21], n_ref, n_gpu);
     total = lo;
   }
   Lane L = {};  // lanes without a candidate step along on zeros
@@ -4313,9 +4434,9 @@ hipError_t bc7_upload_tables(int device) {
 // Blocks up to which a call's annealing runs one lane per pixel from the
 // start.  Its lists (about 7 states a block in the reference search, 1 in the
 // learned one) then leave the one-lane form too few waves, and the longest
-// chain sets the time: 508x380 (12065 blocks) anneals in 2.0 ms against 2.9,
-// 1000x1024 (64000) in 7.9 against 4.6; learned 1024x1024 in 1.15 against
-// 1.18, 2048x2048 in 3.0 against 1.5.
+// chain sets the time: 508x380 (12065 blocks) anneals in 1.7 ms against 2.9,
+// 1000x1024 (64000) in 7.9 against 4.6; learned 1024x1024 in 0.83 against
+// 1.18, 2048x2048 in 3.0 against 1.3.
 constexpr uint32_t kSpreadBlocks = 1u << 14, kSpreadBlocksLearned = 1u << 16;
 // Running candidates at which a wave of the one-lane form hands over
 // (learned 4096x4096: 4..12 3.3 ms, 16 3.5, 24 3.6, never 3.8; reference
@@ -4325,9 +4446,9 @@ constexpr uint32_t kTailLanes = 12;
 // (learned 4096x4096: 4 3.9 ms, 8 3.4, 12 3.3, 16 4.1).
 constexpr uint32_t kRotShare = 10;
 // Workgroups per CU of the one-lane-per-pixel form: five fit, but more waves
-// on a SIMD slow the longest chain (508x380: 4 2.10 ms, 3 1.99, 2 1.83, 1 2.64;
-// learned 1024x1024: 4 1.10, 3 1.04, 2 0.97, 1 1.11).
-constexpr uint32_t kSpreadWgPerCu = 2;
+// on a SIMD slow the longest chains (508x380: 4 1.75 ms, 3 1.71, 2 1.78; learned
+// 1024x1024: 4 0.87, 3 0.83, 2 0.85).
+constexpr uint32_t kSpreadWgPerCu = 3;
 
 // Blocks up to which every mode's set-up runs in one launch (64x64: 0.89 ms of
 // eight launches, 0.17 of one; 508x380 1.07 and 0.72; learned 1024x1024 0.95
