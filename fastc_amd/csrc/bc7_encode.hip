@@ -32,6 +32,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "../../include/fasthip.h"
 #include "bc7_block_decode.h"
 #include "ranker_tile.h"
@@ -229,84 +231,208 @@ __device__ __forceinline__ void normalize4(float a[4]) {
   for (int k = 0; k < 4; k++) a[k] /= l;
 }
 
+// Packed 16-bit lanes: channels 0 and 2 of a pixel are (pix & 0x00FF00FF),
+// channels 1 and 3 are ((pix >> 8) & 0x00FF00FF); every quantity of the
+// index search fits 16 bits (interpolation sums within +-16352, channel
+// differences within +-255), so v_pk_* and v_dot2 give the exact integers.
+typedef short s16x2 __attribute__((ext_vector_type(2)));
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ u16x2 as_u16x2(uint32_t v) { return __builtin_bit_cast(u16x2, v); }
+__device__ __forceinline__ s16x2 as_s16x2(uint32_t v) { return __builtin_bit_cast(s16x2, v); }
+__device__ __forceinline__ s16x2 as_s16x2(u16x2 v) { return __builtin_bit_cast(s16x2, v); }
+
+// Weight of the second endpoint at index j for nb = 4, 8, 16 entries:
+// (64 j + (nb - 1) / 2) / (nb - 1) by a multiply-shift, equal to
+// kInterpolationValues (Compressor.cpp:159-168); bc7_upload_tables checks
+// every entry on the host before the kernels run.  weight_word holds the
+// weight in its high half, where the packed multiply of interp_err reads it
+// without a shift.
+struct WeightFn {
+  uint32_t m, b;
+};
+__host__ __device__ __forceinline__ WeightFn weight_fn(int nb) {
+  if (nb == 4) return {64u * 21846u, 21846u};
+  if (nb == 8) return {64u * 9363u, 3u * 9363u};
+  return {64u * 4370u, 7u * 4370u};
+}
+__host__ __device__ __forceinline__ uint32_t weight_word(WeightFn fn, uint32_t j) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  // both factors are below 2^24: the full-rate 24-bit multiply-add, which
+  // the compiler only finds where it can see the factors' ranges
+  uint32_t w;
+  asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(w) : "v"(j), "v"(fn.m), "v"(fn.b));
+  return w;
+#else
+  return fn.m * j + fn.b;
+#endif
+}
+__host__ __device__ __forceinline__ uint32_t weight_of(WeightFn fn, uint32_t j) {
+  return weight_word(fn, j) >> 16;
+}
+
+// A texel as the pixel pass reads it: 64 times its channel pairs (each 16-bit
+// lane at most 64 * 255 = 16320).  The interpolated value of an index weight
+// w is (e1 (64 - w) + e2 w + 32) >> 6 = (64 e1 + 32 + (e2 - e1) w) >> 6, so
+// with the texel scaled by 64 its difference to the texel is one shift of
+// one sum, and the texel's projection is 64 times the integer one.
+__device__ __forceinline__ uint32_t pair02x64(uint32_t pix) { return (pix & 0x00FF00FFu) << 6; }
+__device__ __forceinline__ uint32_t pair13x64(uint32_t pix) {
+  return ((pix >> 8) & 0x00FF00FFu) << 6;
+}
+
+// a . b + c in the three-operand form of the instruction: asked to saturate
+// (every sum here is far from the 32-bit range) the compiler cannot take the
+// accumulating two-operand form, which needs its start value moved into place
+// first (three moves per pixel in the pixel pass).
+__device__ __forceinline__ int dot2(s16x2 a, s16x2 b, int c) {
+  return __builtin_amdgcn_sdot2(a, b, c, true);
+}
+
+// Per-subset constants of one annealing step.
+struct SubConst {
+  uint32_t a02, a13;  // 64 * endpoint 1 + 32, channel pairs
+  uint32_t d02, d13;  // endpoint 2 - endpoint 1 (signed pairs)
+  uint32_t q02, q13;  // the projection axis (d, or d seen through a rotation)
+  int ad;             // -64 * endpoint 1 . (endpoint 2 - endpoint 1)
+  float rl;           // 1 / (64 l), l the squared endpoint distance (see pixel_bounds)
+};
+
+__device__ __forceinline__ SubConst sub_const(uint32_t e1, uint32_t e2) {
+  SubConst c;
+  const uint32_t a02 = e1 & 0x00FF00FFu, a13 = (e1 >> 8) & 0x00FF00FFu;
+  const uint32_t b02 = e2 & 0x00FF00FFu, b13 = (e2 >> 8) & 0x00FF00FFu;
+  c.d02 = __builtin_bit_cast(uint32_t, as_s16x2(b02) - as_s16x2(a02));
+  c.d13 = __builtin_bit_cast(uint32_t, as_s16x2(b13) - as_s16x2(a13));
+  c.q02 = c.d02;
+  c.q13 = c.d13;
+  // each 16-bit lane: 64 a + 32 <= 16352
+  c.a02 = (a02 << 6) + 0x00200020u;
+  c.a13 = (a13 << 6) + 0x00200020u;
+  // endpoint 1's projection on the axis, subtracted from each pixel's
+  c.ad = -64 * dot2(as_s16x2(a02), as_s16x2(c.d02), dot2(as_s16x2(a13), as_s16x2(c.d13), 0));
+  const int l = dot2(as_s16x2(c.d02), as_s16x2(c.d02), dot2(as_s16x2(c.d13), as_s16x2(c.d13), 0));
+  // equal endpoints give d = 0 for every pixel, so l = 1 yields index 0
+  const float lf = (float)(l > 0 ? l : 1);
+  // v_rcp_f32 is within 1 ulp; one Newton step makes it the correctly
+  // rounded 1 / l for every l <= 4 * 255^2 (checked for starts within 2 ulp)
+  const float r = __builtin_amdgcn_rcpf(lf);
+  c.rl = __builtin_fmaf(__builtin_fmaf(-lf, r, 1.0f), r, r) * 0x1p-6f;
+  return c;
+}
+
+// The projection axis of a rotation mode (ptmode = rotation + 1).  Its
+// points are the texels with channel r - 1 replaced by alpha (r > 0) and
+// alpha 255 (point_of), so a point's projection is the texel's on a permuted
+// axis (alpha taking channel r - 1's component, that channel none) plus
+// 255 times the axis' alpha component.  sel02 / sel13: v_perm_b32 selectors
+// over (d02, d13), identity without a rotation.
+__device__ __forceinline__ void rotation_selectors(int ptmode, uint32_t &sel02, uint32_t &sel13) {
+  // bytes 0-3 of the selector index d13, 4-7 d02, 0x0c a zero byte
+  sel02 = 0x07060504u;
+  sel13 = 0x03020100u;
+  if (ptmode == 1) sel13 = 0x0c0c0100u;
+  if (ptmode == 2) {
+    sel02 = 0x07060c0cu;
+    sel13 = 0x05040100u;
+  }
+  if (ptmode == 3) sel13 = 0x01000c0cu;
+  if (ptmode == 4) {
+    sel02 = 0x0c0c0504u;
+    sel13 = 0x07060100u;
+  }
+}
+__device__ __forceinline__ void rotate_axis(SubConst &c, int ptmode, uint32_t sel02,
+                                            uint32_t sel13) {
+  c.q02 = __builtin_amdgcn_perm(c.d02, c.d13, sel02);
+  c.q13 = __builtin_amdgcn_perm(c.d02, c.d13, sel13);
+  const int da = (int)c.d13 >> 16;
+  c.ad += ptmode ? 64 * 255 * da : 0;
+}
+
+// Difference of the pixel pairs (64 p) to the interpolant of index weight
+// word ww, (64 e1 + 32 - 64 p + (e2 - e1) w) >> 6 = interpolant - p: z holds
+// 64 e1 + 32 - 64 p, and the sum lies within +-16352, so signed 16-bit lanes
+// hold it exactly.
+__device__ __forceinline__ s16x2 interp_diff(s16x2 z, uint32_t d, uint32_t ww) {
+  const s16x2 w = as_s16x2(ww);
+  const s16x2 W = {w.y, w.y};
+  const s16x2 S = {6, 6};
+  return (as_s16x2(d) * W + z) >> S;
+}
+
+// QuantizedError's neighbouring indices (RGBAEndpoints.cpp:240-300) of a
+// pixel: j1 = floor(t), j2 = ceil(t), both clamped to the index range, of the
+// reference's t = fl(fl(d / l) * kf) (float, d the integer projection, l the
+// integer squared distance, kf = nb - 1).  Those equal the floor and ceiling
+// of the rational d kf / l: its distance to an integer, when nonzero, is at
+// least 1 / l >= 1 / (4 * 255^2) = 3.8e-6, more than the float error of at
+// most 2^-23 |t| <= 1.9e-6 for |t| <= 16 (larger |t| is clamped away), and
+// fl(fl(k / kf) kf) = k for every integer 0 <= k <= kf in {3, 7, 15} (checked
+// exhaustively).
+//
+// Here u = fl(64 d * rl) clamped to [0, 1] (64 d is below 2^24, so its
+// conversion is exact; a d below 0 or above l clamps to the end index), and
+// the floor and ceiling are truncations of fma(u, kf, 1.9e-6) and
+// fma(u, kf, 1 - 1.9e-6).  Exact for every l up to 4 * 255^2, d in 0..l and
+// kf: checked exhaustively at the steps of both functions of d, which are
+// monotone.  The pass is bound by VALU issue: an integer quotient corrected
+// with the exact remainder took 17 instructions per pixel where this takes 9;
+// with the texels kept as scaled pairs (no unpacking, one subtraction per
+// pair) and the rotation folded into the axis (no separate point) the pass
+// went from about 54 instructions per pixel to 33, and the 4096 x 4096
+// annealing from 46.0 to 34.3 ms (reference search) and 5.2 to 4.1 ms
+// (learned).
+constexpr float kIndexSlack = 1.9e-6f;
+
+__device__ __forceinline__ void pixel_bounds(uint32_t p02, uint32_t p13, const SubConst &c,
+                                             float kf, uint32_t &j1, uint32_t &j2) {
+  const int d = dot2(as_s16x2(p02), as_s16x2(c.q02), dot2(as_s16x2(p13), as_s16x2(c.q13), c.ad));
+  const float u = __builtin_amdgcn_fmed3f((float)d * c.rl, 0.0f, 1.0f);
+  j1 = (uint32_t)__builtin_fmaf(u, kf, kIndexSlack);
+  j2 = (uint32_t)__builtin_fmaf(u, kf, 1.0f - kIndexSlack);
+}
+
+// The per-pixel index search without branches: both neighbouring indices
+// are scored and the second kept only when strictly better (where the two
+// are the same index the errors are equal).  Returns the error, the index in
+// *best.  p02, p13: the texel's pairs times 64.
+__device__ __forceinline__ uint32_t pixel_err(uint32_t p02, uint32_t p13, const SubConst &c,
+                                              float kf, WeightFn wf, uint32_t *best) {
+  uint32_t j1, j2;
+  pixel_bounds(p02, p13, c, kf, j1, j2);
+  const s16x2 z02 = as_s16x2(c.a02) - as_s16x2(p02), z13 = as_s16x2(c.a13) - as_s16x2(p13);
+  const uint32_t w1 = weight_word(wf, j1), w2 = weight_word(wf, j2);
+  const s16x2 x02 = interp_diff(z02, c.d02, w1), x13 = interp_diff(z13, c.d13, w1);
+  const s16x2 y02 = interp_diff(z02, c.d02, w2), y13 = interp_diff(z13, c.d13, w2);
+  const uint32_t e1 = (uint32_t)dot2(x02, x02, dot2(x13, x13, 0));
+  const uint32_t e2 = (uint32_t)dot2(y02, y02, dot2(y13, y13, 0));
+  *best = e2 < e1 ? j2 : j1;
+  return e2 < e1 ? e2 : e1;
+}
+
 // QuantizedError with endpoints already quantised to qp1/qp2
-// (RGBAEndpoints.cpp:190-310, uniform metric).  Indices are written at pixel
-// positions (4 bits each) for the pixels in smask.
-// UNROLL: 16 when px is a register array (constant indices), 1 when it
-// points to LDS (the loop stays rolled).
-template <int UNROLL>
+// (RGBAEndpoints.cpp:190-310, uniform metric) by the pixel pass above.
+// Indices are written at pixel positions (4 bits each) for the pixels in
+// smask.  (With the reference's float quotient and the weights from their
+// table, two divisions and four dependent loads a pixel, this took about a
+// tenth of a fit.)
 __device__ __forceinline__ uint32_t qerr(const uint32_t px[16], uint32_t smask, int ptmode,
                                          uint32_t qp1, uint32_t qp2, int nb, uint64_t &idx) {
-  int a[4], b[4], dir[4];
-  int lsq = 0;
-#pragma unroll
-  for (int k = 0; k < 4; k++) {
-    a[k] = (int)chan(qp1, k);
-    b[k] = (int)chan(qp2, k);
-    dir[k] = b[k] - a[k];
-    lsq += dir[k] * dir[k];
-  }
+  uint32_t sel02, sel13;
+  rotation_selectors(ptmode, sel02, sel13);
+  SubConst c = sub_const(qp1, qp2);
+  rotate_axis(c, ptmode, sel02, sel13);
+  const WeightFn wf = weight_fn(nb);
+  const float kf = (float)(nb - 1);
   idx = 0;
   uint32_t total = 0;
-  if (lsq == 0) {
-#pragma unroll
-    for (int i = 0; i < 16; i++) {
-      if (!((smask >> i) & 1)) continue;
-      uint32_t e = 0;
-#pragma unroll
-      for (int k = 0; k < 4; k++) {
-        const int d = (int)chan(px[i], k) - a[k];
-        e += (uint32_t)(d * d);
-      }
-      total += e;
-    }
-    return total;
-  }
-  const int prec = nb == 4 ? 2 : (nb == 8 ? 3 : 4);
-  const float flsq = (float)lsq;
-  const float kf = (float)(nb - 1);
-#pragma unroll UNROLL
+#pragma unroll 1
   for (int i = 0; i < 16; i++) {
     if (!((smask >> i) & 1)) continue;
-    const uint32_t pt = point_of(px[i], ptmode);
-    int d = 0;
-#pragma unroll
-    for (int k = 0; k < 4; k++) d += ((int)chan(pt, k) - a[k]) * dir[k];
-    const float pct = (float)d / flsq;
-    const float t = pct * kf;
-    int j1 = (int)floorf(t);
-    int j2 = (int)ceilf(t);
-    j1 = j1 < 0 ? 0 : j1;
-    j1 = j1 > nb - 1 ? nb - 1 : j1;
-    j2 = j2 > nb - 1 ? nb - 1 : j2;
     const uint32_t pix = px[i];
-    uint32_t e1 = 0;
-    {
-      const int w1 = kW[prec - 1][j1], w0 = 64 - w1;
-#pragma unroll
-      for (int k = 0; k < 4; k++) {
-        const int ip = (a[k] * w0 + b[k] * w1 + 32) >> 6;
-        const int dd = (int)chan(pix, k) - ip;
-        e1 += (uint32_t)(dd * dd);
-      }
-    }
-    int best = j1;
-    uint32_t me = e1;
-    if (j2 > j1) {
-      const int w1 = kW[prec - 1][j2], w0 = 64 - w1;
-      uint32_t e2 = 0;
-#pragma unroll
-      for (int k = 0; k < 4; k++) {
-        const int ip = (a[k] * w0 + b[k] * w1 + 32) >> 6;
-        const int dd = (int)chan(pix, k) - ip;
-        e2 += (uint32_t)(dd * dd);
-      }
-      if (e2 < e1) {
-        best = j2;
-        me = e2;
-      }
-    }
-    total += me;
+    uint32_t best;
+    total += pixel_err(pair02x64(pix), pair13x64(pix), c, kf, wf, &best);
     idx |= (uint64_t)best << (4 * i);
   }
   return total;
@@ -675,17 +801,6 @@ struct Rng {
   }
 };
 
-// Packed 16-bit lanes: channels 0 and 2 of a pixel are (pix & 0x00FF00FF),
-// channels 1 and 3 are ((pix >> 8) & 0x00FF00FF); every quantity of the
-// index search fits 16 bits (interpolation sums within +-16352, channel
-// differences within +-255), so v_pk_* and v_dot2 give the exact integers.
-typedef short s16x2 __attribute__((ext_vector_type(2)));
-typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ u16x2 as_u16x2(uint32_t v) { return __builtin_bit_cast(u16x2, v); }
-__device__ __forceinline__ s16x2 as_s16x2(uint32_t v) { return __builtin_bit_cast(s16x2, v); }
-__device__ __forceinline__ s16x2 as_s16x2(u16x2 v) { return __builtin_bit_cast(s16x2, v); }
-
 // One endpoint's neighbour: every channel moved by delta = k1 - bit * k2
 // (channel pairs; bit k of the draw's top half is channel k's), clamped to
 // 0..255.
@@ -932,7 +1047,7 @@ __device__ __forceinline__ void kmeans_setup(const Fit &f, uint32_t q, const uin
   const uint32_t q1 = to_pixel_int(g1, f.qmask, pbc_bit(f.pbit_type, pbc, 0));
   const uint32_t q2 = to_pixel_int(g2, f.qmask, pbc_bit(f.pbit_type, pbc, 1));
   if constexpr (NU) out.err = __float_as_uint(qerr_nu<1>(px, smask, ptmode, q1, q2, nb, *mr, out.idx));
-  else out.err = qerr<1>(px, smask, ptmode, q1, q2, nb, out.idx);
+  else out.err = qerr(px, smask, ptmode, q1, q2, nb, out.idx);
   out.sc = false;
   out.pbc = pbc;
   if (f.pbit_type != PB_NONE) {
@@ -984,16 +1099,17 @@ __device__ __forceinline__ void subset_setup(const Fit &f, uint32_t q, const uin
 // to *nu_err.
 template <bool NU = false>
 __device__ __forceinline__ uint32_t alpha_fit(const Fit &f, const uint32_t px[16], uint64_t &aidx, uint32_t &a1q,
-                              uint32_t &a2q, float aw = 1.0f, double *nu_err = nullptr) {
-  float avals[16];
-  float amin = FLT_MAX, amax = -FLT_MAX;
-#pragma unroll
+                              uint32_t &a2q, uint32_t *km, float aw = 1.0f,
+                              double *nu_err = nullptr) {
+  const int src = f.rot == 0 ? 3 : f.rot - 1;
+  uint32_t lo = 255, hi = 0;
+#pragma unroll 1
   for (int i = 0; i < 16; i++) {
-    const uint32_t src = f.rot == 0 ? 3 : (uint32_t)(f.rot - 1);
-    avals[i] = (float)chan(px[i], (int)src);
-    amin = avals[i] < amin ? avals[i] : amin;
-    amax = amax < avals[i] ? avals[i] : amax;
+    const uint32_t v = chan(px[i], src);
+    lo = v < lo ? v : lo;
+    hi = v > hi ? v : hi;
   }
+  const float amin = (float)lo, amax = (float)hi;
   const int abits = f.idx_mode == 0 ? kModes[f.mode].alpha_idx_bits : kModes[f.mode].idx_bits;
   const int nb = 1 << abits;
   float a1 = amin, a2 = amax;
@@ -1030,55 +1146,46 @@ __device__ __forceinline__ uint32_t alpha_fit(const Fit &f, const uint32_t px[16
 #pragma unroll
     for (int i = 0; i < 8; i++)
       if (i < nb) vals[i] = amin + ((float)i / (float)(nb - 1)) * (amax - amin);
-    uint32_t bk[16];
+    // every value into its nearest entry's LDS word, sum | count << 16 (as
+    // for the colours, integer sums are the reference's float sums exactly)
+    auto assign = [&]() {
 #pragma unroll
-    for (int i = 0; i < 16; i++) {
-      float md = 255.0f;
-      bk[i] = 0;
+      for (int j = 0; j < 8; j++) km[j * 64] = 0u;
+#pragma unroll 1
+      for (int i = 0; i < 16; i++) {
+        const uint32_t val = chan(px[i], src);
+        const float a = (float)val;
+        float md = 255.0f;
+        int b = 0;
 #pragma unroll
-      for (int j = 0; j < 8; j++) {
-        if (j >= nb) continue;
-        const float d = fabsf(avals[i] - vals[j]);
-        if (d < md) {
-          md = d;
-          bk[i] = (uint32_t)j;
+        for (int j = 0; j < 8; j++) {
+          if (j >= nb) continue;
+          const float d = fabsf(a - vals[j]);
+          if (d < md) {
+            md = d;
+            b = j;
+          }
         }
+        km_add(km + b * 64, val | 0x10000u);
       }
-    }
+    };
     float npts[8];
     bool fixed = false;
     int guard = 0;
+    assign();
     while (!fixed && guard++ < 4096) {
       fixed = true;
 #pragma unroll
       for (int j = 0; j < 8; j++) {
-        float s = 0.0f, c = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 16; i++)
-          if (bk[i] == (uint32_t)j) {
-            s += avals[i];
-            c += 1.0f;
-          }
-        // integer sum over a count of 1..16: the double product is the
+        const uint32_t w = km[j * 64];
+        // integer sum over a count of 0..16: the double product is the
         // correctly rounded quotient (as for the colour k-means)
-        if (c > 0.0f) s = (float)((double)s * kInvCount[(int)c]);
-        npts[j] = c;
+        const float s = (float)((double)(w & 0xFFFFu) * kInvCount[w >> 16]);
+        npts[j] = (float)(w >> 16);
         if (j < nb) fixed = fixed && (s == vals[j]);
         vals[j] = s;
       }
-#pragma unroll
-      for (int i = 0; i < 16; i++) {
-        float md = 255.0f;
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-          if (j >= nb) continue;
-          const float d = fabsf(avals[i] - vals[j]);
-          if (d < md) {
-            md = d;
-            bk[i] = (uint32_t)j;
-          }
-        }
-      }
+      if (!fixed) assign();
     }
     float asq = 0.0f, bsq = 0.0f, ab = 0.0f, ax = 0.0f, bx = 0.0f;
 #pragma unroll
@@ -1110,9 +1217,9 @@ __device__ __forceinline__ uint32_t alpha_fit(const Fit &f, const uint32_t px[16
     const uint32_t amask = (uint32_t)((int8_t)-0x7F >> (f.alpha_prec - 1)) & 0xFFu;
     const uint32_t a1b = quant_channel((uint32_t)a1 & 0xFFu, amask, -1);
     const uint32_t a2b = quant_channel((uint32_t)a2 & 0xFFu, amask, -1);
-#pragma unroll
+#pragma unroll 1
     for (int i = 0; i < 16; i++) {
-      const uint32_t val = (uint32_t)avals[i];
+      const uint32_t val = chan(px[i], src);
       uint32_t me = 0xFFFFFFFFu;
       float mef = FLT_MAX;
       uint32_t bb = 0;
@@ -1271,16 +1378,31 @@ struct AState {
 // annealed (annealing lowers a fit's error by a few percent at most).
 constexpr unsigned long long kAnnealMarginDiv = 50;
 
+// Word offsets of the counters.  Each that is counted up while others are read
+// has a cache line of its own: an atomic takes some 7 ns of its line, and
+// loads of a line under atomics wait for them (with all of them on two lines,
+// reading the three state counts at every refill took the 508x380 annealing
+// from 2.0 to 3.2 ms, and mode 4's set-up at 4096 x 4096 1.6 to 3.4).
+enum {
+  kCntQueue = 0,         // 8 words: the type queues' sizes
+  kCntFront = 32,        // annealing states of the modes without rotation
+  kCntRot4 = 64,         // and of modes 4
+  kCntRot5 = 96,         // and 5
+  kCntFetch = 128,       // annealing states taken
+  kCntList = 160,        // length of the learned annealing list
+  kCntFallback = 192,    // learned search: blocks for the full search
+  kCntRotFetch = 224,    // learned search: rotation states taken
+  kCntTail = 256,        // candidates handed over
+  kCntTailFetch = 288,   // and taken
+  kCntWords = 320
+};
+
 struct Work {
   uint32_t *sel;          // per block
   uint16_t *cdesc;        // per block x 16 candidate descriptors
   CandRec *rec;           // per block x 16
   uint32_t *queue;        // per-type candidate queues, kMaxPerType entries per block each
-  // [0..7] queue sizes, [8..15] set-up fetch, [16] annealing states of the
-  // modes without rotation, [17] anneal fetch, [18] learned annealing list
-  // size, [20] fallback blocks, [21] anneal fetch of the rotation states, [22]
-  // candidates handed over, [23] their fetch, [24] and [25] annealing states of
-  // modes 4 and 5
+  // see kCnt*
   uint32_t *counters;
   // the annealing states: those of the modes without rotation from the front,
   // the rotation modes' at the back (state_map)
@@ -1288,7 +1410,7 @@ struct Work {
   uint32_t qcap;          // entries per type queue
   uint32_t astate_cap;
   // learned search: the annealing states to run (slots of astate, in
-  // order), counters[18] of them; null in the reference search
+  // order), kCntList of them; null in the reference search
   const uint32_t *alist;
   // learned search: astate[i].id for every state (read when the list is
   // built, without touching the 64-byte states); null in the reference search
@@ -1298,14 +1420,12 @@ struct Work {
   double *nu_total;
 };
 
-// Annealing state i of the counters[16], [24] and [25]: its slot of astate.
+// Annealing state i of the kCntFront, kCntRot4 and kCntRot5: its slot of astate.
 // The rotation modes come last, mode 5 after mode 4: the longer a mode's
 // chains, the earlier annealing starts on them (it runs from the end).  The
 // three regions cannot meet: mode 4's lies below room for every candidate of
 // mode 5, and a job's candidates all fit.
-// (Read once per kernel: the counters share a cache line with the annealing's
-// fetch counters, and loads of it between their atomics took the 508x380
-// annealing from 2.0 to 3.2 ms.)
+// (Read once per kernel.)
 struct StateMap {
   uint32_t front, c4, c5, base4, base5;
   __device__ __forceinline__ uint32_t count() const { return front + c4 + c5; }
@@ -1318,10 +1438,10 @@ struct StateMap {
 __device__ __forceinline__ StateMap state_map(const Work &w) {
   const volatile uint32_t *c = w.counters;
   StateMap m;
-  m.front = c[16];
-  m.c4 = c[24];
-  m.c5 = c[25];
-  m.base4 = w.astate_cap - c[7] - m.c4;  // below room for mode 5's whole queue
+  m.front = c[kCntFront];
+  m.c4 = c[kCntRot4];
+  m.c5 = c[kCntRot5];
+  m.base4 = w.astate_cap - c[kCntQueue + 7] - m.c4;  // below room for mode 5's whole queue
   m.base5 = w.astate_cap - m.c5;
   return m;
 }
@@ -1390,7 +1510,7 @@ __global__ void __launch_bounds__(256) list_count_kernel(Work w, const unsigned 
 }
 
 // One workgroup: exclusive scan of the chunk counts (at most 64 per thread),
-// the list length into counters[18].
+// the list length into kCntList.
 __global__ void __launch_bounds__(256) list_scan_kernel(Work w, uint32_t *chunk_count) {
   __shared__ uint32_t s_wave[4];
   const uint32_t nchunks = (state_map(w).count() + kListChunk - 1) / kListChunk;
@@ -1405,7 +1525,7 @@ __global__ void __launch_bounds__(256) list_scan_kernel(Work w, uint32_t *chunk_
     chunk_count[c] = excl;
     excl += v;
   }
-  if (threadIdx.x == 0) w.counters[18] = all;
+  if (threadIdx.x == 0) w.counters[kCntList] = all;
 }
 
 __global__ void __launch_bounds__(256) list_write_kernel(Work w, const unsigned long long *cerr,
@@ -1475,178 +1595,9 @@ __device__ __forceinline__ void wg_enqueue(Work &w, bool valid, int type, uint32
   uint32_t local = 0;
   if (valid) local = atomicAdd(&s_cnt[type], 1u);
   __syncthreads();
-  if (t < kNumTypes && s_cnt[t]) s_base[t] = atomicAdd(&w.counters[t], s_cnt[t]);
+  if (t < kNumTypes && s_cnt[t]) s_base[t] = atomicAdd(&w.counters[kCntQueue + t], s_cnt[t]);
   __syncthreads();
   if (valid) w.queue[(size_t)type * w.qcap + s_base[type] + local] = id;
-}
-
-// Weight of the second endpoint at index j for nb = 4, 8, 16 entries:
-// (64 j + (nb - 1) / 2) / (nb - 1) by a multiply-shift, equal to
-// kInterpolationValues (Compressor.cpp:159-168); bc7_upload_tables checks
-// every entry on the host before the kernels run.  weight_word holds the
-// weight in its high half, where the packed multiply of interp_err reads it
-// without a shift.
-struct WeightFn {
-  uint32_t m, b;
-};
-__host__ __device__ __forceinline__ WeightFn weight_fn(int nb) {
-  if (nb == 4) return {64u * 21846u, 21846u};
-  if (nb == 8) return {64u * 9363u, 3u * 9363u};
-  return {64u * 4370u, 7u * 4370u};
-}
-__host__ __device__ __forceinline__ uint32_t weight_word(WeightFn fn, uint32_t j) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  // both factors are below 2^24: the full-rate 24-bit multiply-add, which
-  // the compiler only finds where it can see the factors' ranges
-  uint32_t w;
-  asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(w) : "v"(j), "v"(fn.m), "v"(fn.b));
-  return w;
-#else
-  return fn.m * j + fn.b;
-#endif
-}
-__host__ __device__ __forceinline__ uint32_t weight_of(WeightFn fn, uint32_t j) {
-  return weight_word(fn, j) >> 16;
-}
-
-// A texel as the pixel pass reads it: 64 times its channel pairs (each 16-bit
-// lane at most 64 * 255 = 16320).  The interpolated value of an index weight
-// w is (e1 (64 - w) + e2 w + 32) >> 6 = (64 e1 + 32 + (e2 - e1) w) >> 6, so
-// with the texel scaled by 64 its difference to the texel is one shift of
-// one sum, and the texel's projection is 64 times the integer one.
-__device__ __forceinline__ uint32_t pair02x64(uint32_t pix) { return (pix & 0x00FF00FFu) << 6; }
-__device__ __forceinline__ uint32_t pair13x64(uint32_t pix) {
-  return ((pix >> 8) & 0x00FF00FFu) << 6;
-}
-
-// a . b + c in the three-operand form of the instruction: asked to saturate
-// (every sum here is far from the 32-bit range) the compiler cannot take the
-// accumulating two-operand form, which needs its start value moved into place
-// first (three moves per pixel in the pixel pass).
-__device__ __forceinline__ int dot2(s16x2 a, s16x2 b, int c) {
-  return __builtin_amdgcn_sdot2(a, b, c, true);
-}
-
-// Per-subset constants of one annealing step.
-struct SubConst {
-  uint32_t a02, a13;  // 64 * endpoint 1 + 32, channel pairs
-  uint32_t d02, d13;  // endpoint 2 - endpoint 1 (signed pairs)
-  uint32_t q02, q13;  // the projection axis (d, or d seen through a rotation)
-  int ad;             // -64 * endpoint 1 . (endpoint 2 - endpoint 1)
-  float rl;           // 1 / (64 l), l the squared endpoint distance (see pixel_bounds)
-};
-
-__device__ __forceinline__ SubConst sub_const(uint32_t e1, uint32_t e2) {
-  SubConst c;
-  const uint32_t a02 = e1 & 0x00FF00FFu, a13 = (e1 >> 8) & 0x00FF00FFu;
-  const uint32_t b02 = e2 & 0x00FF00FFu, b13 = (e2 >> 8) & 0x00FF00FFu;
-  c.d02 = __builtin_bit_cast(uint32_t, as_s16x2(b02) - as_s16x2(a02));
-  c.d13 = __builtin_bit_cast(uint32_t, as_s16x2(b13) - as_s16x2(a13));
-  c.q02 = c.d02;
-  c.q13 = c.d13;
-  // each 16-bit lane: 64 a + 32 <= 16352
-  c.a02 = (a02 << 6) + 0x00200020u;
-  c.a13 = (a13 << 6) + 0x00200020u;
-  // endpoint 1's projection on the axis, subtracted from each pixel's
-  c.ad = -64 * dot2(as_s16x2(a02), as_s16x2(c.d02), dot2(as_s16x2(a13), as_s16x2(c.d13), 0));
-  const int l = dot2(as_s16x2(c.d02), as_s16x2(c.d02), dot2(as_s16x2(c.d13), as_s16x2(c.d13), 0));
-  // equal endpoints give d = 0 for every pixel, so l = 1 yields index 0
-  const float lf = (float)(l > 0 ? l : 1);
-  // v_rcp_f32 is within 1 ulp; one Newton step makes it the correctly
-  // rounded 1 / l for every l <= 4 * 255^2 (checked for starts within 2 ulp)
-  const float r = __builtin_amdgcn_rcpf(lf);
-  c.rl = __builtin_fmaf(__builtin_fmaf(-lf, r, 1.0f), r, r) * 0x1p-6f;
-  return c;
-}
-
-// The projection axis of a rotation mode (ptmode = rotation + 1).  Its
-// points are the texels with channel r - 1 replaced by alpha (r > 0) and
-// alpha 255 (point_of), so a point's projection is the texel's on a permuted
-// axis (alpha taking channel r - 1's component, that channel none) plus
-// 255 times the axis' alpha component.  sel02 / sel13: v_perm_b32 selectors
-// over (d02, d13), identity without a rotation.
-__device__ __forceinline__ void rotation_selectors(int ptmode, uint32_t &sel02, uint32_t &sel13) {
-  // bytes 0-3 of the selector index d13, 4-7 d02, 0x0c a zero byte
-  sel02 = 0x07060504u;
-  sel13 = 0x03020100u;
-  if (ptmode == 1) sel13 = 0x0c0c0100u;
-  if (ptmode == 2) {
-    sel02 = 0x07060c0cu;
-    sel13 = 0x05040100u;
-  }
-  if (ptmode == 3) sel13 = 0x01000c0cu;
-  if (ptmode == 4) {
-    sel02 = 0x0c0c0504u;
-    sel13 = 0x07060100u;
-  }
-}
-__device__ __forceinline__ void rotate_axis(SubConst &c, int ptmode, uint32_t sel02,
-                                            uint32_t sel13) {
-  c.q02 = __builtin_amdgcn_perm(c.d02, c.d13, sel02);
-  c.q13 = __builtin_amdgcn_perm(c.d02, c.d13, sel13);
-  const int da = (int)c.d13 >> 16;
-  c.ad += ptmode ? 64 * 255 * da : 0;
-}
-
-// Difference of the pixel pairs (64 p) to the interpolant of index weight
-// word ww, (64 e1 + 32 - 64 p + (e2 - e1) w) >> 6 = interpolant - p: z holds
-// 64 e1 + 32 - 64 p, and the sum lies within +-16352, so signed 16-bit lanes
-// hold it exactly.
-__device__ __forceinline__ s16x2 interp_diff(s16x2 z, uint32_t d, uint32_t ww) {
-  const s16x2 w = as_s16x2(ww);
-  const s16x2 W = {w.y, w.y};
-  const s16x2 S = {6, 6};
-  return (as_s16x2(d) * W + z) >> S;
-}
-
-// QuantizedError's neighbouring indices (RGBAEndpoints.cpp:240-300) of a
-// pixel: j1 = floor(t), j2 = ceil(t), both clamped to the index range, of the
-// reference's t = fl(fl(d / l) * kf) (float, d the integer projection, l the
-// integer squared distance, kf = nb - 1).  Those equal the floor and ceiling
-// of the rational d kf / l: its distance to an integer, when nonzero, is at
-// least 1 / l >= 1 / (4 * 255^2) = 3.8e-6, more than the float error of at
-// most 2^-23 |t| <= 1.9e-6 for |t| <= 16 (larger |t| is clamped away), and
-// fl(fl(k / kf) kf) = k for every integer 0 <= k <= kf in {3, 7, 15} (checked
-// exhaustively).
-//
-// Here u = fl(64 d * rl) clamped to [0, 1] (64 d is below 2^24, so its
-// conversion is exact; a d below 0 or above l clamps to the end index), and
-// the floor and ceiling are truncations of fma(u, kf, 1.9e-6) and
-// fma(u, kf, 1 - 1.9e-6).  Exact for every l up to 4 * 255^2, d in 0..l and
-// kf: checked exhaustively at the steps of both functions of d, which are
-// monotone.  The pass is bound by VALU issue: an integer quotient corrected
-// with the exact remainder took 17 instructions per pixel where this takes 9;
-// with the texels kept as scaled pairs (no unpacking, one subtraction per
-// pair) and the rotation folded into the axis (no separate point) the pass
-// went from about 54 instructions per pixel to 33, and the 4096 x 4096
-// annealing from 46.0 to 34.3 ms (reference search) and 5.2 to 4.1 ms
-// (learned).
-constexpr float kIndexSlack = 1.9e-6f;
-
-__device__ __forceinline__ void pixel_bounds(uint32_t p02, uint32_t p13, const SubConst &c,
-                                             float kf, uint32_t &j1, uint32_t &j2) {
-  const int d = dot2(as_s16x2(p02), as_s16x2(c.q02), dot2(as_s16x2(p13), as_s16x2(c.q13), c.ad));
-  const float u = __builtin_amdgcn_fmed3f((float)d * c.rl, 0.0f, 1.0f);
-  j1 = (uint32_t)__builtin_fmaf(u, kf, kIndexSlack);
-  j2 = (uint32_t)__builtin_fmaf(u, kf, 1.0f - kIndexSlack);
-}
-
-// The per-pixel index search without branches: both neighbouring indices
-// are scored and the second kept only when strictly better (where the two
-// are the same index the errors are equal).  Returns the error, the index in
-// *best.  p02, p13: the texel's pairs times 64.
-__device__ __forceinline__ uint32_t pixel_err(uint32_t p02, uint32_t p13, const SubConst &c,
-                                              float kf, WeightFn wf, uint32_t *best) {
-  uint32_t j1, j2;
-  pixel_bounds(p02, p13, c, kf, j1, j2);
-  const s16x2 z02 = as_s16x2(c.a02) - as_s16x2(p02), z13 = as_s16x2(c.a13) - as_s16x2(p13);
-  const uint32_t w1 = weight_word(wf, j1), w2 = weight_word(wf, j2);
-  const s16x2 x02 = interp_diff(z02, c.d02, w1), x13 = interp_diff(z13, c.d13, w1);
-  const s16x2 y02 = interp_diff(z02, c.d02, w2), y13 = interp_diff(z13, c.d13, w2);
-  const uint32_t e1 = (uint32_t)dot2(x02, x02, dot2(x13, x13, 0));
-  const uint32_t e2 = (uint32_t)dot2(y02, y02, dot2(y13, y13, 0));
-  *best = e2 < e1 ? j2 : j1;
-  return e2 < e1 ? e2 : e1;
 }
 
 // The nonuniform metric's pixel pass (the metric is described above qerr_nu):
@@ -2594,7 +2545,8 @@ __device__ __forceinline__ uint32_t fit_candidate(const Cand &k, const uint32_t 
     Weights mr;
     double aerr_nu = 0.0;
     if constexpr (NU) mr = rotate_weights(*mu, rot);
-    const uint32_t aerr = alpha_fit<NU>(f, px, aidx, a1q, a2q, NU ? mr.w[3] : 1.0f, &aerr_nu);
+    const uint32_t aerr = alpha_fit<NU>(f, px, aidx, a1q, a2q, km, NU ? mr.w[3] : 1.0f,
+                                        &aerr_nu);
     // the RGB fit sees the stale statistics of the unrotated cluster
     float avg[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -2684,26 +2636,26 @@ constexpr int kSetupBuckets(int mode) {
   return mode == 6 ? 16 : ((mode == 0 || mode == 1 || mode == 4) ? 8 : 4);
 }
 
-// One wave takes batches of candidates of the mode's queue until it is used
-// up: one lane each, or with several subsets one adjacent lane per subset (64
+// Runs the batches of the mode's queue from `first` on, `stride` apart: one
+// lane each, or with several subsets one adjacent lane per subset (64
 // candidates, or 32 or 21), whose fits run side by side.  (One lane for all
 // subsets took their fits' time one after another: 155 us for a batch of
-// mode 0.)  s_px: the lanes' texels; s_km: the k-means sums and counts, per
+// mode 0.)  The batches cost alike, so the waves stride over them: fetching
+// them from a counter cost small jobs an atomic per wave and mode, 2048 waves'
+// 16 thousand of them on one cache line.  s_px: the lanes' texels; s_km: the k-means sums and counts, per
 // bucket a row of 64 lanes each.
 template <int MODE, bool NU>
 __device__ __forceinline__ void setup_run(const BlockRange &r, const Bc7Params &prm,
                                           const Work &w, const uint32_t *sctab, uint32_t *s_px,
-                                          uint32_t *s_km) {
+                                          uint32_t *s_km, uint32_t first, uint32_t stride) {
   constexpr int kTypeOf[8] = {0, 2, 1, 3, 6, 7, 5, 4};
   constexpr int t = kTypeOf[MODE], kSub = kModeTab[MODE].subsets, kBatch = 64 / kSub;
   const int lane = threadIdx.x, sub = lane % kSub, lead = lane - sub;
-  const uint32_t count = *(volatile uint32_t *)&w.counters[t];
-  for (;;) {
-    uint32_t b0 = 0;
-    if (lane == 0) b0 = atomicAdd(&w.counters[8 + t], (uint32_t)kBatch);
-    b0 = __shfl(b0, 0);
-    if (b0 >= count) break;
-    const uint32_t item = b0 + (uint32_t)(lane / kSub);
+  const uint32_t count = w.counters[kCntQueue + t];
+  // mode 4's states end below room for mode 5's whole queue
+  const uint32_t top4 = w.astate_cap - 1u - w.counters[kCntQueue + kTypeOf[5]];
+  for (uint32_t batch = first; batch < (count + kBatch - 1) / kBatch; batch += stride) {
+    const uint32_t item = batch * kBatch + (uint32_t)(lane / kSub);
     const bool mine = lane < kBatch * kSub && item < count;
     const uint32_t id = mine ? w.queue[(size_t)t * w.qcap + item] : 0u;
     const uint32_t rel = id_block(id);
@@ -2757,7 +2709,7 @@ __device__ __forceinline__ void setup_run(const BlockRange &r, const Bc7Params &
         if constexpr (NU) tnu += __shfl(terr, from);
       }
       uint32_t slot = 0;
-      if (mine && sub == 0 && active) slot = atomicAdd(&w.counters[16], 1u);
+      if (mine && sub == 0 && active) slot = atomicAdd(&w.counters[kCntFront], 1u);
       slot = (uint32_t)__shfl((int)slot, lead);
       if (mine) {
         out->px1[sub] = e1;
@@ -2815,10 +2767,10 @@ __device__ __forceinline__ void setup_run(const BlockRange &r, const Bc7Params &
                   ((uint32_t)k.nsub << 6) | ((uint32_t)k.shape << 8) | (active << 14) |
                   ((uint32_t)k.entry << 17);
         uint32_t slot;
-        if (MODE == 5) slot = w.astate_cap - 1u - atomicAdd(&w.counters[25], 1u);
+        if (MODE == 5) slot = w.astate_cap - 1u - atomicAdd(&w.counters[kCntRot5], 1u);
         else if (MODE == 4)
-          slot = w.astate_cap - 1u - w.counters[kTypeOf[5]] - atomicAdd(&w.counters[24], 1u);
-        else slot = atomicAdd(&w.counters[16], twin ? 2u : 1u);
+          slot = top4 - atomicAdd(&w.counters[kCntRot4], 1u);
+        else slot = atomicAdd(&w.counters[kCntFront], twin ? 2u : 1u);
         w.astate[slot] = st;
         if (w.aid) w.aid[slot] = id;
         if (twin) {
@@ -2832,41 +2784,51 @@ __device__ __forceinline__ void setup_run(const BlockRange &r, const Bc7Params &
   }
 }
 
-// Three waves per SIMD (168 registers) for every mode but 6, whose 16
-// centroids take 64 registers: mode 4 at two waves took 3.9 ms at 4096 x 4096
-// instead of 2.4.
+// Waves of a mode's set-up that a CU holds: two per SIMD for mode 6, whose 16
+// centroids take 64 registers, four for the modes with 4 buckets and two
+// subsets or more, else three.
+constexpr uint32_t setup_waves(int mode) {
+  return mode == 6 ? 8u : (mode == 2 || mode == 3 || mode == 7 ? 16u : 12u);
+}
+
 template <int MODE, bool NU = false>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MODE == 6 ? 2 : 3)))
-setup_kernel(BlockRange r, Bc7Params prm, Work w,
-                                                   const uint32_t *sctab) {
+__global__ void __launch_bounds__(64)
+    __attribute__((amdgpu_waves_per_eu(setup_waves(MODE) / 4)))
+    setup_kernel(BlockRange r, Bc7Params prm, Work w, const uint32_t *sctab) {
   __shared__ uint32_t s_px[64 * kPxStride];
   __shared__ uint32_t s_km[kSetupBuckets(MODE) * 3 * 64];
-  setup_run<MODE, NU>(r, prm, w, sctab, s_px, s_km);
+  setup_run<MODE, NU>(r, prm, w, sctab, s_px, s_km, blockIdx.x, gridDim.x);
 }
 
 // Every mode in one launch, for jobs that leave the chip idle: a batch of fits
 // takes 50 to 170 us whatever the job's size (one lane's serial fit), so
 // eight launches in a row add up where one lets the modes run side by side.
-// Consecutive workgroups start on different modes; the annealing states come
-// out in no order but the rotation modes' place.
+// The annealing states come out in no order but the rotation modes' place.
 template <bool NU>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
 setup_all_kernel(BlockRange r, Bc7Params prm, Work w,
                                                        const uint32_t *sctab) {
   __shared__ uint32_t s_px[64 * kPxStride];
   __shared__ uint32_t s_km[kSetupBuckets(6) * 3 * 64];
-  for (uint32_t k = 0; k < 8; k++) {
-    switch ((blockIdx.x + k) & 7u) {
-      case 0: setup_run<4, NU>(r, prm, w, sctab, s_px, s_km); break;
-      case 1: setup_run<0, NU>(r, prm, w, sctab, s_px, s_km); break;
-      case 2: setup_run<2, NU>(r, prm, w, sctab, s_px, s_km); break;
-      case 3: setup_run<1, NU>(r, prm, w, sctab, s_px, s_km); break;
-      case 4: setup_run<3, NU>(r, prm, w, sctab, s_px, s_km); break;
-      case 5: setup_run<7, NU>(r, prm, w, sctab, s_px, s_km); break;
-      case 6: setup_run<6, NU>(r, prm, w, sctab, s_px, s_km); break;
-      default: setup_run<5, NU>(r, prm, w, sctab, s_px, s_km); break;
-    }
-  }
+  // this wave's batches of the modes' batches one after another, the slowest
+  // modes' first: each mode's starting where the last one's end left off
+  uint32_t first = blockIdx.x;
+  auto run = [&](auto mode) {
+    constexpr int M = decltype(mode)::value;
+    constexpr int kTypeOf[8] = {0, 2, 1, 3, 6, 7, 5, 4};
+    constexpr uint32_t kBatch = 64 / kModeTab[M].subsets;
+    setup_run<M, NU>(r, prm, w, sctab, s_px, s_km, first, gridDim.x);
+    const uint32_t n = (w.counters[kCntQueue + kTypeOf[M]] + kBatch - 1) / kBatch % gridDim.x;
+    first = first >= n ? first - n : first + gridDim.x - n;
+  };
+  run(std::integral_constant<int, 4>{});
+  run(std::integral_constant<int, 5>{});
+  run(std::integral_constant<int, 1>{});
+  run(std::integral_constant<int, 0>{});
+  run(std::integral_constant<int, 6>{});
+  run(std::integral_constant<int, 2>{});
+  run(std::integral_constant<int, 3>{});
+  run(std::integral_constant<int, 7>{});
 }
 
 // ---------------------------------------------------------------------------
@@ -3487,7 +3449,7 @@ __device__ __forceinline__ void spread_run(const BlockRange &r, const Bc7Params 
     if (!hasm) break;
     if (SRC == kFromListHand && exhausted && __popcll(hasm) <= kHandGroups) {
       uint32_t base = 0;
-      if (lane == 0) base = atomicAdd(&w.counters[22], (uint32_t)__popcll(hasm));
+      if (lane == 0) base = atomicAdd(&w.counters[kCntTail], (uint32_t)__popcll(hasm));
       base = __shfl(base, 0);
       if (has) {
         TailState &o = tail[base + (uint32_t)__popcll(hasm & ((1ull << lead) - 1ull))];
@@ -3705,7 +3667,7 @@ __device__ __forceinline__ void add_counts(const Bc7Params &prm, unsigned long l
   }
 }
 
-// TAIL: the candidates the one-lane form handed over (counters[22] of them);
+// TAIL: the candidates the one-lane form handed over (kCntTail of them);
 // otherwise the whole annealing list.
 template <bool TAIL, bool COUNT>
 __global__ void __launch_bounds__(256) anneal_spread_kernel(BlockRange r, Bc7Params prm, Work w,
@@ -3713,12 +3675,12 @@ __global__ void __launch_bounds__(256) anneal_spread_kernel(BlockRange r, Bc7Par
   __shared__ __align__(4) uint8_t s_quant[kStepQuantBytes];
   step_quant_load(s_quant);
   __syncthreads();
-  const uint32_t total = TAIL      ? *(volatile uint32_t *)&w.counters[22]
-                         : w.alist ? *(volatile uint32_t *)&w.counters[18]
+  const uint32_t total = TAIL      ? *(volatile uint32_t *)&w.counters[kCntTail]
+                         : w.alist ? *(volatile uint32_t *)&w.counters[kCntList]
                                    : state_map(w).count();
   unsigned long long n_ref = 0, n_gpu = 0;
   spread_run<16, TAIL ? kFromTail : kFromList, COUNT>(r, prm, w, tail, s_quant, 0, total,
-                                                      4 * gridDim.x, &w.counters[TAIL ? 23 : 17],
+                                                      4 * gridDim.x, &w.counters[TAIL ? kCntTailFetch : kCntFetch],
                                                       n_ref, n_gpu);
   if constexpr (COUNT) add_counts(prm, n_ref, n_gpu);
 }
@@ -3743,7 +3705,7 @@ anneal_kernel(BlockRange r, Bc7Params prm, Work w, uint32_t unroll, uint32_t tai
   unsigned long long n_ref = 0, n_gpu = 0;  // COUNT
   const uint64_t lt = (1ull << lane) - 1ull;
   const StateMap sm = state_map(w);
-  uint32_t total = w.alist ? *(volatile uint32_t *)&w.counters[18] : sm.count();
+  uint32_t total = w.alist ? *(volatile uint32_t *)&w.counters[kCntList] : sm.count();
   // odd row stride: conflict-free
   __shared__ uint32_t s_px[256 * kRowWords];
   __shared__ __align__(4) uint8_t s_quant[kStepQuantBytes];
@@ -3766,7 +3728,7 @@ anneal_kernel(BlockRange r, Bc7Params prm, Work w, uint32_t unroll, uint32_t tai
     }
     if (blockIdx.x < rot_groups)
       spread_run<4, kFromListHand, COUNT>(r, prm, w, tail, s_quant, lo, total, 4 * rot_groups,
-                                          &w.counters[21], n_ref, n_gpu);
+                                          &w.counters[kCntRotFetch], n_ref, n_gpu);
     total = lo;
   }
   Lane L = {};  // lanes without a candidate step along on zeros
@@ -3788,7 +3750,7 @@ anneal_kernel(BlockRange r, Bc7Params prm, Work w, uint32_t unroll, uint32_t tai
         if (!need || exhausted) break;
         if (wbase >= wend) {
           uint32_t b0 = 0;
-          if (lane == 0) b0 = atomicAdd(&w.counters[17], 64u);
+          if (lane == 0) b0 = atomicAdd(&w.counters[kCntFetch], 64u);
           b0 = __shfl(b0, 0);
           if (b0 >= total) {
             exhausted = true;
@@ -3819,7 +3781,7 @@ anneal_kernel(BlockRange r, Bc7Params prm, Work w, uint32_t unroll, uint32_t tai
       }
       const uint64_t left = __ballot(L.has);
       uint32_t base = 0;
-      if (lane == 0) base = atomicAdd(&w.counters[22], (uint32_t)__popcll(left));
+      if (lane == 0) base = atomicAdd(&w.counters[kCntTail], (uint32_t)__popcll(left));
       base = __shfl(base, 0);
       if (L.has) lane_hand_over(L, tail[base + (uint32_t)__popcll(left & lt)]);
       break;
@@ -4080,12 +4042,12 @@ __global__ void __launch_bounds__(256) guard_kernel(BlockRange r, const uint4 *q
 // the three its natural allocation allows.
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
 cand_error_kernel(BlockRange r, Work w, unsigned long long *cerr, int final_pass) {
-  uint32_t total = 0;
+  uint32_t total = 0, sizes[kNumTypes];
   if (final_pass) {
-    total = w.counters[18];
+    total = w.counters[kCntList];
   } else {
 #pragma unroll
-    for (int q = 0; q < kNumTypes; q++) total += w.counters[q];
+    for (int q = 0; q < kNumTypes; q++) total += sizes[q] = w.counters[kCntQueue + q];
   }
   const uint32_t stride = gridDim.x * blockDim.x;
   for (uint32_t t = blockIdx.x * blockDim.x + threadIdx.x; t < total; t += stride) {
@@ -4097,7 +4059,7 @@ cand_error_kernel(BlockRange r, Work w, unsigned long long *cerr, int final_pass
       int type = kNumTypes - 1;
 #pragma unroll
       for (int q = 0; q < kNumTypes; q++) {
-        const uint32_t c = w.counters[q];
+        const uint32_t c = sizes[q];
         if (t >= base && t < base + c) {
           type = q;
           item = t - base;
@@ -4450,10 +4412,11 @@ constexpr uint32_t kRotShare = 10;
 // 1024x1024: 4 0.87, 3 0.83, 2 0.85).
 constexpr uint32_t kSpreadWgPerCu = 3;
 
-// Blocks up to which every mode's set-up runs in one launch (64x64: 0.89 ms of
-// eight launches, 0.17 of one; 508x380 1.07 and 0.72; learned 1024x1024 0.95
-// and 0.80, 2048x2048 1.35 and 1.26, but the merged launch mixes the modes in
-// the annealing list, which costs the one-lane form as much again).
+// Blocks up to which every mode's set-up runs in one launch (64x64: 0.13 ms
+// against 0.89 for eight launches one after another; 508x380 0.17, learned
+// 1024x1024 0.24).  Larger jobs fill the chip mode by mode, and a merged
+// launch would mix the modes in the annealing list, whose one-lane form wants
+// them in order.
 constexpr uint32_t kSetupAllBlocks = kSpreadBlocks, kSetupAllBlocksLearned = kSpreadBlocksLearned;
 
 // waves: persistent waves of the one-lane form.  tail: memory for tail_cap
@@ -4535,7 +4498,7 @@ hipError_t bc7_scatter(const SurfDesc *surfs, const uint32_t *block_surf, uint32
 size_t bc7_work_bytes(uint32_t num_blocks, bool learned, bool nonuniform) {
   const size_t n = num_blocks;
   // counters, sel, cdesc, rec, queues, astate, q0, alignment slack
-  size_t bytes = 64 * 4 + n * 4 + n * bc7::kMaxCands * 2 +
+  size_t bytes = bc7::kCntWords * 4 + n * 4 + n * bc7::kMaxCands * 2 +
                  n * bc7::kMaxCands * sizeof(bc7::CandRec) +
                  n * bc7::kNumTypes * bc7::kMaxPerType * 4 +
                  n * bc7::kMaxCands * sizeof(bc7::AState) + n * 16 + 8 * 256;
@@ -4568,7 +4531,7 @@ hipError_t bc7_encode(const BlockRange &r, const Bc7Params &p, const Bc7Scratch 
   };
   bc7::Work w;
   const size_t nc = (size_t)n * bc7::kMaxCands;
-  w.counters = reinterpret_cast<uint32_t *>(carve(64 * 4));
+  w.counters = reinterpret_cast<uint32_t *>(carve(bc7::kCntWords * 4));
   w.sel = reinterpret_cast<uint32_t *>(carve((size_t)n * 4));
   w.cdesc = reinterpret_cast<uint16_t *>(carve(nc * 2));
   w.rec = reinterpret_cast<bc7::CandRec *>(carve(nc * sizeof(bc7::CandRec)));
@@ -4597,7 +4560,7 @@ hipError_t bc7_encode(const BlockRange &r, const Bc7Params &p, const Bc7Scratch 
     chunk_count = reinterpret_cast<uint32_t *>(carve((nc / bc7::kListChunk + 1) * 4));
     fallback = reinterpret_cast<uint32_t *>(carve((size_t)n * 4));
   }
-  uint32_t *fallback_count = w.counters + 20;
+  uint32_t *fallback_count = w.counters + bc7::kCntFallback;
   const uint32_t nchunks = (n + 255) / 256;
   const uint32_t ngroups = (n + 15) / 16;
   // persistent workgroups of one wave, no more than the candidates could use
@@ -4614,7 +4577,8 @@ hipError_t bc7_encode(const BlockRange &r, const Bc7Params &p, const Bc7Scratch 
   const size_t tail_cap =
       (size_t)w.qcap * bc7::kNumTypes * sizeof(uint32_t) / sizeof(bc7::TailState);
   int t = timing_begin(stream);
-  hipLaunchKernelGGL(bc7::reset_kernel, dim3(1), dim3(64), 0, stream, w.counters, 64);
+  hipLaunchKernelGGL(bc7::reset_kernel, dim3(1), dim3(bc7::kCntWords), 0, stream, w.counters,
+                     (int)bc7::kCntWords);
   hipLaunchKernelGGL(bc7::solid_scan_kernel, dim3(nchunks), dim3(256), 0, stream, r, s);
   hipLaunchKernelGGL(bc7::chunk_scan_kernel, dim3(1), dim3(1024), 0, stream, s);
   timing_end(t, kTagBc7Scan, stream);
@@ -4655,42 +4619,36 @@ hipError_t bc7_encode(const BlockRange &r, const Bc7Params &p, const Bc7Scratch 
   }
   t = timing_begin(stream);
   if (n <= (learned ? kSetupAllBlocksLearned : kSetupAllBlocks)) {
-    const uint32_t waves = persistent < (uint32_t)g_num_cus[dev] * 8u
-                               ? (persistent + 7u) / 8u * 8u
-                               : (uint32_t)g_num_cus[dev] * 8u;
+    const uint32_t fit = (uint32_t)g_num_cus[dev] * 8u;  // two waves per SIMD
+    const uint32_t waves = persistent < fit ? persistent : fit;
     if (nu)
       hipLaunchKernelGGL(bc7::setup_all_kernel<true>, dim3(waves), dim3(64), 0, stream, r, p, w,
                          sct);
     else
       hipLaunchKernelGGL(bc7::setup_all_kernel<false>, dim3(waves), dim3(64), 0, stream, r, p, w,
                          sct);
-  } else if (nu) {
-    // annealing-state order: modes 0, 2, 3, 7, 6, 1 in front, 5 and 4 behind
-    hipLaunchKernelGGL((bc7::setup_kernel<0, true>), dim3(persistent), dim3(64), 0, stream, r,
-                       p, w, sct);
-    hipLaunchKernelGGL((bc7::setup_kernel<2, true>), dim3(persistent), dim3(64), 0, stream, r,
-                       p, w, sct);
-    hipLaunchKernelGGL((bc7::setup_kernel<3, true>), dim3(persistent), dim3(64), 0, stream, r,
-                       p, w, sct);
-    hipLaunchKernelGGL((bc7::setup_kernel<7, true>), dim3(persistent), dim3(64), 0, stream, r,
-                       p, w, sct);
-    hipLaunchKernelGGL((bc7::setup_kernel<6, true>), dim3(persistent), dim3(64), 0, stream, r,
-                       p, w, sct);
-    hipLaunchKernelGGL((bc7::setup_kernel<1, true>), dim3(persistent), dim3(64), 0, stream, r,
-                       p, w, sct);
-    hipLaunchKernelGGL((bc7::setup_kernel<4, true>), dim3(persistent), dim3(64), 0, stream, r,
-                       p, w, sct);
-    hipLaunchKernelGGL((bc7::setup_kernel<5, true>), dim3(persistent), dim3(64), 0, stream, r,
-                       p, w, sct);
   } else {
-    hipLaunchKernelGGL(bc7::setup_kernel<0>, dim3(persistent), dim3(64), 0, stream, r, p, w, sct);
-    hipLaunchKernelGGL(bc7::setup_kernel<2>, dim3(persistent), dim3(64), 0, stream, r, p, w, sct);
-    hipLaunchKernelGGL(bc7::setup_kernel<3>, dim3(persistent), dim3(64), 0, stream, r, p, w, sct);
-    hipLaunchKernelGGL(bc7::setup_kernel<7>, dim3(persistent), dim3(64), 0, stream, r, p, w, sct);
-    hipLaunchKernelGGL(bc7::setup_kernel<6>, dim3(persistent), dim3(64), 0, stream, r, p, w, sct);
-    hipLaunchKernelGGL(bc7::setup_kernel<1>, dim3(persistent), dim3(64), 0, stream, r, p, w, sct);
-    hipLaunchKernelGGL(bc7::setup_kernel<4>, dim3(persistent), dim3(64), 0, stream, r, p, w, sct);
-    hipLaunchKernelGGL(bc7::setup_kernel<5>, dim3(persistent), dim3(64), 0, stream, r, p, w, sct);
+    // the waves that fit at once (setup_waves), as the batches are dealt out
+    // evenly: 4096 waves over 3072 places took mode 1's 1.17 ms (learned
+    // 4096x4096) to 1.44.  Annealing-state order: modes 0, 2, 3, 7, 6, 1 in
+    // front, 5 and 4 behind.
+    auto run = [&](auto mode) {
+      constexpr int M = decltype(mode)::value;
+      const uint32_t fit = (uint32_t)g_num_cus[dev] * bc7::setup_waves(M);
+      const dim3 grid(persistent < fit ? persistent : fit);
+      if (nu)
+        hipLaunchKernelGGL((bc7::setup_kernel<M, true>), grid, dim3(64), 0, stream, r, p, w, sct);
+      else
+        hipLaunchKernelGGL((bc7::setup_kernel<M, false>), grid, dim3(64), 0, stream, r, p, w, sct);
+    };
+    run(std::integral_constant<int, 0>{});
+    run(std::integral_constant<int, 2>{});
+    run(std::integral_constant<int, 3>{});
+    run(std::integral_constant<int, 7>{});
+    run(std::integral_constant<int, 6>{});
+    run(std::integral_constant<int, 1>{});
+    run(std::integral_constant<int, 4>{});
+    run(std::integral_constant<int, 5>{});
   }
   timing_end(t, kTagBc7Setup, stream);
   if (learned) {
