@@ -13,14 +13,17 @@
 //           picks the shapes.  Each block's candidates (one per mode and shape
 //           entry of CompressClusters, :1752-1817, with the rotation modes split
 //           per rotation and index mode) are appended to per-mode queues.
-//   setup   persistent, one lane per candidate, queue by queue, so a wave runs
-//           one mode: principal axis, k-means, least squares and grid clamp for
-//           every subset (CompressCluster, :921-1094), and the alpha fit of the
-//           rotation modes (:632-919).
-//   anneal  persistent, one lane per candidate: each iteration advances every
-//           still-annealing subset of the candidate by one step and scores all
-//           16 pixels in one pass, each against its subset's endpoints.  Lanes
-//           that finish refill from a wave-local window of the work list.
+//   setup   persistent, one lane per subset of a candidate, queue by queue, so a
+//           wave runs one mode: principal axis, k-means, least squares and grid
+//           clamp (CompressCluster, :921-1094), and the alpha fit of the rotation
+//           modes (:632-919).  Small jobs run every mode in one launch.
+//   anneal  each step advances every still-annealing subset of a candidate and
+//           scores all 16 pixels in one pass, each against its subset's endpoints.
+//           Large lists run one lane per candidate, lanes that finish refilling
+//           from the work list, and hand the last few candidates of each wave
+//           over; those, and small lists from the start, run one lane per pixel,
+//           16 lanes a candidate, where few candidates are left looking several
+//           steps ahead.
 //   pack    one lane per block: sum the subset errors per mode in the
 //           reference's mode order, keep the first strict minimum and write the
 //           128-bit block (CompressionMode::Pack, :1096-1298); solid blocks get
@@ -3997,17 +4000,22 @@ __global__ void __launch_bounds__(256) pack_kernel(BlockRange r, Bc7Scratch scr,
 // quality-0 block, the quality-0 block is written instead.  The error is
 // sum((a*c - a'*c')^2) over pixels and RGB, Image::ComputePSNR's per-pixel
 // term (Base/src/Image.cpp:205-255) scaled by 255^2 to stay an exact integer.
+// |d| <= 255^2, so a square is below 2^32; the three together need more.
+__device__ __forceinline__ uint64_t premul_pixel(uint32_t src, uint32_t dec) {
+  const uint32_t a = src >> 24, b = dec >> 24;
+  uint64_t e = 0;
+#pragma unroll
+  for (int c = 0; c < 3; c++) {
+    const int d = (int)__umul24(a, chan(src, c)) - (int)__umul24(b, chan(dec, c));
+    const uint32_t m = (uint32_t)(d < 0 ? -d : d);
+    e += m * m;
+  }
+  return e;
+}
 __device__ __forceinline__ uint64_t premul_err(const uint32_t src[16], const uint32_t dec[16]) {
   uint64_t e = 0;
 #pragma unroll
-  for (int i = 0; i < 16; i++) {
-    const int a = (int)(src[i] >> 24), b = (int)(dec[i] >> 24);
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-      const int d = a * (int)chan(src[i], c) - b * (int)chan(dec[i], c);
-      e += (uint64_t)((int64_t)d * d);
-    }
-  }
+  for (int i = 0; i < 16; i++) e += premul_pixel(src[i], dec[i]);
   return e;
 }
 
@@ -4018,11 +4026,14 @@ __global__ void __launch_bounds__(256) guard_kernel(BlockRange r, const uint4 *q
   uint4 *out = reinterpret_cast<uint4 *>(r.out);
   const uint4 a = out[b], z = q0[rel];
   if (a.x == z.x && a.y == z.y && a.z == z.z && a.w == z.w) return;
-  uint32_t px[16], da[16], dz[16];
+  uint32_t px[16];
   load_block(r, rel, px);
-  bc7dec::decode_block(a, da);
-  bc7dec::decode_block(z, dz);
-  if (premul_err(px, dz) < premul_err(px, da)) out[b] = z;
+  uint64_t ea = 0, ez = 0;
+  bc7dec::decode_pixels<false>(
+      a, [&](int i, uint32_t pixel) { ea += premul_pixel(px[i], pixel); });
+  bc7dec::decode_pixels<false>(
+      z, [&](int i, uint32_t pixel) { ez += premul_pixel(px[i], pixel); });
+  if (ez < ea) out[b] = z;
 }
 
 // The learned search chooses among a block's candidates by decoded error:
@@ -4038,8 +4049,7 @@ __global__ void __launch_bounds__(256) guard_kernel(BlockRange r, const uint4 *q
 // entry, whose set-up copied the first's record; the final pass walks the
 // annealing list and re-scores only the records annealing rewrote.
 // Grid-stride: the item counts are device counters.  Four waves per SIMD
-// (128 VGPRs, no spills) hide the dependent loads of each item better than
-// the three its natural allocation allows.
+// (101 VGPRs, no spills) hide the dependent loads of each item.
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
 cand_error_kernel(BlockRange r, Work w, unsigned long long *cerr, int final_pass) {
   uint32_t total = 0, sizes[kNumTypes];
@@ -4077,10 +4087,11 @@ cand_error_kernel(BlockRange r, Work w, unsigned long long *cerr, int final_pass
     pack_mode(k.mode, k.shape, rc, bw);
     const uint4 blk = make_uint4((uint32_t)bw.lo, (uint32_t)(bw.lo >> 32), (uint32_t)bw.hi,
                                  (uint32_t)(bw.hi >> 32));
-    uint32_t px[16], dec[16];
+    uint32_t px[16];
     load_block(r, rel, px);
-    bc7dec::decode_block(blk, dec);
-    const unsigned long long e = premul_err(px, dec);
+    unsigned long long e = 0;
+    bc7dec::decode_pixels<false>(
+        blk, [&](int i, uint32_t pixel) { e += premul_pixel(px[i], pixel); });
     cerr[id] = e;
     if (!final_pass && k.mode == 6) {
       const uint32_t c = id_slot(id);

@@ -36,7 +36,7 @@ struct Bc7Params {
   uint32_t topk;         // candidates searched per confident block (1..8)
   float threshold;       // below this top softmax probability: BoxSelection
   uint32_t wg_per_cu;    // persistent workgroups per CU (0 = 16)
-  uint32_t anneal_unroll;  // annealing steps between refills (0 = 1)
+  uint32_t anneal_unroll;  // annealing steps between refills, one-lane form (0 = 1)
   // CompressWithStats' block path: one record per block of the range (null =
   // Compress's BoxSelection search); not combined with the ranker
   fh_bc7_block_stats *stats;

@@ -452,7 +452,8 @@ fh_status fh_kernel_time(const char *kernel, double *total_ms, uint32_t *launche
  * QuantizedError point evaluations the reference's annealing makes for the
  * same encode (every step of a subset scores that subset's points,
  * Compressor.cpp:583-624), counts[1] the pixel scores the GPU's annealing
- * makes (16 per step of a candidate).  fh_bc7_work_counts waits for the
+ * makes (16 per step of a candidate, and per step looked ahead at that the
+ * chain then did not take).  fh_bc7_work_counts waits for the
  * device and returns the counters of the calling thread's current device. */
 fh_status fh_set_work_counting(int enable);
 fh_status fh_bc7_work_counts(uint64_t counts[2]);

@@ -70,6 +70,37 @@ def test_decode_device_unaligned_and_odd_width(fh, oracle, name):
     assert np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("w,skip", [(64, 0), (64, 2), (66, 0), (66, 1), (66, 2), (67, 0)])
+@pytest.mark.parametrize("mode", range(8))
+def test_bc7_decode_one_mode_by_row_access(fh, oracle, mode, w, skip):
+    """Blocks of one BC7 mode (whole waves with one, two or three subsets) at
+    every width of row access: by four pixels, by two and by one, the output
+    `skip` pixels past a 16-byte boundary.  Integers: exact."""
+    h = 18
+    data = random_blocks("bptc", w, h, 100 + mode).reshape(-1, 16)
+    data[:, 0] = (data[:, 0] & (0xFF << (mode + 1) & 0xFF)) | (1 << mode)
+    data = np.ascontiguousarray(data.reshape(-1))
+    want = oracle_decode(oracle, 3, data, w, h)
+    d_in = torch.from_numpy(data).cuda()
+    out = torch.zeros(w * h + skip, dtype=torch.int32, device="cuda")
+    fh.decompress_device(d_in.data_ptr(), out.data_ptr() + 4 * skip, w, h, fmt=3)
+    torch.cuda.synchronize()
+    got = out[skip:].cpu().numpy().view(np.uint32).reshape(h, w)
+    assert np.array_equal(got, want)
+    orig = np.random.default_rng(mode).integers(0, 2**32, (h, w), dtype=np.uint32)
+    pad = np.concatenate([np.zeros(skip, np.uint32), orig.reshape(-1)]).view(np.int32)
+    d_orig = torch.from_numpy(pad).cuda()
+    want_blocks, want_total = oracle.block_errors(orig, want)
+    blocks = torch.zeros(want_blocks.size, dtype=torch.int64, device="cuda")
+    sse = torch.zeros(2, dtype=torch.int64, device="cuda")
+    fh.block_error_device(d_orig.data_ptr() + 4 * skip, d_in.data_ptr(), w, h, sse.data_ptr(),
+                          blocks.data_ptr(), fmt=3)
+    torch.cuda.synchronize()
+    assert np.array_equal(blocks.cpu().numpy().view(np.uint64), want_blocks)
+    s = sse.cpu().numpy().view(np.uint64)
+    assert int(s[0]) + (int(s[1]) << 64) == want_total
+
+
 def _errors(fh, orig, enc, fmt, w, h):
     d_orig = torch.from_numpy(orig.view(np.int32)).cuda()
     d_enc = torch.from_numpy(enc).cuda()
