@@ -35,35 +35,18 @@ struct Tables {
 __device__ __forceinline__ int clamp255(int v) { return v < 0 ? 0 : (v > 255 ? 255 : v); }
 __device__ __forceinline__ int chan(uint32_t p, int k) { return (int)((p >> (8 * k)) & 0xFFu); }
 
-typedef short s16x2_t __attribute__((ext_vector_type(2)));
-
-// Red and green of texel p as two 16-bit lanes.
-__device__ __forceinline__ uint32_t rg_of(uint32_t p) {
-  return __builtin_amdgcn_perm(0u, p, 0x0c010c00u);
-}
-
-// Squared RGB distance of texel p to the colour (rg: red and green lanes,
-// b): the red/green differences as 16-bit lanes in one two-way dot product
-// (all terms below 2^17, so the sums are exact).
-__device__ __forceinline__ uint32_t dist2(uint32_t p, uint32_t rg, int b) {
-  const s16x2_t d = __builtin_bit_cast(s16x2_t, rg_of(p)) - __builtin_bit_cast(s16x2_t, rg);
-  const int db = chan(p, 2) - b;
-  return (uint32_t)__builtin_amdgcn_sdot2(d, d, db * db, false);
-}
-
 struct Solution {
   int r, g, b;      // unscaled block colour
   int inten;
   uint32_t sel;     // 8 selector indices, 2 bits each
-  uint64_t err;
+  uint32_t err;     // at most 8 * 3 * 255^2
   bool valid;
 };
 
 struct Opt {
-  uint32_t px[8];
-  int luma_sorted[8];
-  int idx_sorted[8];
-  uint32_t px_sorted[8];  // px[idx_sorted[k]]
+  uint32_t px[8];  // alpha cleared
+  int luma2[8];    // 2 (r + g + b)
+  uint32_t norm;   // sum of the pixels' squared lengths
   float avg[3];
   int limit;
   int br, bg, bb;
@@ -72,19 +55,21 @@ struct Opt {
   int base_r, base_g, base_b;
 };
 
-// etc1_optimizer::init for 8 pixels (low quality: sorted luma needed).
+// etc1_optimizer::init for 8 pixels.  (rg_etc1 sorts the lumas for its walk over
+// a row's midpoints; evaluate_fast needs no order.)
 __device__ void opt_init(Opt &o, const uint32_t sub[8], bool color4) {
   o.limit = color4 ? 15 : 31;
   o.color4 = color4;
   float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f;
-  int luma[8];
+  o.norm = 0;
 #pragma unroll
   for (int i = 0; i < 8; i++) {
-    o.px[i] = sub[i];
+    o.px[i] = sub[i] & 0x00FFFFFFu;
+    o.norm = __builtin_amdgcn_udot4(o.px[i], o.px[i], o.norm, false);
     s0 += (float)chan(sub[i], 0);
     s1 += (float)chan(sub[i], 1);
     s2 += (float)chan(sub[i], 2);
-    luma[i] = chan(sub[i], 0) + chan(sub[i], 1) + chan(sub[i], 2);
+    o.luma2[i] = 2 * (chan(sub[i], 0) + chan(sub[i], 1) + chan(sub[i], 2));
   }
   const float inv = 1.0f / 8.0f;
   o.avg[0] = s0 * inv;
@@ -94,21 +79,6 @@ __device__ void opt_init(Opt &o, const uint32_t sub[8], bool color4) {
   o.br = min(max((int)(uint32_t)(o.avg[0] * lim / 255.0f + 0.5f), 0), o.limit);
   o.bg = min(max((int)(uint32_t)(o.avg[1] * lim / 255.0f + 0.5f), 0), o.limit);
   o.bb = min(max((int)(uint32_t)(o.avg[2] * lim / 255.0f + 0.5f), 0), o.limit);
-  // stable sort of the 8 lumas (indirect_radix_sort is an LSD radix sort)
-#pragma unroll
-  for (int i = 0; i < 8; i++) {
-    int rank = 0;
-#pragma unroll
-    for (int j = 0; j < 8; j++) rank += (luma[j] < luma[i]) || (luma[j] == luma[i] && j < i);
-    // scatter through a select chain (rank is 0..7)
-#pragma unroll
-    for (int k = 0; k < 8; k++)
-      if (k == rank) {
-        o.luma_sorted[k] = luma[i];
-        o.idx_sorted[k] = i;
-        o.px_sorted[k] = sub[i];
-      }
-  }
 }
 
 __device__ __forceinline__ void scaled(const Opt &o, int r, int g, int b, int &sr, int &sg,
@@ -124,7 +94,25 @@ __device__ __forceinline__ void scaled(const Opt &o, int r, int g, int b, int &s
   }
 }
 
+// A candidate colour of a row as bytes, with its selector index in the top
+// two bits.
+__device__ __forceinline__ uint32_t row_colour(int r, int g, int b, uint32_t cur) {
+  return (uint32_t)r | ((uint32_t)g << 8) | ((uint32_t)b << 16) | (cur << 30);
+}
+
 // evaluate_solution_fast; updates best and returns true on improvement.
+//
+// VALU-bound, so every lane runs one path.  The reference takes shortcuts for
+// rows whose colours all lie above or below the sub-block's lumas, and leaves
+// such a row out where the nearest luma's distance alone reaches the best
+// error; both give what the general walk gives (the walk ends at the first or
+// last colour, and one pixel's squared distance is at least its luma's
+// difference), and a wave of different blocks would run all three.  A pixel
+// costs three comparisons, three selects, two four-way byte dot products (its
+// squared distance is p.p - 2 p.c + c.c, p.p summed once) and one shift that
+// collects the index.
+// 2044x1532: 281 us with the shortcuts, the sorted lumas that they need and 205
+// VGPRs (two waves a SIMD, three to place); 162 us at 122 VGPRs (four).
 __device__ bool evaluate_fast(const Opt &o, int cr, int cg, int cb, Solution &best) {
   if (o.constrain) {
     const int dr = cr - o.base_r, dg = cg - o.base_g, db = cb - o.base_b;
@@ -133,14 +121,10 @@ __device__ bool evaluate_fast(const Opt &o, int cr, int cg, int cb, Solution &be
   }
   int sr, sg, sb;
   scaled(o, cr, cg, cb, sr, sg, sb);
-  uint64_t terr = ~0ull;
+  uint32_t terr = ~0u, tsel = 0;
   int tinten = 0;
-  uint32_t tsel = 0;
-  bool tvalid = false;
-  const int lmax = o.luma_sorted[7], lmin = o.luma_sorted[0];
+#pragma unroll 1
   for (int it = 7; it >= 0; --it) {
-    // the four candidate colours of intensity row it (no private arrays:
-    // a per-lane index into one would live in scratch memory)
     const int y0 = kInten[it][0], y1 = kInten[it][1], y2 = kInten[it][2], y3 = kInten[it][3];
     const int c0r = clamp255(sr + y0), c0g = clamp255(sg + y0), c0b = clamp255(sb + y0);
     const int c1r = clamp255(sr + y1), c1g = clamp255(sg + y1), c1b = clamp255(sb + y1);
@@ -149,50 +133,33 @@ __device__ bool evaluate_fast(const Opt &o, int cr, int cg, int cb, Solution &be
     const int bi0 = c0r + c0g + c0b, bi1 = c1r + c1g + c1b, bi2 = c2r + c2g + c2b,
               bi3 = c3r + c3g + c3b;
     const int mid0 = bi0 + bi1, mid1 = bi1 + bi2, mid2 = bi2 + bi3;
-    const uint32_t c0rg = (uint32_t)c0r | ((uint32_t)c0g << 16);
-    const uint32_t c1rg = (uint32_t)c1r | ((uint32_t)c1g << 16);
-    const uint32_t c2rg = (uint32_t)c2r | ((uint32_t)c2g << 16);
-    const uint32_t c3rg = (uint32_t)c3r | ((uint32_t)c3g << 16);
-    // a row's error is at most 8 * 3 * 255^2 < 2^21: 32-bit sums are exact
-    uint32_t total = 0;
-    uint32_t sel = 0;
-    if (lmax * 2 < mid0) {
-      if (bi0 > lmax && (uint64_t)(bi0 - lmax) >= terr) continue;
+    const uint32_t c0 = row_colour(c0r, c0g, c0b, 0), c1 = row_colour(c1r, c1g, c1b, 1),
+                   c2 = row_colour(c2r, c2g, c2b, 2), c3 = row_colour(c3r, c3g, c3b, 3);
+    // the reference walks its selector up the midpoints as the sorted lumas
+    // rise; the midpoints do not decrease (the row's offsets increase), so
+    // the walk ends at the number of midpoints at or below 2 y
+    uint32_t pc = 0, cc = 0, sel = 0;
 #pragma unroll
-      for (int c = 0; c < 8; c++) total += dist2(o.px[c], c0rg, c0b);
-      sel = 0;
-    } else if (lmin * 2 >= mid2) {
-      if (lmin > bi3 && (uint64_t)(lmin - bi3) >= terr) continue;
-#pragma unroll
-      for (int c = 0; c < 8; c++) total += dist2(o.px[c], c3rg, c3b);
-      sel = 0xFFFFu;
-    } else {
-      // the reference walks cur up the midpoints as the sorted lumas rise;
-      // the midpoints do not decrease (the row's offsets increase), so the
-      // walk ends at the number of midpoints at or below 2 y: 3 if the last
-      // is, else 2 if the middle one is, ...
-#pragma unroll
-      for (int c = 0; c < 8; c++) {
-        const int y2x = o.luma_sorted[c] * 2;
-        const bool g0 = y2x >= mid0, g1 = y2x >= mid1, g2 = y2x >= mid2;
-        const uint32_t cur = g2 ? 3u : (g1 ? 2u : (g0 ? 1u : 0u));
-        const int pi = o.idx_sorted[c];
-        const uint32_t p = o.px_sorted[c];
-        const uint32_t erg = g2 ? c3rg : (g1 ? c2rg : (g0 ? c1rg : c0rg));
-        const int eb = g2 ? c3b : (g1 ? c2b : (g0 ? c1b : c0b));
-        total += dist2(p, erg, eb);
-        sel |= cur << (2 * pi);
-      }
+    for (int c = 7; c >= 0; c--) {
+      const int y2x = o.luma2[c];
+      uint32_t e = y2x >= mid0 ? c1 : c0;
+      e = y2x >= mid1 ? c2 : e;
+      e = y2x >= mid2 ? c3 : e;
+      pc = __builtin_amdgcn_udot4(o.px[c], e, pc, false);
+      cc = __builtin_amdgcn_udot4(e, e, cc, false);
+      sel = __builtin_amdgcn_alignbit(sel, e, 30);  // sel << 2 | index
     }
-    if (total < terr) {
-      terr = total;
-      tinten = it;
-      tsel = sel;
-      tvalid = true;
-      if (!total) break;
-    }
+    // the index in an e's top byte adds (64 index)^2 to its square
+    const uint32_t lo = sel & 0x5555u, hi = (sel >> 1) & 0x5555u;
+    const uint32_t idx2 = (uint32_t)(__popc(lo) + 4 * __popc(hi) + 4 * __popc(lo & hi));
+    const uint32_t total = o.norm - 2 * pc + cc - (idx2 << 12);
+    // a later row never beats a total of 0
+    const bool better = total < terr;
+    terr = better ? total : terr;
+    tinten = better ? it : tinten;
+    tsel = better ? sel : tsel;
   }
-  if (tvalid && terr < best.err) {
+  if (terr < best.err) {
     best.err = terr;
     best.inten = tinten;
     best.sel = tsel;
@@ -208,7 +175,7 @@ __device__ bool evaluate_fast(const Opt &o, int cr, int cg, int cb, Solution &be
 // etc1_optimizer::compute with scan deltas {0} and two refinement trials.
 __device__ bool opt_compute(const Opt &o, Solution &best) {
   best.valid = false;
-  best.err = ~0ull;
+  best.err = ~0u;
   best.r = best.g = best.b = 0;
   best.inten = 0;
   best.sel = 0;
@@ -340,7 +307,7 @@ __device__ uint2 pack_block(const Tables *t, const uint32_t px[16]) {
   for (int r = 1; r < 16; r++) solid = solid && px[r] == px[0];
   if (solid) return pack_solid(t, px[0]);
 
-  uint64_t best_error = ~0ull;
+  uint32_t best_error = ~0u;
   int best_flip = 0, best_c4 = 0;
   Solution best0, best1;
   best0.valid = best1.valid = false;
@@ -352,7 +319,7 @@ __device__ uint2 pack_block(const Tables *t, const uint32_t px[16]) {
     for (int c4 = 0; c4 < 2; c4++) {
       Solution r0, r1;
       if (!fit_subblock(px, flip, 0, c4 != 0, false, 0, 0, 0, r0)) continue;
-      uint64_t trial_error = r0.err;
+      uint32_t trial_error = r0.err;
       if (trial_error >= best_error) continue;
       // the 555 mode's second colour is a delta of the first: constrained
       if (!fit_subblock(px, flip, 1, c4 != 0, !c4, r0.r, r0.g, r0.b, r1)) continue;
