@@ -172,48 +172,72 @@ __device__ uint32_t match_colors(const uint32_t blk[16], const int col[4][3]) {
   return mask;
 }
 
+// A block's colour channels, four texels to a word, and their sums: the sums
+// of products that the fit needs are then four-way byte dot products.
+// 119 -> 87 VGPRs; the dither's serial chain before it stays: 4096x4096 DXT5
+// 57.9 -> 55.9 us, 2048x2048 DXT1 16.1 -> 15.5.
+struct Planes {
+  uint32_t w[3][4];
+  int sum[3];
+};
+
+__device__ __forceinline__ void planes_of(const uint32_t blk[16], Planes &pl) {
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    const uint32_t *p = blk + 4 * k;
+    const uint32_t rg01 = __builtin_amdgcn_perm(p[1], p[0], 0x05010400u);
+    const uint32_t rg23 = __builtin_amdgcn_perm(p[3], p[2], 0x05010400u);
+    const uint32_t b01 = __builtin_amdgcn_perm(p[1], p[0], 0x0c0c0602u);
+    const uint32_t b23 = __builtin_amdgcn_perm(p[3], p[2], 0x0c0c0602u);
+    pl.w[0][k] = __builtin_amdgcn_perm(rg23, rg01, 0x05040100u);
+    pl.w[1][k] = __builtin_amdgcn_perm(rg23, rg01, 0x07060302u);
+    pl.w[2][k] = __builtin_amdgcn_perm(b23, b01, 0x05040100u);
+  }
+#pragma unroll
+  for (int c = 0; c < 3; c++) {
+    uint32_t s = 0;
+#pragma unroll
+    for (int k = 0; k < 4; k++) s = __builtin_amdgcn_udot4(pl.w[c][k], 0x01010101u, s, false);
+    pl.sum[c] = (int)s;
+  }
+}
+
+// Smallest and largest byte of four words.  As 16-bit numbers the words order
+// by their upper bytes, and shifted up by their lower ones.
+__device__ __forceinline__ void byte_range(const uint32_t w[4], int &mn, int &mx) {
+  typedef uint16_t u16x2_t __attribute__((ext_vector_type(2)));
+  u16x2_t lo = __builtin_bit_cast(u16x2_t, w[0]), hi = lo;
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    const u16x2_t odd = __builtin_bit_cast(u16x2_t, w[k]), even = odd << (uint16_t)8;
+    lo = __builtin_elementwise_min(lo, __builtin_elementwise_min(odd, even));
+    hi = __builtin_elementwise_max(hi, __builtin_elementwise_max(odd, even));
+  }
+  mn = (int)(min((uint32_t)lo.x, (uint32_t)lo.y) >> 8);
+  mx = (int)(max((uint32_t)hi.x, (uint32_t)hi.y) >> 8);
+}
+
 // stb__OptimizeColorsBlock
-__device__ void optimize_colors(const uint32_t blk[16], uint32_t &max16, uint32_t &min16) {
+__device__ void optimize_colors(const uint32_t blk[16], const Planes &pl, uint32_t &max16,
+                                uint32_t &min16) {
   int mu[3], mn[3], mx[3];
 #pragma unroll
   for (int c = 0; c < 3; c++) {
-    int muv = ch(blk[0], c), minv = muv, maxv = muv;
-#pragma unroll
-    for (int i = 1; i < 16; i++) {
-      const int v = ch(blk[i], c);
-      muv += v;
-      // stb_dxt's "if (v < min) ... else if (v > max)" with min <= max
-      // throughout is the plain running minimum and maximum
-      minv = min(minv, v);
-      maxv = max(maxv, v);
-    }
-    mu[c] = (muv + 8) >> 4;
-    mn[c] = minv;
-    mx[c] = maxv;
+    mu[c] = (pl.sum[c] + 8) >> 4;
+    byte_range(pl.w[c], mn[c], mx[c]);
   }
   // sum (x - mx)(y - my) = sum xy - my sum x - mx sum y + 16 mx my, exactly
   // in integers: the products are of bytes
-  int sp[6] = {0, 0, 0, 0, 0, 0}, sx[3] = {0, 0, 0};
-#pragma unroll
-  for (int i = 0; i < 16; i++) {
-    const int r = ch(blk[i], 0), g = ch(blk[i], 1), b = ch(blk[i], 2);
-    sp[0] += r * r;
-    sp[1] += r * g;
-    sp[2] += r * b;
-    sp[3] += g * g;
-    sp[4] += g * b;
-    sp[5] += b * b;
-    sx[0] += r;
-    sx[1] += g;
-    sx[2] += b;
-  }
   int cov[6];
   {
     const int pr[6][2] = {{0, 0}, {0, 1}, {0, 2}, {1, 1}, {1, 2}, {2, 2}};
 #pragma unroll
     for (int k = 0; k < 6; k++) {
       const int x = pr[k][0], y = pr[k][1];
-      cov[k] = sp[k] - mu[y] * sx[x] - mu[x] * sx[y] + 16 * mu[x] * mu[y];
+      uint32_t sp = 0;
+#pragma unroll
+      for (int i = 0; i < 4; i++) sp = __builtin_amdgcn_udot4(pl.w[x][i], pl.w[y][i], sp, false);
+      cov[k] = (int)sp - mu[y] * pl.sum[x] - mu[x] * pl.sum[y] + 16 * mu[x] * mu[y];
     }
   }
   // cov / 255.0f, correctly rounded: |cov| < 2^24, and cov / 255 is an
@@ -278,21 +302,11 @@ __device__ __forceinline__ int sclamp(float y, int p0, int p1) {
 }
 
 // stb__RefineBlock; returns whether the endpoints changed.
-__device__ bool refine_block(const uint32_t blk[16], uint32_t &max16, uint32_t &min16,
-                             uint32_t mask) {
+__device__ bool refine_block(const Planes &pl, uint32_t &max16, uint32_t &min16, uint32_t mask) {
   const uint32_t old_min = min16, old_max = max16;
   uint32_t nmin, nmax;
   if ((mask ^ (mask << 2)) < 4) {
-    int r = 8, g = 8, b = 8;
-#pragma unroll
-    for (int i = 0; i < 16; i++) {
-      r += ch(blk[i], 0);
-      g += ch(blk[i], 1);
-      b += ch(blk[i], 2);
-    }
-    r >>= 4;
-    g >>= 4;
-    b >>= 4;
+    const int r = (8 + pl.sum[0]) >> 4, g = (8 + pl.sum[1]) >> 4, b = (8 + pl.sum[2]) >> 4;
     nmax = ((uint32_t)kT.omatch5[r][0] << 11) | ((uint32_t)kT.omatch6[g][0] << 5) | kT.omatch5[b][0];
     nmin = ((uint32_t)kT.omatch5[r][1] << 11) | ((uint32_t)kT.omatch6[g][1] << 5) | kT.omatch5[b][1];
   } else {
@@ -305,22 +319,21 @@ __device__ bool refine_block(const uint32_t blk[16], uint32_t &max16, uint32_t &
     const int xx = 9 * n0 + 4 * n2 + n3;
     const int yy = 9 * n1 + n2 + 4 * n3;
     const int xy = 2 * (n2 + n3);
-    // red and blue in the two 16-bit halves of one word: each half's sum
-    // stays below 3 * 16 * 255 < 2^16, and r | b << 16 < 2^24
-    uint32_t a1rb = 0, a2rb = 0, a1g = 0, a2g = 0;
+    // four texels' weights as bytes: their indices spread to bytes select
+    // from the four weights
+    uint32_t a1[3] = {0, 0, 0};
 #pragma unroll
-    for (int i = 0; i < 16; i++) {
-      const uint32_t w1 = (0x1203u >> (((mask >> (2 * i)) & 3u) * 4u)) & 15u;
-      const uint32_t rb = blk[i] & 0x00FF00FFu, g = (blk[i] >> 8) & 0xFFu;
-      a1rb += w1 * rb;
-      a1g += w1 * g;
-      a2rb += rb;
-      a2g += g;
+    for (int k = 0; k < 4; k++) {
+      const uint32_t m = (mask >> (8 * k)) & 0xFFu;
+      const uint32_t idx = (m | (m << 6) | (m << 12) | (m << 18)) & 0x03030303u;
+      const uint32_t w1 = __builtin_amdgcn_perm(0u, 0x01020003u, idx);
+#pragma unroll
+      for (int c = 0; c < 3; c++) a1[c] = __builtin_amdgcn_udot4(pl.w[c][k], w1, a1[c], false);
     }
-    const int a1r = (int)(a1rb & 0xFFFFu), a1b = (int)(a1rb >> 16), a1gi = (int)a1g;
-    const int a2r = 3 * (int)(a2rb & 0xFFFFu) - a1r;
-    const int a2gi = 3 * (int)a2g - a1gi;
-    const int a2b = 3 * (int)(a2rb >> 16) - a1b;
+    const int a1r = (int)a1[0], a1gi = (int)a1[1], a1b = (int)a1[2];
+    const int a2r = 3 * pl.sum[0] - a1r;
+    const int a2gi = 3 * pl.sum[1] - a1gi;
+    const int a2b = 3 * pl.sum[2] - a1b;
     // 3.0f * 31.0f / 255.0f is evaluated left to right in float
     const float frb = ((3.0f * 31.0f) / 255.0f) / (float)(xx * yy - xy * xy);
     const float fg = (frb * 63.0f) / 31.0f;
@@ -350,7 +363,9 @@ __device__ uint2 compress_color(const uint32_t blk[16], const uint8_t *q) {
   } else {
     uint32_t dblk[16];
     dither_block(blk, dblk, q);
-    optimize_colors(dblk, max16, min16);
+    Planes pl;
+    planes_of(dblk, pl);
+    optimize_colors(dblk, pl, max16, min16);
     int col[4][3];
     if (max16 != min16) {
       eval_colors(col, max16, min16);
@@ -359,7 +374,7 @@ __device__ uint2 compress_color(const uint32_t blk[16], const uint8_t *q) {
       mask = 0;
     }
     const uint32_t last = mask;
-    if (refine_block(dblk, max16, min16, mask)) {
+    if (refine_block(pl, max16, min16, mask)) {
       if (max16 != min16) {
         eval_colors(col, max16, min16);
         mask = match_colors(blk, col);
