@@ -131,6 +131,35 @@ def test_block_error_matches_oracle(fh, oracle, name, w, h):
     assert total == want_total
 
 
+@pytest.mark.parametrize("w,h", [(1024, 9), (1022, 9), (1023, 9), (3, 2)])
+@pytest.mark.parametrize("name", list(FORMATS) + ["rgba8"])
+def test_errors_of_waves_with_and_without_cut_blocks(fh, oracle, name, w, h):
+    """Rows of 256 blocks at every width of row access: whole waves, waves
+    that end in a block the right edge cuts and waves the bottom edge cuts.
+    Integers: exact."""
+    print(f"cut waves {name} {w}x{h}", flush=True)
+    rng = np.random.default_rng(w)
+    orig = rng.integers(0, 2**32, (h, w), dtype=np.uint32)
+    if name == "rgba8":
+        dec = rng.integers(0, 2**32, (h, w), dtype=np.uint32)
+        da = torch.from_numpy(orig.view(np.int32)).cuda()
+        db = torch.from_numpy(dec.view(np.int32)).cuda()
+        blk = torch.zeros((w + 3) // 4 * ((h + 3) // 4), dtype=torch.int64, device="cuda")
+        sse = torch.zeros(2, dtype=torch.int64, device="cuda")
+        fh.image_error_device(da.data_ptr(), db.data_ptr(), w, h, sse.data_ptr(), blk.data_ptr())
+        torch.cuda.synchronize()
+        s = sse.cpu().numpy().view(np.uint64)
+        blocks, total = blk.cpu().numpy().view(np.uint64), int(s[0]) + (int(s[1]) << 64)
+    else:
+        fmt = FORMATS[name][0]
+        data = random_blocks(name, w, h, 3 + fmt)
+        dec = oracle_decode(oracle, fmt, data, w, h)
+        blocks, total = _errors(fh, orig, data, fmt, w, h)
+    want_blocks, want_total = oracle.block_errors(orig, dec)
+    assert np.array_equal(blocks, want_blocks)
+    assert total == want_total
+
+
 def test_image_error_and_psnr(fh, oracle):
     w, h = 257, 131
     a = synth.generate(260, 132, 4)[:h, :w].copy()
