@@ -3136,23 +3136,27 @@ __device__ __forceinline__ void score_pixels(const Lane &L, const SubConst &sc0,
 // The pixel pass under the nonuniform metric: float errors, each subset's
 // summed in pixel order (adding 0 to the other subsets' sums leaves them
 // unchanged).
+template <int NSUB, bool ROT>
 __device__ __forceinline__ void score_pixels_nu(const Lane &L, const SubConst &sc0,
                                                 const SubConst &sc1, const SubConst &sc2,
                                                 float kf, WeightFn wf, float &n0, float &n1,
                                                 float &n2, uint64_t &nidx) {
+  uint32_t lo = 0, hi = 0;
   n0 = n1 = n2 = 0.0f;
-  nidx = 0;
 #pragma unroll
   for (int i = 0; i < 16; i++) {
-    const bool in1 = (L.m12 & (1u << i)) != 0, in2 = (L.m12 & (1u << (16 + i))) != 0;
-    const SubConst c = pixel_const<3, true>(in1, in2, sc0, sc1, sc2);
+    const bool in1 = NSUB > 1 && (L.m12 & (1u << i)) != 0;
+    const bool in2 = NSUB > 2 && (L.m12 & (1u << (16 + i))) != 0;
+    const SubConst c = pixel_const<NSUB, ROT>(in1, in2, sc0, sc1, sc2);
     uint32_t best;
     const float me = pixel_err_nu(L.px[2 * i], L.px[2 * i + 1], c, kf, wf, L.m, &best);
     n0 += in1 || in2 ? 0.0f : me;
-    n1 += in1 ? me : 0.0f;
-    n2 += in2 ? me : 0.0f;
-    nidx |= (uint64_t)best << (4 * i);
+    if (NSUB > 1) n1 += in1 ? me : 0.0f;
+    if (NSUB > 2) n2 += in2 ? me : 0.0f;
+    if (i < 8) lo |= best << (4 * i);
+    else hi |= best << (4 * (i - 8));
   }
+  nidx = (uint64_t)lo | ((uint64_t)hi << 32);
 }
 
 // One annealing step of every active subset, for waves whose running
@@ -3175,7 +3179,7 @@ __device__ __forceinline__ void lane_step_n(Lane &L, const uint8_t *quant, int q
   uint64_t nidx;
   if constexpr (NU) {
     float e0, e1, e2;
-    score_pixels_nu(L, sc0, sc1, sc2, k.kf, k.wf, e0, e1, e2, nidx);
+    score_pixels_nu<NSUB, ROT>(L, sc0, sc1, sc2, k.kf, k.wf, e0, e1, e2, nidx);
     n0.err = __float_as_uint(e0);
     n1.err = __float_as_uint(e1);
     n2.err = __float_as_uint(e2);
@@ -3202,18 +3206,17 @@ __device__ __forceinline__ void lane_step_n(Lane &L, const uint8_t *quant, int q
 
 // The widest subset count among the wave's running lanes picks the compiled
 // step (a wave-uniform branch): the list is ordered by mode, so most waves
-// hold candidates of one subset count.
+// hold candidates of one subset count.  (Under the nonuniform metric, whose
+// steps are mostly the rotation modes', annealing with the three-subset step
+// alone takes 11.5 ms for 1024x1024 and 18.9 for 2048x2048; by count 8.8 and
+// 14.5.)
 template <bool NU>
 __device__ __forceinline__ void lane_step(Lane &L, const uint8_t *quant, int q) {
-  if constexpr (NU) {
-    lane_step_n<3, true, true>(L, quant, q);
-  } else {
-    const bool run = L.active != 0;
-    if (!__ballot(run && L.nsub > 1)) lane_step_n<1, true, false>(L, quant, q);
-    else if (__ballot(run && L.ptmode != 0)) lane_step_n<3, true, false>(L, quant, q);
-    else if (__ballot(run && L.nsub == 3)) lane_step_n<3, false, false>(L, quant, q);
-    else lane_step_n<2, false, false>(L, quant, q);
-  }
+  const bool run = L.active != 0;
+  if (!__ballot(run && L.nsub > 1)) lane_step_n<1, true, NU>(L, quant, q);
+  else if (__ballot(run && L.ptmode != 0)) lane_step_n<3, true, NU>(L, quant, q);
+  else if (__ballot(run && L.nsub == 3)) lane_step_n<3, false, NU>(L, quant, q);
+  else lane_step_n<2, false, NU>(L, quant, q);
 }
 
 template <bool NU = false>

@@ -1,7 +1,8 @@
 """The annealing's forms (one lane per pixel for small lists, one lane per
-candidate with a handed-over tail for large ones) at the sizes where the
-choice changes: whole images against the oracle, and large jobs against the
-same blocks encoded in smaller ones."""
+candidate with a handed-over tail for large ones) and the set-up's (one launch
+or one per mode) at the sizes where the choice changes, for every search that
+takes them: whole images against the oracle, and large jobs against the same
+blocks encoded in smaller ones."""
 import ctypes
 import os
 
@@ -9,6 +10,7 @@ import numpy as np
 import pytest
 
 from fastc_amd import synth
+from tests.test_selection import random_selections
 
 pytestmark = pytest.mark.gpu
 WEIGHTS = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
@@ -42,6 +44,68 @@ def test_reference_search_matches_oracle(fh, oracle, w, h):
     assert n_ref == want and n_gpu % 16 == 0 and n_gpu >= n_ref
     plain = fh.compress(img, quality=4, seed=9, wm_counter=ctypes.c_uint32(0xFFFFFFFF))
     assert np.array_equal(plain, got)
+
+
+@pytest.mark.parametrize("w,h,q", [(512, 512, 0), (516, 512, 2)])
+def test_nonuniform_metric_matches_oracle(fh, oracle, w, h, q):
+    """The nonuniform metric on the last size of the merged set-up and, with
+    annealing, the first of one launch per mode: the waves' steps for one,
+    two and three subsets."""
+    img = synth.generate(w, h, 12)
+    print(f"nonuniform forms {w}x{h}", flush=True)
+    ref, ref_wm = oracle.bc7_compress(img, quality=q, seed=4, q0_guard=True, metric=1)
+    wm = ctypes.c_uint32(0xFFFFFFFF)
+    got = fh.compress(img, quality=q, seed=4, wm_counter=wm, metric=1)
+    bad = _diff(got, ref)
+    assert bad.size == 0, f"{bad.size} blocks differ, first {bad[:8]}"
+    assert wm.value == ref_wm
+
+
+def _row_rects(side, parts):
+    """The image's rows in equal parts: (rect, first row, rows) of each."""
+    rows = side // parts
+    for k in range(parts):
+        y0, y1 = k * rows, (k + 1) * rows
+        # up to the start of the next part's first row
+        yield ((0, y0, 0, y1) if y1 < side else (0, y0, side, side)), y0, rows
+
+
+@pytest.mark.parametrize("search", ["nonuniform"])
+def test_other_searches_compose(fh, search):
+    """25600 blocks, annealed, equal their quarters (which run the forms for
+    small jobs, held against the oracle in those searches' own tests)."""
+    side, parts = 640, 4
+    img = synth.generate(side, side, 23)
+    n = (side // 4) ** 2
+    sels = None
+    if search == "selections":
+        sels = np.tile(random_selections(256, 3, 12), n // 256)
+    print(f"anneal forms {search}", flush=True)
+
+    def encode(rect, first, count):
+        wm = ctypes.c_uint32(0xFFFFFFFF)
+        kw = dict(quality=12, seed=6, rect=rect, wm_counter=wm)
+        if search == "nonuniform":
+            return fh.compress(img, metric=1, **kw), None
+        if search == "statistics":
+            out, st = fh.compress_with_stats(img, **kw)
+            return out, st[:count]
+        return fh.compress_with_selection(img, sels[first:first + count], **kw), None
+
+    whole, stats = encode(None, 0, n)
+    per_row = side // 4
+    for rect, y0, rows in _row_rects(side, parts):
+        first, count = y0 // 4 * per_row, rows // 4 * per_row
+        out, st = encode(rect, first, count)
+        a = whole.reshape(-1, 16)[first:first + count]
+        b = out.reshape(-1, 16)[first:first + count]
+        # each part starts its own watermark: solid blocks differ in it
+        px = synth.blocks(img).reshape(n, 16)[first:first + count]
+        searched = (px != px[:, :1]).any(axis=1)
+        bad = np.nonzero((a != b).any(axis=1) & searched)[0]
+        assert bad.size == 0, f"{bad.size} blocks differ from row {y0}, first {bad[:8]}"
+        if stats is not None:
+            assert stats[first:first + count].tobytes() == st.tobytes()
 
 
 @pytest.mark.parametrize("learned,side,parts", [(False, 640, 4), (True, 1280, 4)])
