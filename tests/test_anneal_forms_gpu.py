@@ -70,7 +70,7 @@ def _row_rects(side, parts):
         yield ((0, y0, 0, y1) if y1 < side else (0, y0, side, side)), y0, rows
 
 
-@pytest.mark.parametrize("search", ["nonuniform"])
+@pytest.mark.parametrize("search", ["nonuniform", "statistics", "selections"])
 def test_other_searches_compose(fh, search):
     """25600 blocks, annealed, equal their quarters (which run the forms for
     small jobs, held against the oracle in those searches' own tests)."""
