@@ -3733,9 +3733,12 @@ anneal_kernel(BlockRange r, Bc7Params prm, Work w, uint32_t unroll, uint32_t tai
   // past the front's) are its suffix.  Their chains are the
   // longest by far (to 1410 steps, against a mean of 66 in mode 1), so the
   // first rot_groups workgroups start on them at once, four lanes each, while
-  // the others run the rest.  (The reference search's list is mostly rotation
-  // states: one lane each is the cheapest form, and the list starts with
-  // them.)
+  // the others run the rest.  That holds while they are few: where one state
+  // in eight or more is a rotation's (blocks the ranker is not sure about
+  // anneal the reference search's candidates, a third of them rotations), the
+  // few workgroups would set the time, and one lane each is the cheapest form:
+  // 2048x2048 with every block unsure 31.8 ms in this phase, 8.9 without;
+  // sure (one in twenty) 1.29 with and 2.38 without.
   if (!NU && rot_groups && w.alist) {
     const uint32_t first_rot = sm.front;
     uint32_t lo = 0, hi = total;  // first list entry >= first_rot
@@ -3744,10 +3747,12 @@ anneal_kernel(BlockRange r, Bc7Params prm, Work w, uint32_t unroll, uint32_t tai
       if (w.alist[mid] < first_rot) lo = mid + 1;
       else hi = mid;
     }
-    if (blockIdx.x < rot_groups)
-      spread_run<4, kFromListHand, COUNT>(r, prm, w, tail, s_quant, lo, total, 4 * rot_groups,
-                                          &w.counters[kCntRotFetch], n_ref, n_gpu);
-    total = lo;
+    if (8u * (total - lo) < total) {
+      if (blockIdx.x < rot_groups)
+        spread_run<4, kFromListHand, COUNT>(r, prm, w, tail, s_quant, lo, total, 4 * rot_groups,
+                                            &w.counters[kCntRotFetch], n_ref, n_gpu);
+      total = lo;
+    }
   }
   Lane L = {};  // lanes without a candidate step along on zeros
   L.nsub = 1;

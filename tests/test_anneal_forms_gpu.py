@@ -21,20 +21,20 @@ def _diff(a, b):
     return np.nonzero((a.reshape(-1, 16) != b.reshape(-1, 16)).any(axis=1))[0]
 
 
-@pytest.mark.parametrize("w,h", [(512, 512), (516, 512), (8, 4)])
-def test_reference_search_matches_oracle(fh, oracle, w, h):
+@pytest.mark.parametrize("w,h,q", [(512, 512, 4), (516, 512, 4), (8, 4, 4)])
+def test_reference_search_matches_oracle(fh, oracle, w, h, q):
     """16384 blocks (the last size of the first form), 16512 (the first of
     the second) and two blocks, with the work counts."""
     img = synth.generate(w, h, 31)
-    print(f"anneal forms {w}x{h}", flush=True)
+    print(f"anneal forms {w}x{h} q={q}", flush=True)
     L = oracle.lib()
     L.ora_anneal_point_count(1)
-    ref, ref_wm = oracle.bc7_compress(img, quality=4, seed=9, q0_guard=True)
+    ref, ref_wm = oracle.bc7_compress(img, quality=q, seed=9, q0_guard=True)
     want = L.ora_anneal_point_count(1)
     wm = ctypes.c_uint32(0xFFFFFFFF)
     fh.set_work_counting(True)
     try:
-        got = fh.compress(img, quality=4, seed=9, wm_counter=wm)
+        got = fh.compress(img, quality=q, seed=9, wm_counter=wm)
         n_ref, n_gpu = fh.work_counts()
     finally:
         fh.set_work_counting(False)
@@ -42,7 +42,7 @@ def test_reference_search_matches_oracle(fh, oracle, w, h):
     assert bad.size == 0, f"{bad.size} blocks differ, first {bad[:8]}"
     assert wm.value == ref_wm
     assert n_ref == want and n_gpu % 16 == 0 and n_gpu >= n_ref
-    plain = fh.compress(img, quality=4, seed=9, wm_counter=ctypes.c_uint32(0xFFFFFFFF))
+    plain = fh.compress(img, quality=q, seed=9, wm_counter=ctypes.c_uint32(0xFFFFFFFF))
     assert np.array_equal(plain, got)
 
 
@@ -108,26 +108,28 @@ def test_other_searches_compose(fh, search):
             assert stats[first:first + count].tobytes() == st.tobytes()
 
 
-@pytest.mark.parametrize("learned,side,parts", [(False, 640, 4), (True, 1280, 4)])
-def test_parts_compose(fh, learned, side, parts):
-    """A job of the second form equals its quarters, which run the first (the
-    annealing streams are keyed by the block's place in the image)."""
+@pytest.mark.parametrize("threshold,side,parts", [(None, 640, 4), (0.6, 1280, 4),
+                                                  (1.5, 1280, 5)])
+def test_parts_compose(fh, threshold, side, parts):
+    """A large job equals its parts, which run the other form (the annealing
+    streams are keyed by the block's place in the image).  threshold: of the
+    learned search, None for the reference's.  At 1.5 every block falls back
+    to the full search's candidates, a third of them rotations, too many for
+    a phase of their own."""
+    learned = threshold is not None
     img = synth.generate(side, side, 17)
     rk = None
     if learned:
         rk = fh.Ranker()
         rk.set_params(np.load(WEIGHTS))
-    print(f"anneal forms learned={learned} {side}", flush=True)
+    print(f"anneal forms threshold={threshold} {side}", flush=True)
+    kw = dict(quality=50, seed=2, ranker=rk, threshold=threshold or 0.6)
     wm = ctypes.c_uint32(0xFFFFFFFF)
-    whole = fh.compress(img, quality=50, seed=2, wm_counter=wm, ranker=rk)
+    whole = fh.compress(img, wm_counter=wm, **kw)
     wm2 = ctypes.c_uint32(0xFFFFFFFF)
     out = np.zeros_like(whole)
-    rows = side // parts
-    for k in range(parts):
-        # rows [k * rows, (k + 1) * rows): up to the start of the next part's first row
-        y1 = (k + 1) * rows
-        rect = (0, k * rows, 0, y1) if y1 < side else (0, k * rows, side, side)
-        fh.compress(img, quality=50, seed=2, wm_counter=wm2, ranker=rk, rect=rect, out=out)
+    for rect, _, _ in _row_rects(side, parts):
+        fh.compress(img, wm_counter=wm2, rect=rect, out=out, **kw)
     bad = _diff(out, whole)
     assert bad.size == 0, f"{bad.size} blocks differ, first {bad[:8]}"
     assert wm.value == wm2.value
