@@ -1428,7 +1428,9 @@ struct Work {
 // chains, the earlier annealing starts on them (it runs from the end).  The
 // three regions cannot meet: mode 4's lies below room for every candidate of
 // mode 5, and a job's candidates all fit.
-// (Read once per kernel.)
+// (Read once per kernel, plainly: the counts stand when it starts.  Volatile
+// loads go past the caches, and every wave's to the same lines, one after
+// another: some 100 us of an annealing of 3072 waves.)
 struct StateMap {
   uint32_t front, c4, c5, base4, base5;
   __device__ __forceinline__ uint32_t count() const { return front + c4 + c5; }
@@ -1439,7 +1441,7 @@ struct StateMap {
   }
 };
 __device__ __forceinline__ StateMap state_map(const Work &w) {
-  const volatile uint32_t *c = w.counters;
+  const uint32_t *c = w.counters;
   StateMap m;
   m.front = c[kCntFront];
   m.c4 = c[kCntRot4];
@@ -1447,6 +1449,28 @@ __device__ __forceinline__ StateMap state_map(const Work &w) {
   m.base4 = w.astate_cap - c[kCntQueue + 7] - m.c4;  // below room for mode 5's whole queue
   m.base5 = w.astate_cap - m.c5;
   return m;
+}
+
+// Whether an annealing list of `total` states runs one lane per pixel
+// (anneal_spread_kernel) rather than one lane per candidate (anneal_kernel);
+// the two are launched together and this decides on the device, where the
+// count is.  Rotation states have the longest chains, which set the one-lane
+// form's time, so a list with at least one in eight of them may be twice as
+// long.  Annealing in ms, one lane per pixel against one per candidate:
+//   quality 50, few rotation states: 24,000 states 0.27 / 0.73, 66,000
+//     (learned search) 0.86 / 1.04, 95,000 0.89 / 0.82, 188,000 1.95 / 1.02;
+//   quality 50, many: 30,000 1.04 / 2.62, 141,000 2.49 / 2.85, 187,000
+//     3.28 / 3.11, 229,000 (noise) 7.56 / 4.22;
+//   quality 8, few: 24,000 0.13 / 0.17, 54,000 0.27 / 0.21;
+//   quality 8, many: 68,000 0.62 / 0.64, 120,000 0.97 / 0.62.
+// By the number of blocks alone, the rule before, a learned job of 64,000
+// blocks none of which the ranker was sure about annealed its 457,000 states
+// in 7.9 ms; 4.2 now.
+constexpr uint32_t kSpreadStates = 90112, kSpreadStatesShort = kSpreadStates / 2;
+constexpr uint32_t kShortChains = 16;  // the quality below which the chains are short
+__device__ __forceinline__ bool spread_list(const StateMap &m, uint32_t total,
+                                            uint32_t max_states) {
+  return total <= (8u * (m.c4 + m.c5) >= total ? 2u * max_states : max_states);
 }
 
 // Learned search: the list of annealing states that pass the margin, in
@@ -3686,16 +3710,19 @@ __device__ __forceinline__ void add_counts(const Bc7Params &prm, unsigned long l
 }
 
 // TAIL: the candidates the one-lane form handed over (kCntTail of them);
-// otherwise the whole annealing list.
+// otherwise the whole annealing list, if spread_list has it so.
 template <bool TAIL, bool COUNT>
 __global__ void __launch_bounds__(256) anneal_spread_kernel(BlockRange r, Bc7Params prm, Work w,
-                                                            TailState *tail) {
+                                                            TailState *tail,
+                                                            uint32_t max_states) {
+  const StateMap sm = state_map(w);
+  const uint32_t total = TAIL      ? w.counters[kCntTail]
+                         : w.alist ? w.counters[kCntList]
+                                   : sm.count();
+  if (total == 0 || (!TAIL && !spread_list(sm, total, max_states))) return;  // whole grid
   __shared__ __align__(4) uint8_t s_quant[kStepQuantBytes];
   step_quant_load(s_quant);
   __syncthreads();
-  const uint32_t total = TAIL      ? *(volatile uint32_t *)&w.counters[kCntTail]
-                         : w.alist ? *(volatile uint32_t *)&w.counters[kCntList]
-                                   : state_map(w).count();
   unsigned long long n_ref = 0, n_gpu = 0;
   spread_run<16, TAIL ? kFromTail : kFromList, COUNT>(r, prm, w, tail, s_quant, 0, total,
                                                       4 * gridDim.x, &w.counters[TAIL ? kCntTailFetch : kCntFetch],
@@ -3703,6 +3730,7 @@ __global__ void __launch_bounds__(256) anneal_spread_kernel(BlockRange r, Bc7Par
   if constexpr (COUNT) add_counts(prm, n_ref, n_gpu);
 }
 
+// max_states: of spread_list (0: the list is this kernel's).
 // unroll: annealing steps between looks at the idle lanes.
 // tail_lanes: once the list is used up, a wave with at most this many
 // running candidates hands them to anneal_spread_kernel (through `tail`),
@@ -3718,12 +3746,13 @@ __global__ void __launch_bounds__(256) anneal_spread_kernel(BlockRange r, Bc7Par
 template <int WAVES, bool NU = false, bool COUNT = false>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES)))
 anneal_kernel(BlockRange r, Bc7Params prm, Work w, uint32_t unroll, uint32_t tail_lanes,
-              uint32_t rot_groups, TailState *tail) {
+              uint32_t rot_groups, TailState *tail, uint32_t max_states) {
   const int lane = threadIdx.x & 63;
   unsigned long long n_ref = 0, n_gpu = 0;  // COUNT
   const uint64_t lt = (1ull << lane) - 1ull;
   const StateMap sm = state_map(w);
-  uint32_t total = w.alist ? *(volatile uint32_t *)&w.counters[kCntList] : sm.count();
+  uint32_t total = w.alist ? w.counters[kCntList] : sm.count();
+  if (spread_list(sm, total, max_states)) return;  // whole grid: anneal_spread_kernel's
   // odd row stride: conflict-free
   __shared__ uint32_t s_px[256 * kRowWords];
   __shared__ __align__(4) uint8_t s_quant[kStepQuantBytes];
@@ -4424,12 +4453,11 @@ hipError_t bc7_upload_tables(int device) {
   return hipSuccess;
 }
 
-// Blocks up to which a call's annealing runs one lane per pixel from the
-// start.  Its lists (about 7 states a block in the reference search, 1 in the
-// learned one) then leave the one-lane form too few waves, and the longest
-// chain sets the time: 508x380 (12065 blocks) anneals in 1.7 ms against 2.9,
-// 1000x1024 (64000) in 7.9 against 4.6; learned 1024x1024 in 0.83 against
-// 1.18, 2048x2048 in 3.0 against 1.3.
+// Blocks up to which a call's annealing may run one lane per pixel
+// (spread_list decides by its states: about 7 a block in the reference
+// search, 1 in the learned one where the ranker is sure).  Above, the list is
+// hardly ever short enough, and the set-up, which changes at the same sizes,
+// has put it in the order the one-lane form wants.
 constexpr uint32_t kSpreadBlocks = 1u << 14, kSpreadBlocksLearned = 1u << 16;
 // Running candidates at which a wave of the one-lane form hands over
 // (learned 4096x4096: 4..12 3.3 ms, 16 3.5, 24 3.6, never 3.8; reference
@@ -4462,17 +4490,20 @@ void launch_anneal(uint32_t waves, int cus, const BlockRange &r, const Bc7Params
   const uint32_t unroll = w.alist ? 4u : (p.anneal_unroll ? p.anneal_unroll : 1u);
   if (w.nu_total) {  // nonuniform metric (the full search or given selections)
     hipLaunchKernelGGL((bc7::anneal_kernel<1, true>), grid, wg, 0, stream, r, p, w, unroll, 0u,
-                       0u, (bc7::TailState *)nullptr);
+                       0u, (bc7::TailState *)nullptr, 0u);
     return;
   }
+  uint32_t max_states = 0;  // of spread_list
   if (r.num_blocks <= (w.alist ? kSpreadBlocksLearned : kSpreadBlocks)) {
+    max_states = p.quality < bc7::kShortChains ? bc7::kSpreadStatesShort : bc7::kSpreadStates;
     if (p.work_counts)
       hipLaunchKernelGGL((bc7::anneal_spread_kernel<false, true>), sgrid, wg, 0, stream, r, p, w,
-                         (bc7::TailState *)nullptr);
+                         (bc7::TailState *)nullptr, max_states);
     else
       hipLaunchKernelGGL((bc7::anneal_spread_kernel<false, false>), sgrid, wg, 0, stream, r, p, w,
-                         (bc7::TailState *)nullptr);
-    return;
+                         (bc7::TailState *)nullptr, max_states);
+    const uint32_t most = p.stats || p.selections ? bc7::kMaxCands : bc7::kMaxBoxCands;
+    if (r.num_blocks <= max_states / most) return;  // however many candidates
   }
   const size_t per_wave = tail_cap / ((size_t)grid.x * 4);
   // each wave hands over at most kHandGroups rotation states and `lanes` others
@@ -4481,14 +4512,14 @@ void launch_anneal(uint32_t waves, int cus, const BlockRange &r, const Bc7Params
   const uint32_t rots = w.alist && room ? (grid.x + kRotShare - 1) / kRotShare : 0u;
   if (p.work_counts) {  // the counting instances (both searches)
     hipLaunchKernelGGL((bc7::anneal_kernel<3, false, true>), grid, wg, 0, stream, r, p, w, unroll,
-                       lanes, rots, tail);
+                       lanes, rots, tail, max_states);
     hipLaunchKernelGGL((bc7::anneal_spread_kernel<true, true>), sgrid, wg, 0, stream, r, p, w,
-                       tail);
+                       tail, 0u);
   } else {
     hipLaunchKernelGGL((bc7::anneal_kernel<3>), grid, wg, 0, stream, r, p, w, unroll, lanes,
-                       rots, tail);
+                       rots, tail, max_states);
     hipLaunchKernelGGL((bc7::anneal_spread_kernel<true, false>), sgrid, wg, 0, stream, r, p, w,
-                       tail);
+                       tail, 0u);
   }
 }
 

@@ -21,10 +21,13 @@ def _diff(a, b):
     return np.nonzero((a.reshape(-1, 16) != b.reshape(-1, 16)).any(axis=1))[0]
 
 
-@pytest.mark.parametrize("w,h,q", [(512, 512, 4), (516, 512, 4), (8, 4, 4)])
+@pytest.mark.parametrize("w,h,q", [(512, 512, 4), (516, 512, 4), (8, 4, 4), (400, 400, 4),
+                                   (512, 512, 16)])
 def test_reference_search_matches_oracle(fh, oracle, w, h, q):
-    """16384 blocks (the last size of the first form), 16512 (the first of
-    the second) and two blocks, with the work counts."""
+    """16384 blocks (the last size where the list's length chooses the form:
+    one lane per candidate at quality 4, one per pixel at 16), 16512 (one lane
+    per candidate always), 10000 (one per pixel, with the choice) and two,
+    with the work counts."""
     img = synth.generate(w, h, 31)
     print(f"anneal forms {w}x{h} q={q}", flush=True)
     L = oracle.lib()
@@ -108,14 +111,15 @@ def test_other_searches_compose(fh, search):
             assert stats[first:first + count].tobytes() == st.tobytes()
 
 
-@pytest.mark.parametrize("threshold,side,parts", [(None, 640, 4), (0.6, 1280, 4),
+@pytest.mark.parametrize("threshold,side,parts", [(None, 640, 4), (0.6, 1280, 4), (1.5, 640, 4),
                                                   (1.5, 1280, 5)])
 def test_parts_compose(fh, threshold, side, parts):
     """A large job equals its parts, which run the other form (the annealing
     streams are keyed by the block's place in the image).  threshold: of the
     learned search, None for the reference's.  At 1.5 every block falls back
-    to the full search's candidates, a third of them rotations, too many for
-    a phase of their own."""
+    to the full search's candidates, a third of them rotations: the list of
+    25600 blocks is then too long for one lane per pixel, and the rotations
+    of 102400 too many for a phase of their own."""
     learned = threshold is not None
     img = synth.generate(side, side, 17)
     rk = None
