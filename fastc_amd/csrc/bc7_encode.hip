@@ -4464,7 +4464,9 @@ constexpr uint32_t kSpreadBlocks = 1u << 14, kSpreadBlocksLearned = 1u << 16;
 // search 2048x2048: 9.5 to 9.7 at 4..24).
 constexpr uint32_t kTailLanes = 12;
 // One workgroup in kRotShare starts on the learned list's rotation states
-// (learned 4096x4096: 4 3.9 ms, 8 3.4, 12 3.3, 16 4.1).
+// (learned 4096x4096: 4 3.9 ms, 8 3.27, 9 3.20, 10 3.14, 12 3.17, 16 4.1), of
+// up to four a CU: three fit, and a larger grid must not give these states a
+// larger part of the chip.
 constexpr uint32_t kRotShare = 10;
 // Workgroups per CU of the one-lane-per-pixel form: five fit, but more waves
 // on a SIMD slow the longest chains (508x380: 4 1.75 ms, 3 1.71, 2 1.78; learned
@@ -4509,7 +4511,8 @@ void launch_anneal(uint32_t waves, int cus, const BlockRange &r, const Bc7Params
   // each wave hands over at most kHandGroups rotation states and `lanes` others
   const uint32_t room = per_wave > bc7::kHandGroups ? (uint32_t)per_wave - bc7::kHandGroups : 0u;
   const uint32_t lanes = room < kTailLanes ? room : kTailLanes;
-  const uint32_t rots = w.alist && room ? (grid.x + kRotShare - 1) / kRotShare : 0u;
+  const uint32_t share_of = grid.x < (uint32_t)cus * 4u ? grid.x : (uint32_t)cus * 4u;
+  const uint32_t rots = w.alist && room ? (share_of + kRotShare - 1) / kRotShare : 0u;
   if (p.work_counts) {  // the counting instances (both searches)
     hipLaunchKernelGGL((bc7::anneal_kernel<3, false, true>), grid, wg, 0, stream, r, p, w, unroll,
                        lanes, rots, tail, max_states);
@@ -4693,7 +4696,7 @@ hipError_t bc7_encode(const BlockRange &r, const Bc7Params &p, const Bc7Scratch 
     // the waves that fit at once (setup_waves), as the batches are dealt out
     // evenly: 4096 waves over 3072 places took mode 1's 1.17 ms (learned
     // 4096x4096) to 1.44.  Annealing-state order: modes 0, 2, 3, 7, 6, 1 in
-    // front, 5 and 4 behind.
+    // front, 4 and 5 behind.
     auto run = [&](auto mode) {
       constexpr int M = decltype(mode)::value;
       const uint32_t fit = (uint32_t)g_num_cus[dev] * bc7::setup_waves(M);

@@ -35,7 +35,7 @@ struct Bc7Params {
   const Ranker *ranker;
   uint32_t topk;         // candidates searched per confident block (1..8)
   float threshold;       // below this top softmax probability: BoxSelection
-  uint32_t wg_per_cu;    // persistent workgroups per CU (0 = 16)
+  uint32_t wg_per_cu;    // persistent waves per CU (0 = 16)
   uint32_t anneal_unroll;  // annealing steps between refills, one-lane form (0 = 1)
   // CompressWithStats' block path: one record per block of the range (null =
   // Compress's BoxSelection search); not combined with the ranker
@@ -125,8 +125,8 @@ struct SurfDesc {
 
 // Launch shapes the batch autotuner chooses.
 struct LaunchTune {
-  uint32_t wg_per_cu = 16;     // persistent workgroups per CU (BC7 set-up / annealing)
-  uint32_t anneal_unroll = 1;  // annealing steps between refills (1, 2 or 4)
+  uint32_t wg_per_cu = 16;     // persistent waves per CU (BC7 set-up by mode, one-lane annealing)
+  uint32_t anneal_unroll = 1;  // one-lane annealing's steps between refills (1, 2 or 4)
   uint32_t simple_wg = 256;    // workgroup size of the DXT / ETC1 batch kernels
 };
 

@@ -403,10 +403,16 @@ typedef struct fh_batch_options {
                                the library's process-wide one */
 } fh_batch_options;
 
-/* Launch shapes chosen by fh_batch_autotune. */
+/* Launch shapes chosen by fh_batch_autotune.  wg_per_cu and anneal_unroll
+ * shape the launches of large BPTC groups only (above 16384 blocks, with a
+ * ranker 65536, and long annealing lists below): smaller ones launch the same
+ * whatever they are, and the fastest of equal trials is reported. */
 typedef struct fh_batch_tune {
-  uint32_t wg_per_cu;      /* persistent workgroups per CU (BPTC set-up and annealing) */
-  uint32_t anneal_unroll;  /* annealing steps between refills of finished lanes */
+  uint32_t wg_per_cu;      /* persistent waves per CU, at most: BPTC set-up by mode (which
+                              launches no more than fit: 8 to 16) and annealing by one lane
+                              per candidate */
+  uint32_t anneal_unroll;  /* that annealing's steps between refills of finished lanes
+                              (with a ranker always 4) */
   uint32_t simple_wg;      /* blocks per workgroup of the DXT / ETC1 kernels */
   float best_ms;           /* time of one run with these shapes */
   uint32_t trials;
