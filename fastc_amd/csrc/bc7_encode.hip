@@ -39,6 +39,7 @@
 
 #include "../../include/fasthip.h"
 #include "bc7_block_decode.h"
+#include "bc7_index.h"
 #include "ranker_tile.h"
 #include "internal.h"
 
@@ -245,35 +246,6 @@ __device__ __forceinline__ u16x2 as_u16x2(uint32_t v) { return __builtin_bit_cas
 __device__ __forceinline__ s16x2 as_s16x2(uint32_t v) { return __builtin_bit_cast(s16x2, v); }
 __device__ __forceinline__ s16x2 as_s16x2(u16x2 v) { return __builtin_bit_cast(s16x2, v); }
 
-// Weight of the second endpoint at index j for nb = 4, 8, 16 entries:
-// (64 j + (nb - 1) / 2) / (nb - 1) by a multiply-shift, equal to
-// kInterpolationValues (Compressor.cpp:159-168); bc7_upload_tables checks
-// every entry on the host before the kernels run.  weight_word holds the
-// weight in its high half, where the packed multiply of interp_err reads it
-// without a shift.
-struct WeightFn {
-  uint32_t m, b;
-};
-__host__ __device__ __forceinline__ WeightFn weight_fn(int nb) {
-  if (nb == 4) return {64u * 21846u, 21846u};
-  if (nb == 8) return {64u * 9363u, 3u * 9363u};
-  return {64u * 4370u, 7u * 4370u};
-}
-__host__ __device__ __forceinline__ uint32_t weight_word(WeightFn fn, uint32_t j) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  // both factors are below 2^24: the full-rate 24-bit multiply-add, which
-  // the compiler only finds where it can see the factors' ranges
-  uint32_t w;
-  asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(w) : "v"(j), "v"(fn.m), "v"(fn.b));
-  return w;
-#else
-  return fn.m * j + fn.b;
-#endif
-}
-__host__ __device__ __forceinline__ uint32_t weight_of(WeightFn fn, uint32_t j) {
-  return weight_word(fn, j) >> 16;
-}
-
 // A texel as the pixel pass reads it: 64 times its channel pairs (each 16-bit
 // lane at most 64 * 255 = 16320).  The interpolated value of an index weight
 // w is (e1 (64 - w) + e2 w + 32) >> 6 = (64 e1 + 32 + (e2 - e1) w) >> 6, so
@@ -316,11 +288,7 @@ __device__ __forceinline__ SubConst sub_const(uint32_t e1, uint32_t e2) {
   c.ad = -64 * dot2(as_s16x2(a02), as_s16x2(c.d02), dot2(as_s16x2(a13), as_s16x2(c.d13), 0));
   const int l = dot2(as_s16x2(c.d02), as_s16x2(c.d02), dot2(as_s16x2(c.d13), as_s16x2(c.d13), 0));
   // equal endpoints give d = 0 for every pixel, so l = 1 yields index 0
-  const float lf = (float)(l > 0 ? l : 1);
-  // v_rcp_f32 is within 1 ulp; one Newton step makes it the correctly
-  // rounded 1 / l for every l <= 4 * 255^2 (checked for starts within 2 ulp)
-  const float r = __builtin_amdgcn_rcpf(lf);
-  c.rl = __builtin_fmaf(__builtin_fmaf(-lf, r, 1.0f), r, r) * 0x1p-6f;
+  c.rl = scaled_rcp(l > 0 ? l : 1);
   return c;
 }
 
@@ -364,36 +332,17 @@ __device__ __forceinline__ s16x2 interp_diff(s16x2 z, uint32_t d, uint32_t ww) {
   return (as_s16x2(d) * W + z) >> S;
 }
 
-// QuantizedError's neighbouring indices (RGBAEndpoints.cpp:240-300) of a
-// pixel: j1 = floor(t), j2 = ceil(t), both clamped to the index range, of the
-// reference's t = fl(fl(d / l) * kf) (float, d the integer projection, l the
-// integer squared distance, kf = nb - 1).  Those equal the floor and ceiling
-// of the rational d kf / l: its distance to an integer, when nonzero, is at
-// least 1 / l >= 1 / (4 * 255^2) = 3.8e-6, more than the float error of at
-// most 2^-23 |t| <= 1.9e-6 for |t| <= 16 (larger |t| is clamped away), and
-// fl(fl(k / kf) kf) = k for every integer 0 <= k <= kf in {3, 7, 15} (checked
-// exhaustively).
-//
-// Here u = fl(64 d * rl) clamped to [0, 1] (64 d is below 2^24, so its
-// conversion is exact; a d below 0 or above l clamps to the end index), and
-// the floor and ceiling are truncations of fma(u, kf, 1.9e-6) and
-// fma(u, kf, 1 - 1.9e-6).  Exact for every l up to 4 * 255^2, d in 0..l and
-// kf: checked exhaustively at the steps of both functions of d, which are
-// monotone.  The pass is bound by VALU issue: an integer quotient corrected
-// with the exact remainder took 17 instructions per pixel where this takes 9;
-// with the texels kept as scaled pairs (no unpacking, one subtraction per
-// pair) and the rotation folded into the axis (no separate point) the pass
-// went from about 54 instructions per pixel to 33, and the 4096 x 4096
-// annealing from 46.0 to 34.3 ms (reference search) and 5.2 to 4.1 ms
-// (learned).
-constexpr float kIndexSlack = 1.9e-6f;
-
+// The neighbouring indices of a pixel (index_bounds).  The pass is bound by VALU
+// issue: an integer quotient corrected with the exact remainder took 17
+// instructions per pixel where this takes 9; with the texels kept as scaled
+// pairs (no unpacking, one subtraction per pair) and the rotation folded into
+// the axis (no separate point) the pass went from about 54 instructions per
+// pixel to 33, and the 4096 x 4096 annealing from 46.0 to 34.3 ms (reference
+// search) and 5.2 to 4.1 ms (learned).
 __device__ __forceinline__ void pixel_bounds(uint32_t p02, uint32_t p13, const SubConst &c,
                                              float kf, uint32_t &j1, uint32_t &j2) {
   const int d = dot2(as_s16x2(p02), as_s16x2(c.q02), dot2(as_s16x2(p13), as_s16x2(c.q13), c.ad));
-  const float u = __builtin_amdgcn_fmed3f((float)d * c.rl, 0.0f, 1.0f);
-  j1 = (uint32_t)__builtin_fmaf(u, kf, kIndexSlack);
-  j2 = (uint32_t)__builtin_fmaf(u, kf, 1.0f - kIndexSlack);
+  index_bounds(d, c.rl, kf, j1, j2);
 }
 
 // The per-pixel index search without branches: both neighbouring indices

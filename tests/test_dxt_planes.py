@@ -1,7 +1,9 @@
 """The DXT encoder keeps a block's channels as planes of four texels to a word.
 Its byte range (16-bit minima of a word as it is and shifted up a byte) and its
 byte weights (a texel's 2-bit index spread to a byte selects 3, 0, 2 or 1) are
-restated here and compared with the plain forms; integers, exactly."""
+restated here and compared with the plain forms; integers, exactly.
+This argues the forms only: the kernels themselves are held against the
+oracle on the GPU in tests/test_dxt_gpu.py."""
 import numpy as np
 import pytest
 

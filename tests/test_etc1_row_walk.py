@@ -2,7 +2,9 @@
 every lane; rg_etc1 (evaluate_solution_fast, rg_etc1.cpp:1767-1885) has
 shortcuts for rows that lie wholly above or below the sub-block's lumas and
 leaves some rows out early.  Both restated in numpy must choose the same row,
-selectors and error; all integers, so exactly."""
+selectors and error; all integers, so exactly.
+This argues the walk only: the kernel itself is held against the oracle on the
+GPU in tests/test_etc1_gpu.py."""
 import numpy as np
 import pytest
 

@@ -2,6 +2,8 @@
 distances up to the largest (black to white in all four channels), where the
 quotient that names the neighbouring indices has the least room."""
 import ctypes
+import os
+import subprocess
 
 import numpy as np
 import pytest
@@ -38,6 +40,17 @@ def test_index_arithmetic(kf):
             j2 = (u.astype(np.float64) * kf + np.float64(rest)).astype(np.float32).astype(int)
             assert np.array_equal(j1[ok], (d * kf // ls)[ok])
             assert np.array_equal(j2[ok], (-(-d * kf // ls))[ok])
+
+
+def test_index_arithmetic_of_the_encoder(tmp_path):
+    """The encoder's own header (bc7_index.h) compiled for the host: every
+    distance, every start of the reciprocal within 2 ulp, every step."""
+    here = os.path.dirname(os.path.abspath(__file__))
+    exe = str(tmp_path / "index_test")
+    subprocess.run(["g++", "-std=c++17", "-O2", "-ffp-contract=off",
+                    os.path.join(here, "cpp", "index_test.cpp"), "-o", exe], check=True)
+    r = subprocess.run([exe], capture_output=True, text=True)
+    assert r.returncode == 0 and int(r.stdout.split()[0]) > 260100 * 145, r.stdout
 
 
 @pytest.mark.gpu
