@@ -21,16 +21,17 @@
 //           scores all 16 pixels in one pass, each against its subset's endpoints.
 //           Large lists run one lane per candidate, lanes that finish refilling
 //           from the work list, and hand the last few candidates of each wave
-//           over; those, and small lists from the start, run one lane per pixel,
-//           16 lanes a candidate, where few candidates are left looking several
-//           steps ahead.
+//           over; those, and short lists from the start (spread_list), run one
+//           lane per pixel, 16 lanes a candidate, where few candidates are left
+//           looking several steps ahead.
 //   pack    one lane per block: sum the subset errors per mode in the
 //           reference's mode order, keep the first strict minimum and write the
 //           128-bit block (CompressionMode::Pack, :1096-1298); solid blocks get
 //           the watermark entry from an exclusive scan of solid-block flags.
 //
-// Uniform error metric only: all errors are then exact integers (< 2^24), so
-// they are kept in uint32 and equal the reference's float/double sums.
+// Under the uniform error metric all errors are exact integers (< 2^24), so
+// they are kept in uint32 and equal the reference's float/double sums; the
+// nonuniform metric's floats are described above qerr_nu.
 #include <float.h>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -3687,6 +3688,9 @@ __global__ void __launch_bounds__(256) anneal_spread_kernel(BlockRange r, Bc7Par
 // set the launch's length, would run on in nearly empty waves.
 // NU: the nonuniform metric (float errors, whose sums have an order: the
 // lanes finish their own candidates).
+// WAVES = 3 gives the uniform form 168 VGPRs, of which 18 spill (80 bytes a lane,
+// stored once per `unroll` steps): two thirds of its 1.7 GB written at 4096x4096
+// are scratch, against a 27 ms issue bound.
 // COUNT: also count the work into prm.work_counts: [0] the QuantizedError
 // point evaluations the reference's annealing makes (each step of a subset
 // scores that subset's points, Compressor.cpp:583-624), [1] the pixel scores

@@ -227,7 +227,8 @@ __device__ __forceinline__ uint64_t pixel_error64(uint32_t p, uint32_t q) {
 // Workgroups of 512: the image total takes one atomic per workgroup on one
 // word, at some 7 ns each.  With the rows loaded before the block is decoded,
 // and by two pixels where the width is even only, a 1918x1078 BC7 error takes
-// 11.0 us (17.0 before, of which the zeroing launch is a third).
+// 11.3 us (17.7 before), of which the zeroing launch is a third and VALU issue
+// a fifth: the kernel itself is a round of loads and the reduction.
 constexpr int kErrorWg = 512;
 
 template <int FMT, int VEC>

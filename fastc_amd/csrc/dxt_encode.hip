@@ -10,9 +10,9 @@
 //
 // One lane per 4x4 block; each lane loads its four 16-byte rows with 128-bit
 // loads, so a wavefront over 64 horizontally adjacent blocks reads four
-// contiguous 1 KiB runs.  The encode is a few hundred integer operations per
-// block, so the kernel is bound by HBM traffic (4 B/texel in, 0.5 or 1 B/texel
-// out).
+// contiguous 1 KiB runs.  A wave issues 1750 vector instructions for its 64
+// DXT1 blocks and 1982 for DXT5: at 4096x4096 53 of DXT5's 56 us are their issue,
+// three times what the bytes (4 B/texel in, 0.5 or 1 out) take.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -73,7 +73,8 @@ __device__ __forceinline__ void eval_colors(int col[4][3], uint32_t c0, uint32_t
 }
 
 // The kernels copy the two tables into LDS (q: red/blue then green, 784
-// bytes each), where the lookups of the dither's serial chain are short.
+// bytes each), where the lookups of the dither's chains (16 texels one after
+// another in each of three channels) are short.
 __device__ __forceinline__ int qtab(const uint8_t *q, int ch_, int idx) {
   return q[(ch_ == 1 ? 784 : 0) + idx + 256];
 }
@@ -174,8 +175,8 @@ __device__ uint32_t match_colors(const uint32_t blk[16], const int col[4][3]) {
 
 // A block's colour channels, four texels to a word, and their sums: the sums
 // of products that the fit needs are then four-way byte dot products.
-// 119 -> 87 VGPRs; the dither's serial chain before it stays: 4096x4096 DXT5
-// 57.9 -> 55.9 us, 2048x2048 DXT1 16.1 -> 15.5.
+// 119 -> 87 VGPRs; the dither before it, most of the instructions, stays:
+// 4096x4096 DXT5 57.9 -> 55.6 us, 2048x2048 DXT1 16.1 -> 15.6.
 struct Planes {
   uint32_t w[3][4];
   int sum[3];

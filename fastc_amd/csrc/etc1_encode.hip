@@ -112,7 +112,8 @@ __device__ __forceinline__ uint32_t row_colour(int r, int g, int b, uint32_t cur
 // squared distance is p.p - 2 p.c + c.c, p.p summed once) and one shift that
 // collects the index.
 // 2044x1532: 281 us with the shortcuts, the sorted lumas that they need and 205
-// VGPRs (two waves a SIMD, three to place); 162 us at 122 VGPRs (four).
+// VGPRs (two waves a SIMD, three to place); 165 us at 122 VGPRs (room for four,
+// still three to place: 68% VALU busy, 114 us of issue).
 __device__ bool evaluate_fast(const Opt &o, int cr, int cg, int cb, Solution &best) {
   if (o.constrain) {
     const int dr = cr - o.base_r, dg = cg - o.base_g, db = cb - o.base_b;
